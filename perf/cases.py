@@ -131,7 +131,8 @@ def _between_planets(case, s):
         clear = np.all((hi[p:, None] < lo[None, :p]) | (lo[p:, None] > hi[None, :p]), axis=1)
         if clear.sum() >= n:
             break
-    keep = np.concatenate([np.arange(np_), first + np.nonzero(clear)[0][:n], first + np.nonzero(~clear)[0][:max(0, n - int(clear.sum()))]])
+    order = np.concatenate([np.nonzero(clear)[0], np.nonzero(~clear)[0]])
+    keep = np.concatenate([np.arange(first), first + order[:n]])
     arrays = {f: getattr(scn, f)[keep] for f in ("mass", "radius", "density", "cd", "gamma_stokes", "gamma_epstein",
                                                  "mig_stop_at", "type", "mig_type", "y0", "target_offsets")}
     counts = dict(scn.counts, test_particle=n, total=first + n)
