@@ -8,10 +8,13 @@
 // run on the host, from one 8-byte error maximum per attempt.
 #include <algorithm>
 #include <cmath>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -489,6 +492,16 @@ int grid_sources(const sol_context *c)
     return std::max(1, std::max(c->n_massive, std::max(ea, eb)));
 }
 
+// Slices of `block` threads the device holds at once.
+int grid_capacity_of(sol_context *c, int ik, int block)
+{
+    const bool gas = c->has_gas && !c->gas_dead;
+    const int bi = block == 64 ? 0 : block == 128 ? 1 : 2;
+    int &cap = c->grid_capacity[(2 * ik + (gas ? 1 : 0)) * 3 + bi];
+    if (cap < 0) cap = resident_grid_capacity(ik, block, block, c->lds_limit, c->cu_count, gas);
+    return cap;
+}
+
 // The grid form (slices of one system, one workgroup each, one body per
 // thread) for systems with few sources: at most a quarter of a slice, at
 // least grid_min_bodies bodies, and no more slices than the device keeps
@@ -511,10 +524,7 @@ bool use_grid(sol_context *c, int ik, SliceMap *m)
     }
     if (src > block / 4) return false;
     const SliceMap sm = slice_map_make(c->n, c->np, src, block);
-    const bool gas = c->has_gas && !c->gas_dead;
-    const int bi = block == 64 ? 0 : block == 128 ? 1 : 2;
-    int &cap = c->grid_capacity[(2 * ik + (gas ? 1 : 0)) * 3 + bi];
-    if (cap < 0) cap = resident_grid_capacity(ik, block, block, c->lds_limit, c->cu_count, gas);
+    const int cap = grid_capacity_of(c, ik, block);
     if (sm.nslices > cap || sm.nslices > kGridMaxSlices) return false;
     if (m) *m = sm;
     return true;
@@ -612,12 +622,40 @@ SliceArrays system_arrays(sol_context *c)
     return s;
 }
 
+// The mesh form (mesh.hip): astrocentric FP64 gravity without gas, sources
+// enough to share out, and no more workgroups than the device holds at once.
+// From 32 sources on: an RKF78 attempt of 33 bodies takes 48 us on the mesh
+// and 58 in one workgroup, of 17 bodies 47 and 35.
+constexpr int kMeshMinSources = 32;
+constexpr int kPathMesh = 100;     // reported as SOL_PATH_GRID
+
+bool use_mesh(sol_context *c, int ik, int *share_out = nullptr, int *groups_out = nullptr)
+{
+    if (c->resident_disabled || c->grid_disabled || c->barycentric) return false;
+    if (c->has_gas && !c->gas_dead) return false;
+    if (c->precision != SOL_PRECISION_FP64) return false;
+    // a profiled context (sol_profile) keeps the launches that are timed
+    if (c->profiling && !use_resident(c, ik)) return false;
+    int ea, eb;
+    source_ends(c, ea, eb);
+    if (std::max(ea, eb) < kMeshMinSources) return false;
+    const int share = mesh_share(c->n, c->n_massive, ea, eb, c->cu_count);
+    if (share == 0) return false;
+    const int groups = mesh_groups(c->n, c->n_massive, ea, eb, share);
+    if (mesh_capacity(ik, c->n, share, c->cu_count) < groups) return false;
+    if (share_out) *share_out = share;
+    if (groups_out) *groups_out = groups;
+    return true;
+}
+
 // The path a Driver call or a caller loop of integrator ik takes: the grid
 // form where it applies (few sources, more bodies than grid_min_bodies),
-// else one workgroup where the system fits, else one launch per stage.
+// the mesh form for many sources, else one workgroup where the system fits,
+// else one launch per stage.
 int path_of(sol_context *c, int ik, SliceMap *m)
 {
     if (use_grid(c, ik, m)) return SOL_PATH_GRID;
+    if (use_mesh(c, ik)) return kPathMesh;
     return use_resident(c, ik) ? SOL_PATH_RESIDENT : SOL_PATH_MULTI_KERNEL;
 }
 
@@ -627,6 +665,76 @@ bool use_resident_any(sol_context *c, int ik) { return path_of(c, ik, nullptr) !
 // that was not resident): the call is to be made again from the same state
 // (on the grid form once more, then on another path).
 constexpr int kGridRetry = -1000;
+
+// The compute units that launches whose workgroups wait for each other (grid
+// and mesh form) hold on a device.  Two such launches of this process that
+// did not fit side by side could each hold a part of the device and wait for
+// the rest, so a launch first takes as many units as it needs, waiting for
+// those of other contexts' launches to end (each at most about 0.2 s).
+class UnitLease {
+public:
+    UnitLease(int device, int units, int total) : d_(pool(device)), units_(std::min(units, total))
+    {
+        std::unique_lock<std::mutex> lock(d_.m);
+        d_.cv.wait(lock, [&] { return d_.used + units_ <= total; });
+        d_.used += units_;
+    }
+    ~UnitLease()
+    {
+        {
+            std::lock_guard<std::mutex> lock(d_.m);
+            d_.used -= units_;
+        }
+        d_.cv.notify_all();
+    }
+    UnitLease(const UnitLease &) = delete;
+    UnitLease &operator=(const UnitLease &) = delete;
+
+private:
+    struct Device {
+        std::mutex m;
+        std::condition_variable cv;
+        int used = 0;
+    };
+    static Device &pool(int device)
+    {
+        static Device devices[64];
+        return devices[device & 63];
+    }
+    Device &d_;
+    int units_;
+};
+
+// Time line, counters, switches and status after a run of the resident
+// drivers that ended with S.
+int resident_finish(sol_context *c, const ResSystem &S, sol_timeline *tl, int64_t max_steps, bool clip,
+                    double *body_h, int64_t *steps_out, int64_t *attempts_out, int32_t stop_mask, int32_t *reason)
+{
+    tl->time = S.t; tl->hNext = S.h_next; tl->hDid = S.h_did;
+    tl->elapsedTime = S.elapsed; tl->lastSave = S.last_save; tl->lastNSteps = S.last_nsteps;
+    if (clip) tl->flush_count = S.flush_count;
+    if (reason) {
+        // the last step's reasons (S.reason is written at every clipped step)
+        *reason = S.reason & (stop_mask | SOL_STOP_END);
+        if (S.status == RES_DONE) *reason |= SOL_STOP_END;
+        if (max_steps > 0 && S.steps >= max_steps) *reason |= SOL_STOP_STEPS;
+    }
+    if (body_h) *body_h = S.body_h;
+    if (steps_out) *steps_out += S.steps;
+    if (attempts_out) *attempts_out += S.attempts;
+    // the Driver leaves the drag switch on and the migration switches off
+    c->eval_drag = 1;
+    c->eval_mig1 = c->eval_mig2 = 0;
+    if (S.status == RES_UNDERFLOW)
+        return c->fail(SOL_ERR_UNDERFLOW, "Stepsize-underflow occurred during Runge-Kutta-Fehlberg7(8) step!");
+    if (S.status == RES_MAXITER)
+        return c->fail(SOL_ERR_MAXITER,
+                       "An error occurred during Prince-Dormand driver: iteration number exceeded maxIter!");
+    return SOL_OK;
+}
+
+int mesh_run(sol_context *c, int ik, double eps, sol_timeline *tl, int64_t max_steps, bool clip, double *body_h,
+             int64_t *steps_out, int64_t *attempts_out, int32_t stop_mask, int32_t *reason);
 
 // Runs accepted steps of integrator ik in the resident kernel: exactly one
 // Driver call when clip is false and max_steps == 1, or the caller loop
@@ -638,7 +746,10 @@ int resident_run(sol_context *c, int ik, double eps, sol_timeline *tl, int64_t m
                  int64_t *steps_out, int64_t *attempts_out, int32_t stop_mask = 0, int32_t *reason = nullptr)
 {
     SliceMap m{};
-    const bool grid = path_of(c, ik, &m) == SOL_PATH_GRID;
+    const int path = path_of(c, ik, &m);
+    if (path == kPathMesh)
+        return mesh_run(c, ik, eps, tl, max_steps, clip, body_h, steps_out, attempts_out, stop_mask, reason);
+    const bool grid = path == SOL_PATH_GRID;
     ResSystem S0 = resident_system(c, eps, tl, clip, stop_mask);
     ResArrays A;
     ResSystem *sys_d = c->res_d;
@@ -673,7 +784,10 @@ int resident_run(sol_context *c, int ik, double eps, sol_timeline *tl, int64_t m
     const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(20000, (int64_t)(0.2 / per_step)));
     for (;;) {
         const int64_t k = max_steps > 0 ? std::min(chunk, max_steps - S.steps) : chunk;
+        std::unique_ptr<UnitLease> lease;
         if (grid) {
+            const int per_cu = std::max(1, grid_capacity_of(c, ik, m.stride) / std::max(1, c->cu_count));
+            lease.reset(new UnitLease(c->device, (nsys + per_cu - 1) / per_cu, c->cu_count));
             HIPCHECK(c, launch_resident_grid(c->stream, ik, sys_d, nsys, A, (int)k, m.stride, m.stride,
                                              c->lds_limit));
             HIPCHECK(c, hipMemcpyAsync(c->grid_sys_h.data(), sys_d, nsys * sizeof(ResSystem),
@@ -714,29 +828,94 @@ int resident_run(sol_context *c, int ik, double eps, sol_timeline *tl, int64_t m
         HIPCHECK(c, hipGetLastError());
         HIPCHECK(c, hipStreamSynchronize(c->stream));
     }
-    tl->time = S.t; tl->hNext = S.h_next; tl->hDid = S.h_did;
-    tl->elapsedTime = S.elapsed; tl->lastSave = S.last_save; tl->lastNSteps = S.last_nsteps;
-    if (clip) tl->flush_count = S.flush_count;
-    if (reason) {
-        // the last step's reasons (S.reason is written at every clipped step)
-        *reason = S.reason & (stop_mask | SOL_STOP_END);
-        if (S.status == RES_DONE) *reason |= SOL_STOP_END;
-        if (max_steps > 0 && S.steps >= max_steps) *reason |= SOL_STOP_STEPS;
-    }
-    if (body_h) *body_h = S.body_h;
-    if (steps_out) *steps_out += S.steps;
-    if (attempts_out) *attempts_out += S.attempts;
-    // the Driver leaves the drag switch on and the migration switches off
-    c->eval_drag = 1;
-    c->eval_mig1 = c->eval_mig2 = 0;
-    if (S.status == RES_UNDERFLOW)
-        return c->fail(SOL_ERR_UNDERFLOW, "Stepsize-underflow occurred during Runge-Kutta-Fehlberg7(8) step!");
-    if (S.status == RES_MAXITER)
-        return c->fail(SOL_ERR_MAXITER,
-                       "An error occurred during Prince-Dormand driver: iteration number exceeded maxIter!");
-    return SOL_OK;
+    return resident_finish(c, S, tl, max_steps, clip, body_h, steps_out, attempts_out, stop_mask, reason);
 }
 
+// Arrays and exchange words of the mesh form.
+int mesh_buffers(sol_context *c)
+{
+    sol_context::Mesh &m = c->mesh;
+    if (m.pos) return SOL_OK;
+    const size_t np = c->np;
+    unsigned char *sys = nullptr;
+    int r;
+    if ((r = dalloc(c, &m.y0, 6 * np)) || (r = dalloc(c, &m.y, 6 * np)) || (r = dalloc(c, &m.acc0, 6 * np)) ||
+        (r = dalloc(c, &m.yscale, 6 * np)) || (r = dalloc(c, &m.error, 6 * np)) || (r = dalloc(c, &m.rm3, np)) ||
+        (r = dalloc(c, &m.nnd, np)) || (r = dalloc(c, &m.nni, np)) || (r = dalloc(c, &m.part, 1)) ||
+        (r = dalloc(c, &m.part_of, (size_t)kMeshMaxGroups)) ||
+        (r = dalloc(c, &sys, sizeof(ResSystem) + sizeof(MeshSync))))
+        return r;
+    m.sys = reinterpret_cast<ResSystem *>(sys);
+    m.sync = reinterpret_cast<MeshSync *>(sys + sizeof(ResSystem));
+    if (!c->mesh_h && hipHostMalloc((void **)&c->mesh_h, sizeof(ResSystem) + 8 + sizeof(MeshPart), hipHostMallocDefault) != hipSuccess) {
+        c->mesh_h = nullptr;
+        return c->fail(SOL_ERR_DEVICE, "hipHostMalloc failed");
+    }
+    return dalloc(c, &m.pos, 6 * np);
+}
+
+// resident_run on the mesh form: accepted steps of integrator ik with the
+// system's bodies shared out over workgroups, about 0.2 s of work per
+// launch.  The context's arrays are replaced by the run's at its end only.
+int mesh_run(sol_context *c, int ik, double eps, sol_timeline *tl, int64_t max_steps, bool clip, double *body_h,
+             int64_t *steps_out, int64_t *attempts_out, int32_t stop_mask, int32_t *reason)
+{
+    int share = 0, groups = 0;
+    if (!use_mesh(c, ik, &share, &groups)) return kGridRetry;
+    int r = mesh_buffers(c);
+    if (r) return r;
+    sol_context::Mesh &m = c->mesh;
+    ResSystem &S = *reinterpret_cast<ResSystem *>(c->mesh_h);
+    uint32_t &lost = *reinterpret_cast<uint32_t *>(c->mesh_h + sizeof(ResSystem));
+    S = resident_system(c, eps, tl, clip, stop_mask);
+    HIPCHECK(c, hipMemcpyAsync(m.sys, &S, sizeof S, hipMemcpyHostToDevice, c->stream));
+    MeshPart &P = *reinterpret_cast<MeshPart *>(c->mesh_h + sizeof(ResSystem) + 8);
+    P = MeshPart{0, 0, groups, share};
+    HIPCHECK(c, hipMemcpyAsync(m.part, &P, sizeof P, hipMemcpyHostToDevice, c->stream));
+    MeshArgs A{};
+    A.systems = m.sys;
+    A.parts = m.part; A.part_of = m.part_of;
+    A.sync = m.sync;
+    A.pos = m.pos; A.gm = c->gm;
+    A.tot = c->np;
+    A.mass = c->mass; A.radius = c->radius;
+    A.y0 = m.y0; A.y = m.y; A.acc0 = m.acc0; A.yscale = m.yscale; A.err = m.error;
+    A.rm3 = m.rm3; A.nnd = m.nnd; A.nni = m.nni;
+    A.eps2 = c->softening * c->softening;
+    A.ticks = (uint64_t)(c->grid_wait_s * (double)c->rtc_hz);
+    const double per_step = 13.0 * (5.0e-6 + (double)c->n * (double)c->n * 1.0e-12);
+    const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(20000, (int64_t)(0.2 / per_step)));
+    A.y0_in = c->y0;
+    for (;;) {
+        const int64_t k = max_steps > 0 ? std::min(chunk, max_steps - S.steps) : chunk;
+        const UnitLease lease(c->device, groups, c->cu_count);
+        HIPCHECK(c, launch_mesh(c->stream, ik, A, 1, groups, c->n, share, (int)k));
+        HIPCHECK(c, hipMemcpyAsync(c->mesh_h, m.sys, sizeof(ResSystem) + sizeof(uint32_t), hipMemcpyDeviceToHost,
+                                   c->stream));
+        HIPCHECK(c, hipStreamSynchronize(c->stream));
+        if (lost != 0 || S.status == RES_SYNC_ERROR) {
+            // a workgroup that was not resident: as for the grid form, the
+            // call runs again from its unchanged start
+            if (++c->grid_failures >= 2) c->grid_disabled = true;
+            return kGridRetry;
+        }
+        if (!std::isfinite(S.t) || !std::isfinite(S.h_next))
+            return c->fail(SOL_ERR_DEVICE, "mesh driver: non-finite time or step size (t %g, hNext %g)", S.t,
+                           S.h_next);
+        if (S.status != RES_RUNNING) break;
+        if (max_steps > 0 && S.steps >= max_steps) break;
+        A.y0_in = m.y0;
+    }
+    std::swap(c->y0, m.y0);
+    std::swap(c->y, m.y);
+    std::swap(c->acc0, m.acc0);
+    if (ik == INTEG_RKF78) std::swap(c->yscale, m.yscale);
+    if (ik != INTEG_RK4) std::swap(c->error, m.error);
+    std::swap(c->rm3, m.rm3);
+    std::swap(c->nnd, m.nnd);
+    std::swap(c->nni, m.nni);
+    return resident_finish(c, S, tl, max_steps, clip, body_h, steps_out, attempts_out, stop_mask, reason);
+}
 
 int driver_rkf78(sol_context *c, double eps, sol_timeline *tl, double *body_h, int64_t *attempts)
 {
@@ -999,6 +1178,7 @@ int sol_destroy(sol_context *c)
     if (c->h_scal) (void)hipHostFree(c->h_scal);
     if (c->res_h) (void)hipHostFree(c->res_h);
     if (c->integ_h) (void)hipHostFree(c->integ_h);
+    if (c->mesh_h) (void)hipHostFree(c->mesh_h);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -1354,8 +1534,10 @@ int sol_integrate_until(sol_context *c, int32_t integrator, double eps, sol_time
         stats->force_evaluations = steps + attempts * per;
         stats->interactions = (double)stats->force_evaluations * c->interactions_per_eval;
         stats->device_ms = ms;
-        stats->path = path;
-        stats->slices = path == SOL_PATH_GRID ? gm.nslices : 0;
+        int groups = 0;
+        if (path == kPathMesh) (void)use_mesh(c, ik, nullptr, &groups);
+        stats->path = path == kPathMesh ? SOL_PATH_GRID : path;
+        stats->slices = path == SOL_PATH_GRID ? gm.nslices : groups;
     }
     return r;
 }

@@ -11,6 +11,7 @@
 
 #include "sol_internal.h"
 #include "resident.h"
+#include "mesh.h"
 
 namespace sol { struct AdjointState; }
 
@@ -76,6 +77,20 @@ struct sol_context {
     int grid_failures = 0;           // grid runs that gave up; two turn the grid form off
     int grid_capacity[18] = {-1, -1, -1, -1, -1, -1, -1, -1, -1,
                              -1, -1, -1, -1, -1, -1, -1, -1, -1};   // per integrator, gas, slice size
+    // self-gravitating systems over several workgroups (mesh.hip): the arrays
+    // a run writes, which change places with the context's own at its end
+    // (a run that could not complete leaves those untouched)
+    struct Mesh {
+        double *y0 = nullptr, *y = nullptr, *acc0 = nullptr, *yscale = nullptr, *error = nullptr;
+        double *rm3 = nullptr, *nnd = nullptr;
+        int32_t *nni = nullptr;
+        double *pos = nullptr;
+        sol::ResSystem *sys = nullptr;       // followed by the MeshSync
+        sol::MeshSync *sync = nullptr;
+        sol::MeshPart *part = nullptr;
+        int32_t *part_of = nullptr;
+    } mesh;
+    unsigned char *mesh_h = nullptr;         // pinned: ResSystem and the error word
     // profiling (sol_profile)
     bool profiling = false;
     std::vector<hipEvent_t> ev_pool;
