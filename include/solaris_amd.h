@@ -418,13 +418,13 @@ int sol_adjoint_backward(sol_context *ctx, const double *grad_y_final, double *g
  * ranges: Kepler term, pair terms, indirect term; the star's derivative
  * zero) for a gas-free astrocentric system whose arrays are already on the
  * current device: y and dydt are device arrays of 6*total doubles (AoS),
- * mass a device array of total doubles.  It allocates no device memory:
- * its scratch is a static device array of the library (64 bytes per body),
- * so total is at most 131072 (larger sizes are rejected with
+ * mass a device array of total doubles.  It allocates no device memory.
+ * total is at most 131072 (larger sizes are rejected with
  * SOL_ERR_ARGUMENT).  The kernels are queued on `stream` (a hipStream_t,
- * NULL for the null stream) and the call returns without waiting.  Calls
- * on one GPU share its scratch array, so calls that overlap on one GPU
- * (on different streams or host threads) race.  err (may be NULL) receives
+ * NULL for the null stream) and the call returns without waiting.  Where y
+ * and dydt overlap, y is first copied to a static device array of the
+ * library (48 bytes per body), so such calls that overlap on one GPU (on
+ * different streams or host threads) race; others do not.  err (may be NULL) receives
  * the message of a failure, at most err_len bytes with the terminating
  * zero.  No counterpart in the reference: it is for callers that cannot
  * allocate device memory, such as code under HIP graph capture and
