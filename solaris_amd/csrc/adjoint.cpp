@@ -36,6 +36,7 @@ struct AdjointState {
     int64_t nsteps = 0;
     int K = 0;
     bool recorded = false;
+    bool few = false;                  // recorded by the chains of adjoint_few.hip
     std::vector<double> h, t;          // step sizes and start times
     size_t ncp = 0, ckpt_cap = 0;      // checkpoints held / allocated
     double *ckpt = nullptr;            // [ncp][6 NP]
@@ -49,8 +50,13 @@ struct AdjointState {
     double *mbar = nullptr, *m0blk = nullptr, *mout = nullptr;
     double *psink = nullptr, *psrc = nullptr;
     int psink_cap = 0, psrc_cap = 0;   // chunks allocated
-    double *hd = nullptr;              // step sizes on the device (resident path)
+    double *hd = nullptr;              // step sizes on the device
     size_t hd_cap = 0;
+    // few sources (adjoint_few.hip): steps per chunk, the sources' stage
+    // records of two chunks, the sinks' weights and the sums over them
+    int few_chunk = 0, few_src = 0;
+    double4 *few_sp = nullptr;
+    double *few_u = nullptr, *few_sums = nullptr, *m0src = nullptr;
     VjpArgs shape{};                   // launch shape of the products
     std::vector<void *> allocs;
 };
@@ -64,6 +70,10 @@ void adjoint_release(sol_context *c)
     if (c->adj->psink) (void)hipFree(c->adj->psink);
     if (c->adj->psrc) (void)hipFree(c->adj->psrc);
     if (c->adj->hd) (void)hipFree(c->adj->hd);
+    if (c->adj->few_sp) (void)hipFree(c->adj->few_sp);
+    if (c->adj->few_u) (void)hipFree(c->adj->few_u);
+    if (c->adj->few_sums) (void)hipFree(c->adj->few_sums);
+    if (c->adj->m0src) (void)hipFree(c->adj->m0src);
     delete c->adj;
     c->adj = nullptr;
 }
@@ -198,6 +208,86 @@ int rk4_step(sol_context *c, AdjointState *A, const double *y, double t, double 
     return SOL_OK;
 }
 
+// Whether the chains of adjoint_few.hip take this system: 1 to 32 sources.
+// SOLARIS_AMD_VJP_WIDE=1, which asks for k_vjp_src, keeps the products of
+// adjoint.hip.
+bool few_ok(const sol_context *c)
+{
+    int ea, eb;
+    source_ends(c, ea, eb);
+    const int src = std::min(c->n, std::max(ea, eb));
+    const char *wide = getenv("SOLARIS_AMD_VJP_WIDE");
+    return src >= 2 && src - 1 <= kFewMaxSources && !(wide && wide[0] == '1');
+}
+
+// Buffers of the chains: chunks of 64 steps, fewer where their weights would
+// take more than 64 MB.
+int few_buffers(sol_context *c)
+{
+    AdjointState *A = c->adj;
+    int ea, eb;
+    source_ends(c, ea, eb);
+    const int src = std::min(c->n, std::max(ea, eb));
+    if (A->few_sp && A->few_src >= src) return SOL_OK;
+    for (void *p : {(void *)A->few_sp, (void *)A->few_u, (void *)A->few_sums, (void *)A->m0src})
+        if (p) (void)hipFree(p);
+    A->few_sp = nullptr; A->few_u = nullptr; A->few_sums = nullptr; A->m0src = nullptr;
+    const size_t step = 12 * (size_t)c->np * sizeof(double);
+    const int chunk = (int)std::max<size_t>(1, std::min<size_t>(64, ((size_t)64 << 20) / step));
+    HIPCHECK(c, hipMalloc(&A->few_u, chunk * step));
+    HIPCHECK(c, hipMalloc(&A->few_sums, (size_t)chunk * 4 * src * 7 * sizeof(double)));
+    HIPCHECK(c, hipMalloc(&A->m0src, (size_t)src * sizeof(double)));
+    HIPCHECK(c, hipMalloc(&A->few_sp, (size_t)2 * chunk * 4 * src * sizeof(double4)));
+    A->few_chunk = chunk;
+    A->few_src = src;
+    return SOL_OK;
+}
+
+FewArgs few_args(const sol_context *c)
+{
+    const AdjointState *A = c->adj;
+    FewArgs f{};
+    f.n = c->n; f.np = c->np; f.nm = c->n_massive;
+    source_ends(c, f.ea, f.eb);
+    f.src = std::min(c->n, std::max(f.ea, f.eb));
+    f.K = 1;
+    f.gm = c->gm;
+    f.h = A->hd;
+    f.mbar = A->mbar;
+    f.m0src = A->m0src;
+    f.u = A->few_u;
+    f.sums = A->few_sums;
+    return f;
+}
+
+// Steps [n0, n1) of the forward pass from y, in place; stage states of the
+// steps from n0 on to stages, checkpoints every K steps (either may be null).
+// The sources run a chunk ahead of the sinks.
+int few_forward(sol_context *c, double *y, int64_t n0, int64_t n1, double *stages, double *ckpt, int K)
+{
+    AdjointState *A = c->adj;
+    FewArgs f = few_args(c);
+    f.y = y;
+    f.stages = stages;
+    f.first = (int32_t)n0;
+    f.ckpt = ckpt;
+    f.K = K;
+    const size_t half = (size_t)A->few_chunk * 4 * f.src;
+    int parity = 0;
+    for (int64_t s = n0; s < n1 + A->few_chunk; s += A->few_chunk, parity ^= 1) {
+        f.t0 = f.s0; f.t1 = f.s1;                 // the sinks take the chunk before
+        f.s0 = (int32_t)std::min<int64_t>(s, n1);
+        f.s1 = (int32_t)std::min<int64_t>(s + A->few_chunk, n1);
+        if (s == n0) f.t0 = f.t1 = 0;
+        if (f.s0 >= f.s1 && f.t0 >= f.t1) break;
+        f.sp_out = A->few_sp + (size_t)parity * half;
+        f.sp_in = A->few_sp + (size_t)(parity ^ 1) * half;
+        launch_few_forward(c->stream, f);
+    }
+    HIPCHECK(c, hipGetLastError());
+    return SOL_OK;
+}
+
 int check_supported(sol_context *c)
 {
     if (c->barycentric) return c->fail(SOL_ERR_UNSUPPORTED, "adjoint: barycentric frame not supported");
@@ -248,8 +338,8 @@ int sol_adjoint_forward(sol_context *c, double t0, double h, const double *h_seq
     A->all_stages = all;
     HIPCHECK(c, hipMemcpyAsync(A->ya, c->y0, v * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
     double *cur = A->ya, *nxt = A->yb;
-    if (resident_rk4_ok(c)) {
-        // one launch of the workgroup-resident driver per segment
+    const bool few = few_ok(c) && nsteps < INT32_MAX;
+    if (few || resident_rk4_ok(c)) {
         if (A->hd_cap < (size_t)nsteps) {
             if (A->hd) (void)hipFree(A->hd);
             A->hd = nullptr;
@@ -258,6 +348,13 @@ int sol_adjoint_forward(sol_context *c, double t0, double h, const double *h_seq
             A->hd_cap = (size_t)nsteps;
         }
         HIPCHECK(c, hipMemcpyAsync(A->hd, hs.data(), nsteps * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    }
+    A->few = few;
+    if (few) {
+        if ((r = few_buffers(c))) return r;
+        if ((r = few_forward(c, cur, 0, nsteps, all ? A->seg : nullptr, all ? nullptr : A->ckpt, K))) return r;
+    } else if (resident_rk4_ok(c)) {
+        // one launch of the workgroup-resident driver per segment
         for (int64_t n0 = 0; n0 < nsteps; n0 += K) {
             const int64_t n1 = std::min<int64_t>(nsteps, n0 + K);
             HIPCHECK(c, hipMemcpyAsync(A->ckpt + (size_t)(n0 / K) * v, cur, v * sizeof(double),
@@ -314,7 +411,41 @@ int sol_adjoint_backward(sol_context *c, const double *grad_y_final, double *gra
     a.mbar = A->mbar;
     a.m0blk = A->m0blk;
     double *lam = A->lam, *ybar = A->ybar;
-    for (int64_t sg = (int64_t)A->ncp - 1; sg >= 0; --sg) {
+    if (A->few) {
+        FewArgs f = few_args(c);
+        f.lam = lam;
+        f.stages = A->seg;
+        HIPCHECK(c, hipMemsetAsync(A->m0src, 0, (size_t)A->few_src * sizeof(double), c->stream));
+        // chunk by chunk backwards: the sinks of a chunk beside the sources of
+        // the one after it, then the chunk's sums
+        for (int64_t sg = (int64_t)A->ncp - 1; sg >= 0; --sg) {
+            const int64_t n0 = A->all_stages ? 0 : sg * A->K;
+            const int64_t n1 = A->all_stages ? A->nsteps : std::min<int64_t>(A->nsteps, n0 + A->K);
+            if (!A->all_stages) {
+                // the sources are done with the segment's stage states too
+                f.t0 = f.t1 = 0;
+                if (f.s1 > f.s0) launch_few_backward(c->stream, f);
+                f.s0 = f.s1 = 0;
+                HIPCHECK(c, hipMemcpyAsync(A->ya, A->ckpt + (size_t)sg * v, v * sizeof(double), hipMemcpyDeviceToDevice,
+                                           c->stream));
+                if ((r = few_forward(c, A->ya, n0, n1, A->seg, nullptr, 1))) return r;
+            }
+            f.first = (int32_t)n0;
+            for (int64_t t1 = n1; t1 > n0; t1 -= A->few_chunk) {
+                f.t0 = (int32_t)std::max<int64_t>(n0, t1 - A->few_chunk);
+                f.t1 = (int32_t)t1;
+                launch_few_backward(c->stream, f);
+                launch_few_sums(c->stream, f);
+                f.s0 = f.t0; f.s1 = f.t1;
+            }
+            if (A->all_stages) break;
+        }
+        f.t0 = f.t1 = 0;
+        launch_few_backward(c->stream, f);
+        if (grad_mass) launch_few_mass(c->stream, f, A->mout);
+        HIPCHECK(c, hipGetLastError());
+    }
+    for (int64_t sg = A->few ? -1 : (int64_t)A->ncp - 1; sg >= 0; --sg) {
         const int64_t n0 = sg * A->K, n1 = std::min<int64_t>(A->nsteps, n0 + A->K);
         // recompute the segment's stage states from its checkpoint
         if (A->all_stages) {
@@ -366,7 +497,7 @@ int sol_adjoint_backward(sol_context *c, const double *grad_y_final, double *gra
                                    c->stream));
     }
     if (grad_mass) {
-        launch_adj_mass(c->stream, c->n, A->mbar, A->m0blk, c->nblk, A->mout);
+        if (!A->few) launch_adj_mass(c->stream, c->n, A->mbar, A->m0blk, c->nblk, A->mout);
         HIPCHECK(c, hipMemcpyAsync(grad_mass, A->mout, (size_t)c->n * sizeof(double), hipMemcpyDeviceToHost,
                                    c->stream));
     }

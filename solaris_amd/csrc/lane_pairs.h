@@ -73,6 +73,14 @@ __device__ __forceinline__ void sum8(double (&v)[3])
     for (int k = 0; k < 3; ++k) v[k] += dpp_mov<0x141>(v[k]);
 }
 
+__device__ __forceinline__ double sum8(double v)
+{
+    v += dpp_mov<0xB1>(v);
+    v += dpp_mov<0x4E>(v);
+    v += dpp_mov<0x141>(v);
+    return v;
+}
+
 // Sums over each group of sixteen lanes, in all of them.
 __device__ __forceinline__ void sum16(double (&v)[3])
 {

@@ -126,6 +126,28 @@ struct VjpArgs {
     int32_t src_few;          // source sums by k_vjp_parts (at most 64 sources)
 };
 
+// The adjoint of a system with few sources (adjoint_few.hip): bodies [1, src)
+// are sources, at most kFewMaxSources of them.  Steps are counted from the
+// recorded pass's first; stages holds the stage states of steps first, ...
+constexpr int kFewMaxSources = 32;
+struct FewArgs {
+    int32_t n, np, nm, ea;
+    int32_t eb, src, K, first;
+    int32_t s0, s1, t0, t1;       // steps of the sources' chain and of the sinks'
+    const double *gm, *h;
+    double *y;                    // forward: the state (6 x NP), in place
+    double *stages;               // [step - first][4][6][NP], or null (forward)
+    double *ckpt;                 // forward: every K-th state, or null
+    const double4 *sp_in;         // forward: the sources' stage records of the sinks' chunk
+    double4 *sp_out;              // ... and of the sources' chunk, [step][4][src]
+    double *lam, *mbar, *m0src;   // backward: adjoint state, mass gradients
+    double *u, *sums;
+};
+void launch_few_forward(hipStream_t st, const FewArgs &a);
+void launch_few_backward(hipStream_t st, const FewArgs &a);
+void launch_few_sums(hipStream_t st, const FewArgs &a);
+void launch_few_mass(hipStream_t st, const FewArgs &a, double *out);
+
 // Integrator coefficient tables packed at the offsets the kernels read
 // (275 doubles).
 void fill_coefficients(std::vector<double> &c);
