@@ -8,18 +8,17 @@
 // run on the host, from one 8-byte error maximum per attempt.
 #include <algorithm>
 #include <cmath>
-#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <memory>
-#include <mutex>
 #include <string>
 #include <vector>
 
 #include "context.h"
 #include "tableaux.h"
+#include "unit_lease.h"
 
 using namespace sol;
 
@@ -665,45 +664,6 @@ bool use_resident_any(sol_context *c, int ik) { return path_of(c, ik, nullptr) !
 // that was not resident): the call is to be made again from the same state
 // (on the grid form once more, then on another path).
 constexpr int kGridRetry = -1000;
-
-// The compute units that launches whose workgroups wait for each other (grid
-// and mesh form) hold on a device.  Two such launches of this process that
-// did not fit side by side could each hold a part of the device and wait for
-// the rest, so a launch first takes as many units as it needs, waiting for
-// those of other contexts' launches to end (each at most about 0.2 s).
-class UnitLease {
-public:
-    UnitLease(int device, int units, int total) : d_(pool(device)), units_(std::min(units, total))
-    {
-        std::unique_lock<std::mutex> lock(d_.m);
-        d_.cv.wait(lock, [&] { return d_.used + units_ <= total; });
-        d_.used += units_;
-    }
-    ~UnitLease()
-    {
-        {
-            std::lock_guard<std::mutex> lock(d_.m);
-            d_.used -= units_;
-        }
-        d_.cv.notify_all();
-    }
-    UnitLease(const UnitLease &) = delete;
-    UnitLease &operator=(const UnitLease &) = delete;
-
-private:
-    struct Device {
-        std::mutex m;
-        std::condition_variable cv;
-        int used = 0;
-    };
-    static Device &pool(int device)
-    {
-        static Device devices[64];
-        return devices[device & 63];
-    }
-    Device &d_;
-    int units_;
-};
 
 // Time line, counters, switches and status after a run of the resident
 // drivers that ended with S.

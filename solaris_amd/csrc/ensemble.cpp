@@ -23,6 +23,10 @@
 // 1 << wide_lsh lanes that split its source loop.  Each queue's launch (the
 // counter reset and the kernel) is captured once in a HIP graph of its own
 // and replayed until every system is done.
+//
+// Once the systems still running fit the device at several workgroups each,
+// those with many sources go on in the mesh form (run_mesh), so that the last
+// few do not take their steps on one CU each.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -33,6 +37,8 @@
 
 #include "sol_internal.h"
 #include "resident.h"
+#include "mesh.h"
+#include "unit_lease.h"
 
 using namespace sol;
 
@@ -85,6 +91,19 @@ struct sol_ensemble {
     int graphw_integ = -1, graphw_steps = 0, graph_nw = 0;
     int64_t launches = 0, graph_launches = 0;
     std::vector<int64_t> last_steps;     // per slot: steps of the previous launch
+    // the mesh form for the last systems (mesh.h): their descriptors while it
+    // runs, its copy of the states, k^2 m, positions, parts and exchange words
+    // (mesh_state null: no system of the ensemble can take it, or off)
+    bool mesh_off = false;
+    int mesh_failures = 0;               // launches that gave up; two turn it off
+    double wait_s = 2.0;                 // seconds a wait of it lasts before it gives up
+    uint64_t rtc_hz = 100000000;
+    double *mesh_state = nullptr, *mesh_gm = nullptr, *mesh_pos = nullptr;
+    ResSystem *mesh_sys = nullptr;
+    MeshPart *mesh_part = nullptr;
+    int32_t *mesh_part_of = nullptr;
+    MeshSync *mesh_sync = nullptr;
+    std::vector<double> gm_h;
 
     int fail(int code, const std::string &m) { err = m; return code; }
 };
@@ -96,6 +115,9 @@ struct sol_ensemble {
     } while (0)
 
 namespace {
+
+// Accepted steps of a run's first launch.
+constexpr int kFirstSteps = 16;
 
 int nmassive(const sol_nbodies &b) { return b.central_body + b.giant_planet + b.rocky_planet + b.proto_planet; }
 
@@ -137,6 +159,12 @@ int upload(sol_ensemble *e)
                                  e->stream));
         ECHECK(e, hipMemcpyAsync(e->mass, e->mass_h.data(), e->mass_h.size() * sizeof(double),
                                  hipMemcpyHostToDevice, e->stream));
+        if (e->mesh_state) {
+            e->gm_h.resize(e->mass_h.size());
+            for (size_t i = 0; i < e->mass_h.size(); ++i) e->gm_h[i] = kGauss2 * e->mass_h[i];
+            ECHECK(e, hipMemcpyAsync(e->mesh_gm, e->gm_h.data(), e->gm_h.size() * sizeof(double),
+                                     hipMemcpyHostToDevice, e->stream));
+        }
     }
     if (e->sys_dirty)
         ECHECK(e, hipMemcpyAsync(e->sys_d, e->sys_h.data(), e->sys_h.size() * sizeof(ResSystem),
@@ -165,16 +193,16 @@ int grid_for(sol_ensemble *e, int ik, int block, int nrun)
 
 bool is_wide(const sol_ensemble *e, int s) { return e->wide_block > 0 && e->sys_h[s].n >= e->wide_min; }
 
-// Queue orders for the next launch: the running systems of each queue
-// (the narrow one only when `narrow_only`), the most work expected first
+// Queue orders for the next launch: the running systems of each queue that
+// have not had their steps (the narrow one only when `narrow_only`), the most work expected first
 // (n^2 times the steps the system took in the previous launch, n^2 alone
 // before the first), so that the long ones start early.
-int make_order(sol_ensemble *e, bool narrow_only = false)
+int make_order(sol_ensemble *e, bool narrow_only = false, const std::vector<char> *had = nullptr)
 {
     e->order_h.clear();
     e->order_w.clear();
     for (int s = 0; s < e->nsys; ++s) {
-        if (e->sys_h[s].status != RES_RUNNING) continue;
+        if (e->sys_h[s].status != RES_RUNNING || (had && (*had)[s])) continue;
         if (!is_wide(e, s)) e->order_h.push_back(s);
         else if (!narrow_only) e->order_w.push_back(s);
     }
@@ -280,6 +308,97 @@ int read_systems(sol_ensemble *e)
     ECHECK(e, hipMemcpyAsync(e->sys_h.data(), e->sys_d, e->sys_h.size() * sizeof(ResSystem), hipMemcpyDeviceToHost,
                              e->stream));
     ECHECK(e, hipStreamSynchronize(e->stream));
+    return SOL_OK;
+}
+
+// The mesh form (mesh.hip) takes systems whose larger class of bodies has at
+// least this many sources: per RKF78 attempt in the queue and in the mesh form
+// 33 bodies take 48 and 47 us, 49 bodies 54 and 48, 66 69 and 50, 97 63 and
+// 51, 129 104 and 54, 193 138 and 56, 257 324 and 69.
+constexpr int kMeshMinSources = 48;
+
+bool mesh_takes(const ResSystem &S) { return std::max(S.end_a, S.end_b) >= kMeshMinSources; }
+
+// Runs `steps` accepted steps of the running systems that the mesh form
+// takes, over several workgroups each, if all of them fit the device at once;
+// `had` marks them, and the caller's next queue launch leaves them out.  A
+// run lasts as long as its slowest systems, which leave most of the device
+// idle once the others are done: 1,024 systems over two days, of 3 to 257
+// bodies and 9 steps in the mean, have 31 to 49 systems of more than 16 steps
+// and need up to 504; 46 to 145 ms with the queue alone, 25 to 53 with these
+// in the mesh form.  (Several launches of it in turn for more systems than
+// fit gained nothing over the queue.)
+int run_mesh(sol_ensemble *e, int ik, int steps, std::vector<char> &had)
+{
+    had.assign((size_t)e->nsys, 0);
+    if (!e->mesh_state || e->mesh_off) return SOL_OK;
+    std::vector<int> slots;
+    int max_n = 0;
+    for (int s = 0; s < e->nsys; ++s)
+        if (e->sys_h[s].status == RES_RUNNING && mesh_takes(e->sys_h[s])) {
+            slots.push_back(s);
+            max_n = std::max(max_n, e->sys_h[s].n);
+        }
+    if (slots.empty() || (int)slots.size() > e->cu_count) return SOL_OK;
+    // the smallest share of bodies per workgroup with which they fit
+    auto groups_of = [&](int s, int share) {
+        const ResSystem &S = e->sys_h[s];
+        return mesh_groups(S.n, S.nm, S.end_a, S.end_b, share);
+    };
+    int share = 7, groups = 0;
+    for (;; share += 8) {
+        if (share > kMeshMaxShare) return SOL_OK;
+        groups = 0;
+        int most = 0;
+        for (int s : slots) {
+            const int g = groups_of(s, share);
+            groups += g;
+            most = std::max(most, g);
+        }
+        if (most <= kMeshMaxGroups && groups <= e->cu_count &&
+            groups <= mesh_capacity(ik, max_n, share, e->cu_count)) break;
+    }
+    std::vector<MeshPart> parts;
+    std::vector<int32_t> part_of;
+    std::vector<int64_t> before;
+    for (int s : slots) {
+        const int g = groups_of(s, share);
+        parts.push_back(MeshPart{s, (int32_t)part_of.size(), g, share});
+        part_of.insert(part_of.end(), (size_t)g, (int32_t)parts.size() - 1);
+        before.push_back(e->sys_h[s].steps);
+    }
+    ECHECK(e, hipMemcpyAsync(e->mesh_part, parts.data(), parts.size() * sizeof(MeshPart), hipMemcpyHostToDevice,
+                             e->stream));
+    ECHECK(e, hipMemcpyAsync(e->mesh_part_of, part_of.data(), part_of.size() * sizeof(int32_t),
+                             hipMemcpyHostToDevice, e->stream));
+    ECHECK(e, hipMemcpyAsync(e->mesh_sys, e->sys_d, (size_t)e->nsys * sizeof(ResSystem), hipMemcpyDeviceToDevice,
+                             e->stream));
+    MeshArgs A{};
+    A.systems = e->mesh_sys;
+    A.parts = e->mesh_part; A.part_of = e->mesh_part_of;
+    A.sync = e->mesh_sync;
+    A.pos = e->mesh_pos; A.gm = e->mesh_gm;
+    A.tot = e->tot;
+    A.y0_in = e->y0; A.mass = e->mass;
+    A.y0 = e->mesh_state; A.y = e->y; A.acc0 = e->acc0; A.yscale = e->yscale; A.err = e->errv;
+    A.rm3 = e->rm3; A.nnd = e->nnd; A.nni = e->nni;
+    A.ticks = (uint64_t)(e->wait_s * (double)e->rtc_hz);
+    {
+        const UnitLease lease(e->device, groups, e->cu_count);
+        ECHECK(e, launch_mesh(e->stream, ik, A, (int)parts.size(), groups, max_n, share, steps));
+        ECHECK(e, launch_mesh_commit(e->stream, A, (int)parts.size(), e->sys_d, e->y0));
+        if (int r = read_systems(e)) return r;
+    }
+    // a system whose workgroups were not all resident has kept its state, and
+    // the queue takes it
+    bool lost = false;
+    for (size_t p = 0; p < parts.size(); ++p) {
+        const ResSystem &S = e->sys_h[parts[p].system];
+        const bool ran = S.status != RES_RUNNING || S.steps != before[p];
+        had[parts[p].system] = ran;
+        lost |= !ran;
+    }
+    if (lost && ++e->mesh_failures >= 2) e->mesh_off = true;
     return SOL_OK;
 }
 
@@ -457,6 +576,31 @@ int sol_ensemble_create(sol_ensemble **out, int32_t nsys, const sol_nbodies *nbs
         sol_ensemble_destroy(e);
         return r;
     }
+    bool mesh = false;
+    for (int k = 0; k < nsys; ++k) {
+        ResSystem S{};
+        S.n = nbs[k].total;
+        S.nm = nmassive(nbs[k]);
+        S.end_a = S.nm + nbs[k].super_planetesimal;
+        S.end_b = S.nm;
+        mesh |= mesh_takes(S);
+    }
+    if (const char *w = std::getenv("SOLARIS_AMD_NO_GRID")) mesh &= w[0] != '1';
+    if (const char *w = std::getenv("SOLARIS_AMD_GRID_WAIT")) e->wait_s = std::max(0.0, std::atof(w));
+    {
+        int khz = 0;
+        if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0)
+            e->rtc_hz = (uint64_t)khz * 1000;
+    }
+    const size_t most = (size_t)e->cu_count;      // parts, and workgroups, of a mesh launch
+    if (mesh && ((r = ealloc(e, &e->mesh_state, 6 * tot)) || (r = ealloc(e, &e->mesh_gm, tot)) ||
+                 (r = ealloc(e, &e->mesh_pos, 6 * tot)) || (r = ealloc(e, &e->mesh_sys, nsys)) ||
+                 (r = ealloc(e, &e->mesh_part, most)) || (r = ealloc(e, &e->mesh_part_of, most)) ||
+                 (r = ealloc(e, &e->mesh_sync, most)))) {
+        g_ens_create_error = e->err;
+        sol_ensemble_destroy(e);
+        return r;
+    }
     e->y0_h.assign(6 * tot, 0.0);
     e->mass_h.assign(tot, 0.0);
     e->sys_h.assign(nsys, ResSystem{});
@@ -483,7 +627,9 @@ int sol_ensemble_destroy(sol_ensemble *e)
     if (e->graph) (void)hipGraphExecDestroy(e->graph);
     if (e->graph_w) (void)hipGraphExecDestroy(e->graph_w);
     void *ptrs[] = {e->sys_d, e->y0,  e->y,   e->acc0, e->yscale,  e->errv,  e->fst,
-                    e->mass,  e->rm3, e->nnd, e->nni,  e->order_d, e->head_d};
+                    e->mass,  e->rm3, e->nnd, e->nni,  e->order_d, e->head_d,
+                    e->mesh_state, e->mesh_gm, e->mesh_pos, e->mesh_sys, e->mesh_part, e->mesh_part_of,
+                    e->mesh_sync};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (e->ev_fork) (void)hipEventDestroy(e->ev_fork);
@@ -574,21 +720,29 @@ int sol_ensemble_run(sol_ensemble *e, int32_t integrator, double eps, int64_t ma
     const double per_step = 13.0 * (3000.0 + 12.0 * e->nmax) / 2.1e9;
     int chunk = (int)std::max<int64_t>(16, std::min<int64_t>(20000, (int64_t)(0.25 / per_step)));
     if (max_steps > 0) chunk = (int)std::min<int64_t>(chunk, max_steps);
+    // where the last systems may take the mesh form, the launches start short
+    // and grow, so that few running systems are soon noticed (run_mesh)
+    int next = e->mesh_state && !e->mesh_off ? std::min(chunk, kFirstSteps) : chunk;
+    std::vector<char> had((size_t)e->nsys, 0);
     hipEvent_t t0, t1;
     ECHECK(e, hipEventCreate(&t0));
     ECHECK(e, hipEventCreate(&t1));
     ECHECK(e, hipEventRecord(t0, e->stream));
     int64_t done_steps = 0;
     for (;;) {
-        int k = chunk;
+        int k = next;
+        next = std::min(2 * next, chunk);
         if (max_steps > 0) k = (int)std::min<int64_t>(k, max_steps - done_steps);
-        if (int r = make_order(e)) return r;
-        if (e->order_h.empty() && e->order_w.empty()) break;
         std::vector<int64_t> before(e->nsys);
         for (int s = 0; s < e->nsys; ++s) before[s] = e->sys_h[s].steps;
-        if (int r = launch_queue(e, ik, k, e->block, true)) return r;
+        if (done_steps > 0)
+            if (int r = run_mesh(e, ik, k, had)) return r;
+        if (int r = make_order(e, false, &had)) return r;
+        if (!e->order_h.empty() || !e->order_w.empty()) {
+            if (int r = launch_queue(e, ik, k, e->block, true)) return r;
+            if (int r = read_systems(e)) return r;
+        }
         done_steps += k;
-        if (int r = read_systems(e)) return r;
         for (int s = 0; s < e->nsys; ++s) e->last_steps[s] = e->sys_h[s].steps - before[s];
         const bool any = std::any_of(e->sys_h.begin(), e->sys_h.end(), [](const ResSystem &S) { return S.status == RES_RUNNING; });
         if (!any) break;

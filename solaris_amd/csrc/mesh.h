@@ -58,6 +58,11 @@ int mesh_groups(int n, int nm, int end_a, int end_b, int share);
 // groups and has to be resident at once.
 hipError_t launch_mesh(hipStream_t st, int integ, const MeshArgs &a, int nparts, int ngroups, int max_n,
                        int max_share, int max_steps);
+// After that launch: the state of every part that ran to its end (no wait
+// timed out) into y0 (component stride tot) and its descriptor into systems.
+// The mesh launch itself may have written some workgroups' rows of a part
+// that did not, so y0 is another array than a.y0, and systems than a.systems.
+hipError_t launch_mesh_commit(hipStream_t st, const MeshArgs &a, int nparts, ResSystem *systems, double *y0);
 // Workgroups of that launch the device holds at once.
 int mesh_capacity(int integ, int n, int share, int cu_count);
 

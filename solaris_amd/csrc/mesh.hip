@@ -746,6 +746,19 @@ __global__ __launch_bounds__(256) void k_mesh_zero(MeshSync *s)
     }
 }
 
+__global__ __launch_bounds__(256) void k_mesh_commit(MeshArgs A, ResSystem *systems, double *y0)
+{
+    const int psys = A.parts[blockIdx.x].system;
+    const ResSystem &S = A.systems[psys];
+    if (A.sync[blockIdx.x].error != 0 || S.status == RES_SYNC_ERROR) return;
+    const int n = S.n;
+    for (int q = threadIdx.x; q < 6 * n; q += blockDim.x) {
+        const int64_t o = q / n * A.tot + S.base + q % n;
+        y0[o] = A.y0[o];
+    }
+    if (threadIdx.x == 0) systems[psys] = S;
+}
+
 // The smallest of 8, 16, 24 and 32 places that holds `share` bodies and the
 // one at the origin.
 template <int INTEG>
@@ -811,6 +824,13 @@ hipError_t launch_mesh(hipStream_t st, int integ, const MeshArgs &a, int nparts,
     const size_t lds = mesh_tile_bytes(max_n, &records);
     void *kargs[] = {&args, &max_steps, &records};
     return hipLaunchKernel(mesh_kernel(integ, max_share), dim3(ngroups), dim3(kMeshThreads), kargs, lds, st);
+}
+
+hipError_t launch_mesh_commit(hipStream_t st, const MeshArgs &a, int nparts, ResSystem *systems, double *y0)
+{
+    if (nparts < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_mesh_commit, dim3(nparts), dim3(256), 0, st, a, systems, y0);
+    return hipGetLastError();
 }
 
 }  // namespace sol
