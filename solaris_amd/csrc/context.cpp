@@ -159,10 +159,18 @@ void build_plan(sol_context *c)
     // largest M such that every body of [1, M) is a source of every other
     const int M = std::min(ea, eb) > nm ? std::min(std::min(ea, eb), c->n) : std::min(nm, ea);
     if (M - 1 < kSymMinBodies) return;
-    // 4 waves per SIMD (two rounds at the kernel's occupancy of two);
+    // Workgroups of the same number of items k each, at most 26 per CU (of
+    // which 3 or 4 run at a time): short ones fill the device evenly to the
+    // end, and each adds a record per column it touches to the epilogue's
+    // reads.  k = 1, 2, 3, 4, 5: at 32,769 bodies 482, 460, 450, 481 (k = 4)
+    // and 509 us for FP64 with 2 or 3 items in a workgroup; at 65,537 1,604
+    // (k = 5) to 1,697 (k = 8) and 1,683 (k = 1), the epilogue 54, 49 and 90.
     // SOLARIS_AMD_SYM_WAVES overrides the count (tests use it to give each
-    // wave many items)
-    int64_t waves = (int64_t)c->cu_count * 4 * 4;
+    // workgroup many items).
+    const int64_t groups = (M - 1 + kSymGroup - 1) / kSymGroup, items = groups * (groups + 1) / 2;
+    const int64_t most = (int64_t)c->cu_count * 26;
+    const int64_t per = (items + most - 1) / most;
+    int64_t waves = (items + per - 1) / per;
     if (const char *e = std::getenv("SOLARIS_AMD_SYM_WAVES")) {
         const long v = std::atol(e);
         if (v > 0) waves = v;

@@ -298,29 +298,67 @@ void launch_mixed(hipStream_t st, const PairPlan &plan, const float4 *J32, const
 }
 
 // ---- symmetric pair sum over the mutual block ------------------------------
-// One wave per range of group-pair items (sym_plan.h).  The wave holds the
-// 256 bodies of the row group, four per lane, and streams the column group
-// as four packets of 64 bodies.  At step k (0..63) lane l pairs its four
-// row bodies with packet body (l + k) mod 64: the packet's positions and
-// k^2 m are read from the wave's own LDS slice, where the packet is stored
-// twice in a row so that entry l + k needs no wrap, and the packet's force
-// sums travel with it, rotating one lane per step (DPP wave_rol:1); after
-// 64 steps every row body has met every packet body and the sums are back
-// on their lanes.  Each step evaluates four pairs per lane and forms both
-// accelerations from each, so a pair of the block costs one reciprocal
-// square root and 20 FP64 operations for two interactions, plus 6 rotated
-// dwords and two 16-byte LDS reads per step of four pairs.  In a diagonal
-// item (row == column) the row tile t meets packet j only for t < j, and
-// for t == j at steps 1..32 (step 32 on lanes 0..31): each unordered pair
-// once, no self pair.
+// One workgroup of four waves per range of group-pair items (sym_plan.h).
+// Every wave holds the 256 bodies of the column group, four per lane, over
+// the consecutive items of a column, and streams one packet of 64 bodies of
+// the row group per item: wave j packet j.  At step k (0..63) lane l pairs
+// its four column bodies with packet body (l + k) mod 64: the packet's
+// positions and k^2 m are read from the wave's own LDS slice, where the
+// packet is stored twice in a row so that entry l + k needs no wrap, and the
+// packet's force sums travel with it, rotating one lane per step (DPP
+// wave_rol:1); after 64 steps every column body has met every packet body,
+// the sums are back on their lanes and go to the item's row record.  Each
+// step evaluates four pairs per lane and forms both accelerations from each,
+// so a pair of the block costs one reciprocal square root and 20 FP64
+// operations for two interactions, plus 6 rotated dwords and two 16-byte LDS
+// reads per step of four pairs.  The four waves' column sums are added in LDS
+// when the column changes.
+//
+// What bounds it: the FP64 issue (20 operations of 2.0 ns per wave at the
+// clock under this load and one v_rsq_f64 of 7.1 ns: 47 of the measured 50 ns
+// per wave's pair at 65,537 bodies), once every SIMD has two waves.  A wave
+// alone takes 60 us over the pairs of an item, so with whole items per wave
+// 2,000 to 5,000 bodies took that time and 16,385 (2,080 items on 2,048
+// places) twice a round; a quarter of an item per wave, and no column sums
+// but the current ones in registers (164 VGPRs and three waves per SIMD; with
+// the row sums held and the columns carried 246 and two), measured before and
+// after, us: 3,001 bodies 59 and 21, 5,001 61 and 23, 8,193 65 and 47, 12,001
+// 115 and 76, 16,385 168 and 125, 32,769 526 and 460, 65,537 1,676 and 1,604.
+//
+// In a diagonal item (row == column) wave j meets the column tile t by
+// d = (t - j) mod 4: for d == 0 at steps 1..32 (step 32 on lanes 0..31), for
+// d == 1 at all steps, and for d == 2 the tile pair is met by two waves, by
+// the lower one at steps 0..31 and by the other at 1..32 (its step k is the
+// other's step -k mod 64): each unordered pair once, no self pair, and two
+// tiles' work for each wave.
 // Bodies past the end of the block are far sentinels of zero mass at
-// +1e30 AU (row side) and -1e30 AU (column side), so that no pair has zero
+// +1e30 AU (column side) and -1e30 AU (row side), so that no pair has zero
 // distance; their sums are never read.
 //
-// The LDS slices are private to their waves, and the four waves of a block
-// run different item ranges, so there is no block barrier: a wave's LDS
-// operations execute in order, and a wavefront-scope fence keeps the
-// compiler from moving a packet's reads across the stores of the next.
+// The packets' LDS slices are private to their waves: a wave's LDS operations
+// execute in order, and a wavefront-scope fence keeps the compiler from moving
+// a packet's reads across the stores of the next.  The block meets at barriers
+// only where a column's sums are added up.
+
+// Diagonal item: does wave j meet column tile t at step k, and on all lanes?
+__device__ __forceinline__ bool sym_diag_meets(int t, int j, int k)
+{
+    const int d = (t - j) & 3;
+    return d == 1 || (d == 0 && k >= 1 && k <= 32) || (d == 2 && (j < 2 ? k < 32 : (k >= 1 && k <= 32)));
+}
+__device__ __forceinline__ bool sym_diag_half(int t, int j, int k) { return t == j && k == 32; }
+
+// Adds the four waves' column sums (three components of 256 bodies each, in
+// lds) into the record q.
+__device__ __forceinline__ void sym_flush(const double (*lds)[3][kSymGroup], double *__restrict__ q)
+{
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        q[c * kSymGroup + threadIdx.x] = (lds[0][c][threadIdx.x] + lds[1][c][threadIdx.x]) +
+                                         (lds[2][c][threadIdx.x] + lds[3][c][threadIdx.x]);
+    __syncthreads();
+}
 
 __device__ __forceinline__ double rot_lane(double v)
 {
@@ -353,99 +391,90 @@ __device__ __forceinline__ void sym_pair(double x, double y, double z, double gm
     gz = __builtin_fma(-fb, dz, gz);
 }
 
-// 246 VGPRs, two waves per SIMD: bounding it to three (168 VGPRs, four
-// values spilled outside the step loop) measured 1.1% slower at C3
 template <bool SOFT>
-__global__ __launch_bounds__(256) void k_pairs_sym_fp64(SymPlan sp, const double4 *__restrict__ J,
-                                                        double *__restrict__ apart, double *__restrict__ bpart,
-                                                        double eps2, double c15, double c1875)
+__global__ __launch_bounds__(kBlock) void k_pairs_sym_fp64(SymPlan sp, const double4 *__restrict__ J,
+                                                           double *__restrict__ apart, double *__restrict__ bpart,
+                                                           double eps2, double c15, double c1875)
 {
-    __shared__ double4 pk_lds[kBlock / kWave][2 * kWave];
+    __shared__ double4 pk_lds[kSymWaves][2 * kWave];
+    __shared__ double sums[kSymWaves][3][kSymGroup];
     const int lane = threadIdx.x & (kWave - 1);
-    const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int w = blockIdx.x * (kBlock / kWave) + wib;
-    if (w >= sp.nwaves) return;
+    const int j = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int w = blockIdx.x;
     const int64_t lo = sym_wave_lo(sp, w), hi = sym_wave_lo(sp, w + 1);
     if (lo >= hi) return;
-    int a0, h0;
-    sym_decode(lo, a0, h0);
-    int hcur = -1;
-    double bs[4][3];                         // column-side sums of the current column group
-    double4 *pk = pk_lds[wib];
-
-    auto flush_col = [&]() {
-        double *q = bpart + ((int64_t)w * sp.slots_per_wave + (hcur - h0)) * (3 * kSymGroup);
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) q[c * kSymGroup + t * kWave + lane] = bs[t][c];
-    };
-
-    for (int64_t it = lo; it < hi; ++it) {
-        int ag, hg;
-        sym_decode(it, ag, hg);
-        if (hg != hcur) {
-            if (hcur >= 0) flush_col();
-            hcur = hg;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) bs[t][0] = bs[t][1] = bs[t][2] = 0.0;
-        }
-        double px[4], py[4], pz[4], pm[4], fx[4], fy[4], fz[4];
+    int ag, hg;
+    sym_decode(lo, ag, hg);
+    double4 *pk = pk_lds[j];
+    double *record = bpart + (int64_t)w * sp.slots_per_wave * (3 * kSymGroup);
+    double px[4], py[4], pz[4], pm[4], fx[4], fy[4], fz[4];
+    auto load_col = [&]() {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const int ia = 1 + ag * kSymGroup + t * kWave + lane;
+            const int ia = 1 + hg * kSymGroup + t * kWave + lane;
             const double4 v = ia < sp.M ? J[ia] : make_double4(1.0e30, 0.0, 0.0, 0.0);
             px[t] = v.x; py[t] = v.y; pz[t] = v.z; pm[t] = v.w;
             fx[t] = fy[t] = fz[t] = 0.0;
         }
-        const bool diag = (ag == hg);
-        for (int j = 0; j < 4; ++j) {
-            const int ib = 1 + hg * kSymGroup + j * kWave + lane;
-            const double4 q0 = ib < sp.M ? J[ib] : make_double4(-1.0e30, 0.0, 0.0, 0.0);
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            pk[lane] = q0;
-            pk[lane + kWave] = q0;
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            double gx = 0.0, gy = 0.0, gz = 0.0;
-            // one step: the four row bodies against packet body q, then the
-            // packet's sums move one lane on
-            auto step = [&](const double4 &q, int k, auto diag_c) {
-                constexpr bool D = decltype(diag_c)::value;
+    };
+    load_col();
+    for (int64_t it = lo;; ) {
+        const int ib = 1 + ag * kSymGroup + j * kWave + lane;
+        const double4 q0 = ib < sp.M ? J[ib] : make_double4(-1.0e30, 0.0, 0.0, 0.0);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        pk[lane] = q0;
+        pk[lane + kWave] = q0;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        double gx = 0.0, gy = 0.0, gz = 0.0;
+        // one step: the four column bodies against packet body q, then the
+        // packet's sums move one lane on
+        auto step = [&](const double4 &q, int k, auto diag_c) {
+            constexpr bool D = decltype(diag_c)::value;
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    if (!D || t < j || (t == j && k >= 1 && (k < 32 || (k == 32 && lane < 32))))
-                        sym_pair<SOFT>(px[t], py[t], pz[t], pm[t], q, eps2, c15, c1875, fx[t], fy[t], fz[t],
-                                       gx, gy, gz);
-                }
-                gx = rot_lane(gx); gy = rot_lane(gy); gz = rot_lane(gz);
-            };
-            // two steps per iteration, each step's packet body read one step
-            // ahead (entry lane + k + 2 <= 127 stays in the slice)
-            auto steps = [&](auto diag_c) {
-                double4 qa = pk[lane];
-                for (int k = 0; k < kWave; k += 2) {
-                    const double4 qb = pk[lane + k + 1];
-                    step(qa, k, diag_c);
-                    qa = pk[lane + k + 2];
-                    step(qb, k + 1, diag_c);
-                }
-            };
-            if (diag) steps(std::true_type{}); else steps(std::false_type{});
-            bs[j][0] += gx;
-            bs[j][1] += gy;
-            bs[j][2] += gz;
-        }
-        double *r = apart + it * (3 * kSymGroup);
+            for (int t = 0; t < 4; ++t) {
+                if (!D || (sym_diag_meets(t, j, k) && (!sym_diag_half(t, j, k) || lane < 32)))
+                    sym_pair<SOFT>(px[t], py[t], pz[t], pm[t], q, eps2, c15, c1875, fx[t], fy[t], fz[t],
+                                   gx, gy, gz);
+            }
+            gx = rot_lane(gx); gy = rot_lane(gy); gz = rot_lane(gz);
+        };
+        // two steps per iteration, each step's packet body read one step
+        // ahead (entry lane + k + 2 <= 127 stays in the slice)
+        auto steps = [&](auto diag_c) {
+            double4 qa = pk[lane];
+            for (int k = 0; k < kWave; k += 2) {
+                const double4 qb = pk[lane + k + 1];
+                step(qa, k, diag_c);
+                qa = pk[lane + k + 2];
+                step(qb, k + 1, diag_c);
+            }
+        };
+        if (ag == hg) steps(std::true_type{}); else steps(std::false_type{});
+        double *r = apart + it * (3 * kSymGroup) + j * kWave + lane;
+        r[0] = gx;
+        r[kSymGroup] = gy;
+        r[2 * kSymGroup] = gz;
+        ++it;
+        const bool last = it >= hi;
+        if (last || ag == hg) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            r[t * kWave + lane] = fx[t];
-            r[kSymGroup + t * kWave + lane] = fy[t];
-            r[2 * kSymGroup + t * kWave + lane] = fz[t];
+            for (int t = 0; t < 4; ++t) {
+                sums[j][0][t * kWave + lane] = fx[t];
+                sums[j][1][t * kWave + lane] = fy[t];
+                sums[j][2][t * kWave + lane] = fz[t];
+            }
+            sym_flush(sums, record);
+            if (last) break;
+            record += 3 * kSymGroup;
+            ++hg;
+            ag = 0;
+            load_col();
+        } else {
+            ++ag;
         }
     }
-    if (hcur >= 0) flush_col();
 }
 
 __device__ __forceinline__ float rot_lane_f(float v)
@@ -456,7 +485,7 @@ __device__ __forceinline__ float rot_lane_f(float v)
 // Mixed-precision form of k_pairs_sym_fp64: FP32 pair terms from J32 (and
 // FP32 sums over the 256 bodies an item pairs with each body, folded into
 // FP64), with the close pairs evaluated in FP64.  A pair is close when
-// |d|^2 < near_frac2 |r_a|^2, r_a the row body (one decision for both
+// |d|^2 < near_frac2 |r_a|^2, r_a the column body (one decision for both
 // bodies; a close pair has |r_b| = |r_a| to within |d|, so this is the
 // one-directional kernel's test, |d| < near_frac |r_i|, from either side).
 // The softening is folded into the squared distance (rs = eps2 + dx^2 +
@@ -471,169 +500,162 @@ __device__ __forceinline__ float rot_lane_f(float v)
 // (positions from J) to FP64 sums that travel with the packet.  As in the
 // FP64 kernel the packet's (x, y, z, k^2 m) are read from the wave's LDS
 // slice, one 16-byte read per step, and only its three FP32 sums rotate.
-// Per pair: 17 FP32 VALU operations and one v_rsq_f32.
-// At least four waves per SIMD (128 VGPRs; six values spilled outside the
-// step loop): 1.5% faster at C3 than the unbounded three waves
+// Per pair: 17 FP32 VALU operations and one v_rsq_f32.  Four waves per SIMD.
+// Measured before (whole items per wave) and after, us: 5,001 bodies 82 and
+// 44, 16,385 110 and 93, 32,769 339 and 277, 65,537 1,070 and 868.
 template <bool SOFT>
 __global__ __launch_bounds__(256, 4) void k_pairs_sym_mixed(SymPlan sp, const float4 *__restrict__ J32,
                                                          const double4 *__restrict__ J, double *__restrict__ apart,
                                                          double *__restrict__ bpart, float eps2, double eps2d,
                                                          float near_frac2, double c15, double c1875)
 {
-    __shared__ float4 pk_lds[kBlock / kWave][2 * kWave];
+    __shared__ float4 pk_lds[kSymWaves][2 * kWave];
+    __shared__ double sums[kSymWaves][3][kSymGroup];
     const int lane = threadIdx.x & (kWave - 1);
-    const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int w = blockIdx.x * (kBlock / kWave) + wib;
-    if (w >= sp.nwaves) return;
+    const int j = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int w = blockIdx.x;
     const int64_t lo = sym_wave_lo(sp, w), hi = sym_wave_lo(sp, w + 1);
     if (lo >= hi) return;
-    int a0, h0;
-    sym_decode(lo, a0, h0);
-    int hcur = -1;
-    double bs[4][3];
+    int ag, hg;
+    sym_decode(lo, ag, hg);
     const float e2 = SOFT ? eps2 : 0.0f;
-    float4 *pk = pk_lds[wib];
-
-    auto flush_col = [&]() {
-        double *q = bpart + ((int64_t)w * sp.slots_per_wave + (hcur - h0)) * (3 * kSymGroup);
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) q[c * kSymGroup + t * kWave + lane] = bs[t][c];
-    };
-    // diagonal items: row tile t meets packet j for t < j, and for t == j at
-    // steps 1..32 (wave-uniform tests); at step 32 of t == j only lanes 0..31
-    // take the pair, which is masked arithmetically, not branched on, so that
-    // every lane reaches the packet rotations and the FP32 pass has no
-    // divergent branch (its close-pair mask stays wave-uniform)
-    auto skip = [&](bool diag, int t, int j, int k) { return diag && (t > j || (t == j && (k < 1 || k > 32))); };
-    auto masked = [&](bool diag, int t, int j, int k) { return diag && t == j && k == 32 && lane >= 32; };
-
-    for (int64_t it = lo; it < hi; ++it) {
-        int ag, hg;
-        sym_decode(it, ag, hg);
-        if (hg != hcur) {
-            if (hcur >= 0) flush_col();
-            hcur = hg;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) bs[t][0] = bs[t][1] = bs[t][2] = 0.0;
-        }
-        float px[4], py[4], pz[4], pm[4], th[4];
-        double ax[4], ay[4], az[4];
+    float4 *pk = pk_lds[j];
+    double *record = bpart + (int64_t)w * sp.slots_per_wave * (3 * kSymGroup);
+    float px[4], py[4], pz[4], pm[4], th[4];
+    double ax[4], ay[4], az[4];
+    auto load_col = [&]() {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const int ia = 1 + ag * kSymGroup + t * kWave + lane;
+            const int ia = 1 + hg * kSymGroup + t * kWave + lane;
             const float4 v = ia < sp.M ? J32[ia] : make_float4(1.0e18f, 0.0f, 0.0f, 0.0f);
             px[t] = v.x; py[t] = v.y; pz[t] = v.z; pm[t] = v.w;
             th[t] = __builtin_fmaf(near_frac2, __builtin_fmaf(v.z, v.z, __builtin_fmaf(v.y, v.y, v.x * v.x)), e2);
             ax[t] = ay[t] = az[t] = 0.0;
         }
+    };
+    // diagonal items: the step-32 pairs of a tile with itself are taken by
+    // lanes 0..31 only, which is masked arithmetically, not branched on, so
+    // that every lane reaches the packet rotations and the FP32 pass has no
+    // divergent branch (its close-pair mask stays wave-uniform)
+    auto skip = [&](bool diag, int t, int k) { return diag && !sym_diag_meets(t, j, k); };
+    auto masked = [&](bool diag, int t, int k) { return diag && sym_diag_half(t, j, k) && lane >= 32; };
+
+    load_col();
+    for (int64_t it = lo;; ) {
         const bool diag = (ag == hg);
-        for (int j = 0; j < 4; ++j) {
-            const int ib = 1 + hg * kSymGroup + j * kWave + lane;
-            const float4 v = ib < sp.M ? J32[ib] : make_float4(-1.0e18f, 0.0f, 0.0f, 0.0f);
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            pk[lane] = v;
-            pk[lane + kWave] = v;
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            float fx[4] = {0.f, 0.f, 0.f, 0.f}, fy[4] = {0.f, 0.f, 0.f, 0.f}, fz[4] = {0.f, 0.f, 0.f, 0.f};
-            float gx = 0.f, gy = 0.f, gz = 0.f;
-            uint64_t wave_far = ~0ull;   // lanes that met no close pair in this packet's pass
-            // one FP32 step against packet body q; the diagonal test is
-            // resolved at compile time so that the off-diagonal loop has no branch
-            auto step = [&](const float4 &q, int k, auto diag_c) {
-                constexpr bool D = decltype(diag_c)::value;
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    if (D && skip(true, t, j, k)) continue;
-                    const bool off = D && masked(true, t, j, k);
-                    const float dx = q.x - px[t], dy = q.y - py[t], dz = q.z - pz[t];
-                    const float rs = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, e2)));
-                    const float y0 = __builtin_amdgcn_rsqf(rs);
-                    const bool far = !(rs < th[t]);
-                    wave_far &= __ballot(far);
-                    if (far && !off) {
-                        const float wv = y0 * (y0 * y0);
-                        const float fa = q.w * wv, fb = pm[t] * wv;
-                        fx[t] = __builtin_fmaf(fa, dx, fx[t]);
-                        fy[t] = __builtin_fmaf(fa, dy, fy[t]);
-                        fz[t] = __builtin_fmaf(fa, dz, fz[t]);
-                        gx = __builtin_fmaf(-fb, dx, gx);
-                        gy = __builtin_fmaf(-fb, dy, gy);
-                        gz = __builtin_fmaf(-fb, dz, gz);
-                    }
-                }
-                gx = rot_lane_f(gx); gy = rot_lane_f(gy); gz = rot_lane_f(gz);
-            };
-            // two steps per iteration, each packet body read one step ahead
-            // (entry lane + k + 2 <= 127 stays in the slice)
-            auto fp32_pass = [&](auto diag_c) {
-                float4 qa = pk[lane];
-                for (int k = 0; k < kWave; k += 2) {
-                    const float4 qb = pk[lane + k + 1];
-                    step(qa, k, diag_c);
-                    qa = pk[lane + k + 2];
-                    step(qb, k + 1, diag_c);
-                }
-            };
-            if (diag) fp32_pass(std::true_type{}); else fp32_pass(std::false_type{});
+        const int ib = 1 + ag * kSymGroup + j * kWave + lane;
+        const float4 v = ib < sp.M ? J32[ib] : make_float4(-1.0e18f, 0.0f, 0.0f, 0.0f);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        pk[lane] = v;
+        pk[lane + kWave] = v;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        float fx[4] = {0.f, 0.f, 0.f, 0.f}, fy[4] = {0.f, 0.f, 0.f, 0.f}, fz[4] = {0.f, 0.f, 0.f, 0.f};
+        float gx = 0.f, gy = 0.f, gz = 0.f;
+        uint64_t wave_far = ~0ull;   // lanes that met no close pair in this packet's pass
+        // one FP32 step against packet body q; the diagonal test is
+        // resolved at compile time so that the off-diagonal loop has no branch
+        auto step = [&](const float4 &q, int k, auto diag_c) {
+            constexpr bool D = decltype(diag_c)::value;
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                ax[t] += (double)fx[t];
-                ay[t] += (double)fy[t];
-                az[t] += (double)fz[t];
-            }
-            double cx = (double)gx, cy = (double)gy, cz = (double)gz;
-            if (wave_far != ~0ull) {
-                // replay the packet's steps for the close pairs, in FP64
-                double hx = 0.0, hy = 0.0, hz = 0.0;
-                for (int k = 0; k < kWave; ++k) {
-                    const float4 q = pk[lane + k];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        if (skip(diag, t, j, k)) continue;
-                        const float dx = q.x - px[t], dy = q.y - py[t], dz = q.z - pz[t];
-                        const float rs =
-                            __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, e2)));
-                        if (!masked(diag, t, j, k) && rs < th[t]) {
-                            const double4 A = J[1 + ag * kSymGroup + t * kWave + lane];
-                            const double4 B = J[1 + hg * kSymGroup + j * kWave + ((lane + k) & (kWave - 1))];
-                            const double ex = B.x - A.x, ey = B.y - A.y, ez = B.z - A.z;
-                            const double s2 = ex * ex + ey * ey + ez * ez;
-                            const double r2d = SOFT ? s2 + eps2d : s2;
-                            const double y0 = __builtin_amdgcn_rsq(r2d);
-                            const double tt = y0 * y0;
-                            const double e = __builtin_fma(-r2d, tt, 1.0);
-                            const double y3 = tt * y0;
-                            const double wv = __builtin_fma(y3, e * __builtin_fma(c1875, e, c15), y3);
-                            const double fa = B.w * wv, fb = A.w * wv;
-                            ax[t] = __builtin_fma(fa, ex, ax[t]);
-                            ay[t] = __builtin_fma(fa, ey, ay[t]);
-                            az[t] = __builtin_fma(fa, ez, az[t]);
-                            hx = __builtin_fma(-fb, ex, hx);
-                            hy = __builtin_fma(-fb, ey, hy);
-                            hz = __builtin_fma(-fb, ez, hz);
-                        }
-                    }
-                    hx = rot_lane(hx); hy = rot_lane(hy); hz = rot_lane(hz);
+                if (D && skip(true, t, k)) continue;
+                const bool off = D && masked(true, t, k);
+                const float dx = q.x - px[t], dy = q.y - py[t], dz = q.z - pz[t];
+                const float rs = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, e2)));
+                const float y0 = __builtin_amdgcn_rsqf(rs);
+                const bool far = !(rs < th[t]);
+                wave_far &= __ballot(far);
+                if (far && !off) {
+                    const float wv = y0 * (y0 * y0);
+                    const float fa = q.w * wv, fb = pm[t] * wv;
+                    fx[t] = __builtin_fmaf(fa, dx, fx[t]);
+                    fy[t] = __builtin_fmaf(fa, dy, fy[t]);
+                    fz[t] = __builtin_fmaf(fa, dz, fz[t]);
+                    gx = __builtin_fmaf(-fb, dx, gx);
+                    gy = __builtin_fmaf(-fb, dy, gy);
+                    gz = __builtin_fmaf(-fb, dz, gz);
                 }
-                cx += hx; cy += hy; cz += hz;
             }
-            bs[j][0] += cx;
-            bs[j][1] += cy;
-            bs[j][2] += cz;
-        }
-        double *r = apart + it * (3 * kSymGroup);
+            gx = rot_lane_f(gx); gy = rot_lane_f(gy); gz = rot_lane_f(gz);
+        };
+        // two steps per iteration, each packet body read one step ahead
+        // (entry lane + k + 2 <= 127 stays in the slice)
+        auto fp32_pass = [&](auto diag_c) {
+            float4 qa = pk[lane];
+            for (int k = 0; k < kWave; k += 2) {
+                const float4 qb = pk[lane + k + 1];
+                step(qa, k, diag_c);
+                qa = pk[lane + k + 2];
+                step(qb, k + 1, diag_c);
+            }
+        };
+        if (diag) fp32_pass(std::true_type{}); else fp32_pass(std::false_type{});
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            r[t * kWave + lane] = ax[t];
-            r[kSymGroup + t * kWave + lane] = ay[t];
-            r[2 * kSymGroup + t * kWave + lane] = az[t];
+            ax[t] += (double)fx[t];
+            ay[t] += (double)fy[t];
+            az[t] += (double)fz[t];
+        }
+        double cx = (double)gx, cy = (double)gy, cz = (double)gz;
+        if (wave_far != ~0ull) {
+            // replay the packet's steps for the close pairs, in FP64
+            double hx = 0.0, hy = 0.0, hz = 0.0;
+            for (int k = 0; k < kWave; ++k) {
+                const float4 q = pk[lane + k];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    if (skip(diag, t, k)) continue;
+                    const float dx = q.x - px[t], dy = q.y - py[t], dz = q.z - pz[t];
+                    const float rs = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, e2)));
+                    if (!masked(diag, t, k) && rs < th[t]) {
+                        const double4 A = J[1 + hg * kSymGroup + t * kWave + lane];
+                        const double4 B = J[1 + ag * kSymGroup + j * kWave + ((lane + k) & (kWave - 1))];
+                        const double ex = B.x - A.x, ey = B.y - A.y, ez = B.z - A.z;
+                        const double s2 = ex * ex + ey * ey + ez * ez;
+                        const double r2d = SOFT ? s2 + eps2d : s2;
+                        const double y0 = __builtin_amdgcn_rsq(r2d);
+                        const double tt = y0 * y0;
+                        const double e = __builtin_fma(-r2d, tt, 1.0);
+                        const double y3 = tt * y0;
+                        const double wv = __builtin_fma(y3, e * __builtin_fma(c1875, e, c15), y3);
+                        const double fa = B.w * wv, fb = A.w * wv;
+                        ax[t] = __builtin_fma(fa, ex, ax[t]);
+                        ay[t] = __builtin_fma(fa, ey, ay[t]);
+                        az[t] = __builtin_fma(fa, ez, az[t]);
+                        hx = __builtin_fma(-fb, ex, hx);
+                        hy = __builtin_fma(-fb, ey, hy);
+                        hz = __builtin_fma(-fb, ez, hz);
+                    }
+                }
+                hx = rot_lane(hx); hy = rot_lane(hy); hz = rot_lane(hz);
+            }
+            cx += hx; cy += hy; cz += hz;
+        }
+        double *r = apart + it * (3 * kSymGroup) + j * kWave + lane;
+        r[0] = cx;
+        r[kSymGroup] = cy;
+        r[2 * kSymGroup] = cz;
+        ++it;
+        const bool last = it >= hi;
+        if (last || diag) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                sums[j][0][t * kWave + lane] = ax[t];
+                sums[j][1][t * kWave + lane] = ay[t];
+                sums[j][2][t * kWave + lane] = az[t];
+            }
+            sym_flush(sums, record);
+            if (last) break;
+            record += 3 * kSymGroup;
+            ++hg;
+            ag = 0;
+            load_col();
+        } else {
+            ++ag;
         }
     }
-    if (hcur >= 0) flush_col();
 }
 
 }  // namespace
@@ -642,7 +664,7 @@ void launch_pairs_sym_mixed(hipStream_t st, const SymPlan &sp, const float4 *J32
                             double *bpart, double eps2)
 {
     if (sp.M <= 2) return;
-    const int blocks = (sp.nwaves + (kBlock / kWave) - 1) / (kBlock / kWave);
+    const int blocks = sp.nwaves;
     const float nf2 = kNearFrac * kNearFrac;
     if (eps2 != 0.0)
         hipLaunchKernelGGL(k_pairs_sym_mixed<true>, dim3(blocks), dim3(kBlock), 0, st, sp, J32, J, apart, bpart,
@@ -656,7 +678,7 @@ void launch_pairs_sym(hipStream_t st, const SymPlan &sp, const double4 *J, doubl
                       double eps2)
 {
     if (sp.M <= 2) return;
-    const int blocks = (sp.nwaves + (kBlock / kWave) - 1) / (kBlock / kWave);
+    const int blocks = sp.nwaves;
     if (eps2 != 0.0)
         hipLaunchKernelGGL(k_pairs_sym_fp64<true>, dim3(blocks), dim3(kBlock), 0, st, sp, J, apart, bpart, eps2,
                            1.5, 1.875);

@@ -6,15 +6,16 @@
 // accelerations are formed from it.  The block is cut into groups of 256
 // bodies; a work item is an unordered pair of groups (row a <= column h),
 // numbered column by column: item = h (h + 1) / 2 + a.  The items are split
-// into nwaves contiguous ranges of equal length (to within one).
+// into nwaves contiguous ranges of equal length (to within one), one
+// workgroup of kSymWaves waves each ("wave" below is such a workgroup).
 //
 // Partial sums:
 //   row side    (the bodies of group a) -- one record per item, in
 //               apart[item][3][256];
-//   column side (the bodies of group h) -- summed by a wave over the
-//               consecutive items of one column, one record per (wave,
-//               column touched) in bpart[wave * slots_per_wave + (h - h_first)]
-//               [3][256], h_first the column of the wave's first item.
+//   column side (the bodies of group h) -- summed over the consecutive items
+//               of one column, one record per (wave, column touched) in
+//               bpart[wave * slots_per_wave + (h - h_first)][3][256], h_first
+//               the column of the wave's first item.
 // A body in group g thus finds its partials in items (g, h), h >= g, and in
 // the records of the waves that cover column g.
 //
@@ -33,6 +34,7 @@
 namespace sol {
 
 constexpr int kSymGroup = 256;     // bodies per group: four tiles of 64, one body of each per lane
+constexpr int kSymWaves = 4;       // waves of a workgroup, one packet of 64 row bodies each
 
 struct SymPlan {
     int32_t M;                     // mutual block [1, M); 0 when the symmetric sum is off
