@@ -122,6 +122,16 @@ PairPlan make_plan(const sol_context *c, const SegSpec *segs, int ns, double *pa
 // Bodies of the mutual block below which the one-directional sum is kept.
 constexpr int kSymMinBodies = 2048;
 
+// A call's arrays go through pinned memory that the kernels read and write in
+// place, up to this many bodies of six doubles: it saves a copy command, its
+// wait and a kernel on each side.  Measured for set_state, get_array and a
+// force evaluation of giants and test particles, us, with copies and without:
+// 515 bodies 35, 36, 66 and 22, 16, 38; 16,385 50, 61, 117 and 40, 49, 99;
+// 40,001 93, 140, 234 and 95, 140, 245 (the host's own copy then costs what
+// the copy command does).  The side outputs, half the size and four copies:
+// 515 bodies 73 and 19, 16,385 58 and 35, 65,537 117 and 96.
+constexpr int kIoBodies = 32768;
+
 // Builds the pair-sum work plans for the context's sink classes: the full
 // one-directional plan (every evaluation that tracks nearest neighbours,
 // the mixed form, barycentric frames) and, when the self-interacting block
@@ -376,15 +386,20 @@ void pair_sums(sol_context *c, bool nn, EpiArgs &a)
 
 // One full force evaluation of the state `st` (6 x NP) at time t, the
 // reference's Acceleration::Compute, with the derivative in `out`.
-// kind: EPI_COMPUTE or EPI_STAGE0 (the Driver's evaluation at y0; also
+// rows: the state in the interface's rows instead, which go to st = cin.
+// kind: EPI_COMPUTE, EPI_ROWS or EPI_STAGE0 (the Driver's evaluation at y0; also
 // writes yscale for RKF78 with the trial h).
 int evaluate_at(sol_context *c, const double *st, double t, double h, double *out, int kind, int integ,
-                bool last, bool want_yscale)
+                bool last, bool want_yscale, const double *rows = nullptr)
 {
     int ea, eb;
     source_ends(c, ea, eb);
-    launch_prep(c->stream, c->n, c->np, st, c->gm, c->J, mixed_on(c) ? c->J32 : nullptr, ind_buf(c, 0),
-                c->barycentric, ea, eb);
+    if (rows)
+        launch_prep_rows(c->stream, c->n, c->np, rows, c->cin, c->gm, c->J, mixed_on(c) ? c->J32 : nullptr,
+                         ind_buf(c, 0), c->barycentric, ea, eb);
+    else
+        launch_prep(c->stream, c->n, c->np, st, c->gm, c->J, mixed_on(c) ? c->J32 : nullptr, ind_buf(c, 0),
+                    c->barycentric, ea, eb);
     const bool gas_live = c->has_gas && !c->gas_dead;
     if (gas_live && (c->eval_mig1 || c->eval_mig2)) {
         const int do1 = c->eval_mig1 && c->nb.proto_planet > 0;
@@ -1095,7 +1110,7 @@ int sol_create(sol_context **out, const sol_nbodies *nb, int32_t barycentric, in
         (r = dalloc(c, &c->migt, np)) || (r = dalloc(c, &c->y0, 6 * np)) || (r = dalloc(c, &c->y, 6 * np)) ||
         (r = dalloc(c, &c->acc0, 6 * np)) || (r = dalloc(c, &c->yscale, 6 * np)) ||
         (r = dalloc(c, &c->error, 6 * np)) || (r = dalloc(c, &c->fst, 12 * 6 * np)) ||
-        (r = dalloc(c, &c->cin, 6 * np)) || (r = dalloc(c, &c->cout, 6 * np)) || (r = dalloc(c, &c->aos, 6 * np)) ||
+        (r = dalloc(c, &c->cin, 6 * np)) || (r = dalloc(c, &c->aos, 6 * np)) ||
         (r = dalloc(c, &c->J, np)) || (r = dalloc(c, &c->ind, 2 * (size_t)c->nblk * 6)) ||
         (r = dalloc(c, &c->rm3, np)) || (r = dalloc(c, &c->nnd, np)) || (r = dalloc(c, &c->nni, np)) ||
         (r = dalloc(c, &c->migc, 3 * np)) || (r = dalloc(c, &c->dragc, 3 * np)) ||
@@ -1106,6 +1121,13 @@ int sol_create(sol_context **out, const sol_nbodies *nb, int32_t barycentric, in
         hipHostMalloc((void **)&c->res_h, sizeof(ResSystem), hipHostMallocDefault) != hipSuccess) {
         c->err = "hipHostMalloc failed";
         return bail(SOL_ERR_DEVICE);
+    }
+    if (c->n <= 2 * kIoBodies) {
+        c->io_bytes = 6 * sizeof(double) * (size_t)std::min(c->n, kIoBodies);
+        if (hipHostMalloc((void **)&c->io_h, c->io_bytes, hipHostMallocDefault) != hipSuccess) {
+            c->err = "hipHostMalloc failed";
+            return bail(SOL_ERR_DEVICE);
+        }
     }
     std::vector<double> coef;
     fill_coefficients(coef);
@@ -1146,6 +1168,7 @@ int sol_destroy(sol_context *c)
     if (c->h_scal) (void)hipHostFree(c->h_scal);
     if (c->res_h) (void)hipHostFree(c->res_h);
     if (c->integ_h) (void)hipHostFree(c->integ_h);
+    if (c->io_h) (void)hipHostFree(c->io_h);
     if (c->mesh_h) (void)hipHostFree(c->mesh_h);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -1252,19 +1275,45 @@ int sol_set_source_ranges(sol_context *c, int32_t a, int32_t b)
     return ensure_partials(c);
 }
 
+// A call's rows of six doubles per body in: where the kernels read them.
+static size_t row_bytes(const sol_context *c) { return 6 * (size_t)c->n * sizeof(double); }
+static bool rows_pinned(const sol_context *c) { return row_bytes(c) <= c->io_bytes; }
+static int rows_in(sol_context *c, const double *host, const double **rows)
+{
+    if (rows_pinned(c)) {
+        std::memcpy(c->io_h, host, row_bytes(c));
+        *rows = c->io_h;
+        return SOL_OK;
+    }
+    HIPCHECK(c, hipMemcpyAsync(c->aos, host, row_bytes(c), hipMemcpyHostToDevice, c->stream));
+    *rows = c->aos;
+    return SOL_OK;
+}
+
+// ... and out: where the last kernel writes them, and the end of the call.
+// The rows read and the rows written share a buffer: the kernel that reads is
+// done before the one that writes starts.
+static double *rows_out(sol_context *c) { return rows_pinned(c) ? c->io_h : c->aos; }
+static int rows_done(sol_context *c, double *host)
+{
+    HIPCHECK(c, hipGetLastError());
+    if (!rows_pinned(c))
+        HIPCHECK(c, hipMemcpyAsync(host, c->aos, row_bytes(c), hipMemcpyDeviceToHost, c->stream));
+    HIPCHECK(c, hipStreamSynchronize(c->stream));
+    if (rows_pinned(c)) std::memcpy(host, c->io_h, row_bytes(c));
+    return SOL_OK;
+}
+
 int sol_compute(sol_context *c, double t, const double *yh, double *dydt)
 {
     if (check_ctx(c) || !yh || !dydt) return SOL_ERR_ARGUMENT;
     HIPCHECK(c, hipSetDevice(c->device));
-    const size_t bytes = 6 * (size_t)c->n * sizeof(double);
-    HIPCHECK(c, hipMemcpyAsync(c->aos, yh, bytes, hipMemcpyHostToDevice, c->stream));
-    launch_aos_to_soa(c->stream, c->n, c->np, c->aos, c->cin);
-    int r = evaluate_at(c, c->cin, t, 0.0, c->cout, EPI_COMPUTE, INTEG_RKF78, c->side_outputs, false);
+    const double *rows;
+    int r = rows_in(c, yh, &rows);
     if (r) return r;
-    launch_soa_to_aos(c->stream, c->n, c->np, c->cout, c->aos);
-    HIPCHECK(c, hipMemcpyAsync(dydt, c->aos, bytes, hipMemcpyDeviceToHost, c->stream));
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    return SOL_OK;
+    r = evaluate_at(c, c->cin, t, 0.0, rows_out(c), EPI_ROWS, INTEG_RKF78, c->side_outputs, false, rows);
+    if (r) return r;
+    return rows_done(c, dydt);
 }
 
 int sol_get_side_outputs(sol_context *c, double *rm3, int32_t *nn, double *dist, int32_t *mig)
@@ -1272,6 +1321,17 @@ int sol_get_side_outputs(sol_context *c, double *rm3, int32_t *nn, double *dist,
     if (check_ctx(c)) return SOL_ERR_ARGUMENT;
     HIPCHECK(c, hipSetDevice(c->device));
     const size_t n = c->n;
+    if (24 * n <= c->io_bytes) {
+        launch_pack_side(c->stream, c->n, c->rm3, c->nnd, c->nni, c->migt, c->io_h);
+        HIPCHECK(c, hipGetLastError());
+        HIPCHECK(c, hipStreamSynchronize(c->stream));
+        const int32_t *k = reinterpret_cast<const int32_t *>(c->io_h + 2 * n);
+        if (rm3) std::memcpy(rm3, c->io_h, n * sizeof(double));
+        if (dist) std::memcpy(dist, c->io_h + n, n * sizeof(double));
+        if (nn) std::memcpy(nn, k, n * sizeof(int32_t));
+        if (mig) std::memcpy(mig, k + n, n * sizeof(int32_t));
+        return SOL_OK;
+    }
     if (rm3) HIPCHECK(c, hipMemcpyAsync(rm3, c->rm3, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     if (nn) HIPCHECK(c, hipMemcpyAsync(nn, c->nni, n * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
     if (dist) HIPCHECK(c, hipMemcpyAsync(dist, c->nnd, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -1292,8 +1352,9 @@ int sol_set_mig_type(sol_context *c, const int32_t *mig)
 static int upload_soa(sol_context *c, const double *host, double *dst)
 {
     HIPCHECK(c, hipSetDevice(c->device));
-    HIPCHECK(c, hipMemcpyAsync(c->aos, host, 6 * (size_t)c->n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    launch_aos_to_soa(c->stream, c->n, c->np, c->aos, dst);
+    const double *rows;
+    if (int r = rows_in(c, host, &rows)) return r;
+    launch_aos_to_soa(c->stream, c->n, c->np, rows, dst);
     HIPCHECK(c, hipStreamSynchronize(c->stream));
     return SOL_OK;
 }
@@ -1323,10 +1384,8 @@ int sol_get_array(sol_context *c, int32_t which, double *out)
     default: return c->fail(SOL_ERR_ARGUMENT, "unknown array %d", which);
     }
     HIPCHECK(c, hipSetDevice(c->device));
-    launch_soa_to_aos(c->stream, c->n, c->np, src, c->aos);
-    HIPCHECK(c, hipMemcpyAsync(out, c->aos, 6 * (size_t)c->n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHECK(c, hipStreamSynchronize(c->stream));
-    return SOL_OK;
+    launch_soa_to_aos(c->stream, c->n, c->np, src, rows_out(c));
+    return rows_done(c, out);
 }
 
 int sol_driver(sol_context *c, int32_t integrator, double eps, sol_timeline *tl, double *body_h)

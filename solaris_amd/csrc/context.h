@@ -40,7 +40,7 @@ struct sol_context {
     double *gs = nullptr, *ge = nullptr, *stop = nullptr;
     int32_t *type = nullptr, *migt = nullptr;
     double *y0 = nullptr, *y = nullptr, *acc0 = nullptr, *yscale = nullptr, *error = nullptr;
-    double *fst = nullptr, *cin = nullptr, *cout = nullptr, *aos = nullptr;
+    double *fst = nullptr, *cin = nullptr, *aos = nullptr;
     double4 *J = nullptr;
     float4 *J32 = nullptr;     // allocated when the mixed form is selected
     sol::NNGrid grid{};       // nearest-neighbour search of the symmetric path
@@ -53,6 +53,10 @@ struct sol_context {
     double *errblk = nullptr, *scal = nullptr, *coef = nullptr, *integ = nullptr;
     double *h_scal = nullptr;   // pinned: [0] h, [1] t, [2] error max
     double *integ_h = nullptr;  // pinned, 12 * np: the integrals' rows and the masses (made on first use)
+    // pinned: the arrays of a call, which the kernels read and write in place
+    // (those that do not fit are copied to and from aos)
+    double *io_h = nullptr;
+    size_t io_bytes = 0;
     size_t part_slots = 0;
     std::vector<void *> allocs;
     // workgroup-resident drivers (resident.hip) for small systems

@@ -60,7 +60,8 @@ struct GasDev {
     double eta_c, eta_i, tau_c, tau_i, sh_c, sh_i, rho_c, rho_i, mfp_c, mfp_i;
 };
 
-enum EpiKind { EPI_COMPUTE = 0, EPI_STAGE0 = 1, EPI_MID = 2, EPI_FINAL = 3 };
+// EPI_ROWS: as EPI_COMPUTE, the derivative in the interface's rows of six
+enum EpiKind { EPI_COMPUTE = 0, EPI_STAGE0 = 1, EPI_MID = 2, EPI_FINAL = 3, EPI_ROWS = 4 };
 enum IntegKind { INTEG_RKF78 = 0, INTEG_RK4 = 1, INTEG_DP = 2 };
 
 // Arguments of the per-stage epilogue (see stages.hip).
@@ -194,6 +195,13 @@ void launch_pairs_sym_mixed(hipStream_t st, const SymPlan &sp, const float4 *J32
 void launch_prep(hipStream_t st, int n, int np, const double *state, const double *gm,
                  double4 *J, float4 *J32, double *ind_out, int barycentric, int src_end_a,
                  int src_end_b);
+// launch_prep from rows of six doubles (device or pinned host memory), which
+// also go to `state` as components.
+void launch_prep_rows(hipStream_t st, int n, int np, const double *aos, double *state, const double *gm,
+                      double4 *J, float4 *J32, double *ind_out, int barycentric, int src_end_a, int src_end_b);
+// rm3 and nnd (n doubles each), then nni and migt (n int32 each) into out.
+void launch_pack_side(hipStream_t st, int n, const double *rm3, const double *nnd, const int32_t *nni,
+                      const int32_t *migt, double *out);
 void launch_migration(hipStream_t st, int n_central, int n_giant, int n_massive, int np,
                       const double *state, const double *mass, const double *stop,
                       int32_t *migt, double *migc, const GasDev &gas, int barycentric,

@@ -136,6 +136,62 @@ __global__ __launch_bounds__(256) void k_prep(int n, int np, const double *__res
         for (int k = 0; k < 6; ++k) ind_out[blockIdx.x * 6 + k] = v[k];
 }
 
+// Rows of six doubles (the interface's layout) through LDS, so that both
+// sides move whole lines: aos may be pinned host memory, which the kernels
+// read and write across the bus without a copy command of its own.
+__device__ __forceinline__ void load_rows(const double *__restrict__ aos, int n, double *lds, double v[6])
+{
+    const int64_t first = (int64_t)blockIdx.x * kBlock * 6;
+    const int len = min(6 * kBlock, (int)max((int64_t)0, 6 * (int64_t)n - first));
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        const int q = k * kBlock + threadIdx.x;
+        lds[q] = q < len ? aos[first + q] : 0.0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 6; ++c) v[c] = lds[6 * threadIdx.x + c];
+}
+
+__device__ __forceinline__ void store_rows(double *__restrict__ aos, int n, double *lds, const double v[6])
+{
+    const int64_t first = (int64_t)blockIdx.x * kBlock * 6;
+    const int len = min(6 * kBlock, (int)max((int64_t)0, 6 * (int64_t)n - first));
+#pragma unroll
+    for (int c = 0; c < 6; ++c) lds[6 * threadIdx.x + c] = v[c];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        const int q = k * kBlock + threadIdx.x;
+        if (q < len) aos[first + q] = lds[q];
+    }
+}
+
+// k_prep from the interface's rows, which are also laid out as components
+// (what k_aos_to_soa would do first).
+__global__ __launch_bounds__(256) void k_prep_rows(int n, int np, const double *__restrict__ aos,
+                                                    double *__restrict__ st, const double *__restrict__ gm,
+                                                    double4 *__restrict__ J, float4 *__restrict__ J32,
+                                                    double *__restrict__ ind_out, int bc, int ea, int eb)
+{
+    __shared__ double rows[6 * kBlock];
+    __shared__ double lds[kBlock / kWave][6];
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    double s[6];
+    const double m = i < n ? gm[i] : 0.0;
+    load_rows(aos, n, rows, s);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) st[c * np + i] = s[c];
+    J[i] = make_double4(s[0], s[1], s[2], m);
+    if (J32) J32[i] = make_float4((float)s[0], (float)s[1], (float)s[2], (float)m);
+    if (bc) return;
+    double v[6];
+    indirect_contrib(i, n, s[0], s[1], s[2], m, ea, eb, v);
+    block_sum6(v, lds);
+    if (threadIdx.x == 0)
+        for (int k = 0; k < 6; ++k) ind_out[blockIdx.x * 6 + k] = v[k];
+}
+
 // ---- pair-partial lookup ------------------------------------------------
 __device__ __forceinline__ int64_t wave_lo(const PairPlan &p, int64_t w)
 {
@@ -339,6 +395,7 @@ __global__ __launch_bounds__(256) void k_epilogue(EpiArgs a)
     __shared__ double ind_sum[6];
     __shared__ double lds[kBlock / kWave][6];
     __shared__ double red[kBlock / kWave];
+    __shared__ double rows[6 * kBlock];
     const int i = blockIdx.x * kBlock + threadIdx.x;
     const int np = a.np;
     const double h = a.scal ? a.scal[0] : a.h, t = a.scal ? a.scal[1] : a.t;
@@ -405,7 +462,7 @@ __global__ __launch_bounds__(256) void k_epilogue(EpiArgs a)
         }
         if (a.kind == EPI_COMPUTE || a.kind == EPI_STAGE0) {
             for (int c = 0; c < 6; ++c) a.fout[c * np + i] = f[c];
-        } else {
+        } else if (a.kind != EPI_ROWS) {
             for (int c = 3; c < 6; ++c) a.fout[c * np + i] = f[c];
         }
         if (a.last) {
@@ -425,7 +482,9 @@ __global__ __launch_bounds__(256) void k_epilogue(EpiArgs a)
         }
     }
 
-    if (a.kind == EPI_STAGE0) {
+    if (a.kind == EPI_ROWS) {
+        store_rows(a.fout, a.n, rows, f);
+    } else if (a.kind == EPI_STAGE0) {
         // yscale = |y0| + |h f0| + TINY (RungeKuttaFehlberg78.cpp:87-89)
         if (valid && a.yscale_out)
             for (int c = 0; c < 6; ++c)
@@ -531,18 +590,40 @@ __global__ void k_errmax_final(const double *__restrict__ blk, int nblk, double 
     if (threadIdx.x == 0) *out = m;
 }
 
-__global__ void k_aos_to_soa(int n, int np, const double *__restrict__ aos, double *__restrict__ soa)
+__global__ __launch_bounds__(256) void k_aos_to_soa(int n, int np, const double *__restrict__ aos,
+                                                     double *__restrict__ soa)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= np) return;
-    for (int c = 0; c < 6; ++c) soa[c * np + i] = (i < n) ? aos[6 * (int64_t)i + c] : 0.0;
+    __shared__ double rows[6 * kBlock];
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    double v[6];
+    load_rows(aos, n, rows, v);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) soa[c * np + i] = v[c];
 }
 
-__global__ void k_soa_to_aos(int n, int np, const double *__restrict__ soa, double *__restrict__ aos)
+__global__ __launch_bounds__(256) void k_soa_to_aos(int n, int np, const double *__restrict__ soa,
+                                                     double *__restrict__ aos)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double rows[6 * kBlock];
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    double v[6];
+#pragma unroll
+    for (int c = 0; c < 6; ++c) v[c] = soa[c * np + i];
+    store_rows(aos, n, rows, v);
+}
+
+// The side outputs one after another: rm3, nnd, then nni and migType.
+__global__ __launch_bounds__(256) void k_pack_side(int n, const double *__restrict__ rm3,
+                                                    const double *__restrict__ nnd, const int32_t *__restrict__ nni,
+                                                    const int32_t *__restrict__ migt, double *__restrict__ out)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
-    for (int c = 0; c < 6; ++c) aos[6 * (int64_t)i + c] = soa[c * np + i];
+    out[i] = rm3[i];
+    out[(int64_t)n + i] = nnd[i];
+    int32_t *k = reinterpret_cast<int32_t *>(out + 2 * (int64_t)n);
+    k[i] = nni[i];
+    k[(int64_t)n + i] = migt[i];
 }
 
 // Tools::CheckAgainstSmallestNumber on two state arrays (Solaris/Tools.cpp:39-46).
@@ -690,6 +771,19 @@ void launch_prep(hipStream_t st, int n, int np, const double *state, const doubl
 {
     hipLaunchKernelGGL(k_prep, dim3(np / kBlock), dim3(kBlock), 0, st, n, np, state, gm, J, J32, ind_out, bc,
                        ea, eb);
+}
+
+void launch_prep_rows(hipStream_t st, int n, int np, const double *aos, double *state, const double *gm, double4 *J,
+                      float4 *J32, double *ind_out, int bc, int ea, int eb)
+{
+    hipLaunchKernelGGL(k_prep_rows, dim3(np / kBlock), dim3(kBlock), 0, st, n, np, aos, state, gm, J, J32, ind_out,
+                       bc, ea, eb);
+}
+
+void launch_pack_side(hipStream_t st, int n, const double *rm3, const double *nnd, const int32_t *nni,
+                      const int32_t *migt, double *out)
+{
+    hipLaunchKernelGGL(k_pack_side, dim3(nblocks(n)), dim3(kBlock), 0, st, n, rm3, nnd, nni, migt, out);
 }
 
 void launch_migration(hipStream_t st, int n_central, int n_giant, int n_massive, int np, const double *state,
