@@ -29,7 +29,7 @@ HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 HIP_FLAGS = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-Wall", "-Wno-unused-function", "-Wno-unused-variable"]
-HIP_SOURCES = ["pairs.hip", "stages.hip", "resident.hip", "mesh.hip", "adjoint.hip", "adjoint_few.hip", "nngrid.hip", "noalloc.hip", "context.cpp",
+HIP_SOURCES = ["pairs.hip", "stages.hip", "resident.hip", "mesh.hip", "quad.hip", "adjoint.hip", "adjoint_few.hip", "nngrid.hip", "noalloc.hip", "context.cpp",
                "ensemble.cpp", "adjoint.cpp"]
 
 

@@ -649,7 +649,7 @@ SliceArrays system_arrays(sol_context *c)
 // From 32 sources on: an RKF78 attempt of 33 bodies takes 48 us on the mesh
 // and 58 in one workgroup, of 17 bodies 47 and 35.
 constexpr int kMeshMinSources = 32;
-constexpr int kPathMesh = 100;     // reported as SOL_PATH_GRID
+constexpr int kPathMesh = 100, kPathQuad = 101;     // reported as SOL_PATH_GRID
 
 bool use_mesh(sol_context *c, int ik, int *share_out = nullptr, int *groups_out = nullptr)
 {
@@ -670,12 +670,30 @@ bool use_mesh(sol_context *c, int ik, int *share_out = nullptr, int *groups_out 
     return true;
 }
 
-// The path a Driver call or a caller loop of integrator ik takes: the grid
-// form where it applies (few sources, more bodies than grid_min_bodies),
-// the mesh form for many sources, else one workgroup where the system fits,
+// The quad form (quad.hip) takes the systems of the grid form, and smaller
+// ones, that have at most eight sources besides the star, no live gas, and
+// bodies for at most a workgroup per CU (14,339 with two planets).  The Sun,
+// two planets and test particles, us per RKF78 attempt in one workgroup or in
+// slices, and in quads: 4 bodies 15 and 5.4, 128 15 and 5.2, 515 17.6 and 5.6,
+// 5,001 18.6 and 6.1, 14,338 20.4 and 6.9.
+bool use_quad(sol_context *c, int ik, int *groups_out = nullptr)
+{
+    if (c->resident_disabled || c->grid_disabled || c->barycentric || c->grid_block != 0) return false;
+    if (c->has_gas && !c->gas_dead) return false;
+    if (c->precision != SOL_PRECISION_FP64 || c->softening != 0.0 || c->n < c->quad_min_bodies) return false;
+    const int sources = grid_sources(c) - 1, groups = quad_groups(c->n, sources, c->cu_count);
+    if (groups == 0 || quad_capacity(ik, sources, c->cu_count) < groups) return false;
+    if (groups_out) *groups_out = groups;
+    return true;
+}
+
+// The path a Driver call or a caller loop of integrator ik takes: the quad
+// and the grid form where they apply (few sources, more bodies than
+// grid_min_bodies), the mesh form for many sources, else one workgroup where the system fits,
 // else one launch per stage.
 int path_of(sol_context *c, int ik, SliceMap *m)
 {
+    if (use_quad(c, ik)) return kPathQuad;
     if (use_grid(c, ik, m)) return SOL_PATH_GRID;
     if (use_mesh(c, ik)) return kPathMesh;
     return use_resident(c, ik) ? SOL_PATH_RESIDENT : SOL_PATH_MULTI_KERNEL;
@@ -716,8 +734,8 @@ int resident_finish(sol_context *c, const ResSystem &S, sol_timeline *tl, int64_
     return SOL_OK;
 }
 
-int mesh_run(sol_context *c, int ik, double eps, sol_timeline *tl, int64_t max_steps, bool clip, double *body_h,
-             int64_t *steps_out, int64_t *attempts_out, int32_t stop_mask, int32_t *reason);
+int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int64_t max_steps, bool clip,
+             double *body_h, int64_t *steps_out, int64_t *attempts_out, int32_t stop_mask, int32_t *reason);
 
 // Runs accepted steps of integrator ik in the resident kernel: exactly one
 // Driver call when clip is false and max_steps == 1, or the caller loop
@@ -730,8 +748,8 @@ int resident_run(sol_context *c, int ik, double eps, sol_timeline *tl, int64_t m
 {
     SliceMap m{};
     const int path = path_of(c, ik, &m);
-    if (path == kPathMesh)
-        return mesh_run(c, ik, eps, tl, max_steps, clip, body_h, steps_out, attempts_out, stop_mask, reason);
+    if (path == kPathMesh || path == kPathQuad)
+        return mesh_run(c, path, ik, eps, tl, max_steps, clip, body_h, steps_out, attempts_out, stop_mask, reason);
     const bool grid = path == SOL_PATH_GRID;
     ResSystem S0 = resident_system(c, eps, tl, clip, stop_mask);
     ResArrays A;
@@ -814,7 +832,7 @@ int resident_run(sol_context *c, int ik, double eps, sol_timeline *tl, int64_t m
     return resident_finish(c, S, tl, max_steps, clip, body_h, steps_out, attempts_out, stop_mask, reason);
 }
 
-// Arrays and exchange words of the mesh form.
+// Arrays and exchange words of the mesh and the quad form.
 int mesh_buffers(sol_context *c)
 {
     sol_context::Mesh &m = c->mesh;
@@ -826,10 +844,10 @@ int mesh_buffers(sol_context *c)
         (r = dalloc(c, &m.yscale, 6 * np)) || (r = dalloc(c, &m.error, 6 * np)) || (r = dalloc(c, &m.rm3, np)) ||
         (r = dalloc(c, &m.nnd, np)) || (r = dalloc(c, &m.nni, np)) || (r = dalloc(c, &m.part, 1)) ||
         (r = dalloc(c, &m.part_of, (size_t)kMeshMaxGroups)) ||
-        (r = dalloc(c, &sys, sizeof(ResSystem) + sizeof(MeshSync))))
+        (r = dalloc(c, &sys, sizeof(ResSystem) + std::max(sizeof(MeshSync), sizeof(QuadSync)))))
         return r;
     m.sys = reinterpret_cast<ResSystem *>(sys);
-    m.sync = reinterpret_cast<MeshSync *>(sys + sizeof(ResSystem));
+    m.sync = sys + sizeof(ResSystem);
     if (!c->mesh_h && hipHostMalloc((void **)&c->mesh_h, sizeof(ResSystem) + 8 + sizeof(MeshPart), hipHostMallocDefault) != hipSuccess) {
         c->mesh_h = nullptr;
         return c->fail(SOL_ERR_DEVICE, "hipHostMalloc failed");
@@ -837,14 +855,15 @@ int mesh_buffers(sol_context *c)
     return dalloc(c, &m.pos, 6 * np);
 }
 
-// resident_run on the mesh form: accepted steps of integrator ik with the
-// system's bodies shared out over workgroups, about 0.2 s of work per
+// resident_run on the mesh or the quad form: accepted steps of integrator ik
+// with the system's bodies shared out over workgroups, about 0.2 s of work per
 // launch.  The context's arrays are replaced by the run's at its end only.
-int mesh_run(sol_context *c, int ik, double eps, sol_timeline *tl, int64_t max_steps, bool clip, double *body_h,
-             int64_t *steps_out, int64_t *attempts_out, int32_t stop_mask, int32_t *reason)
+int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int64_t max_steps, bool clip,
+             double *body_h, int64_t *steps_out, int64_t *attempts_out, int32_t stop_mask, int32_t *reason)
 {
+    const bool quad = path == kPathQuad;
     int share = 0, groups = 0;
-    if (!use_mesh(c, ik, &share, &groups)) return kGridRetry;
+    if (quad ? !use_quad(c, ik, &groups) : !use_mesh(c, ik, &share, &groups)) return kGridRetry;
     int r = mesh_buffers(c);
     if (r) return r;
     sol_context::Mesh &m = c->mesh;
@@ -858,7 +877,7 @@ int mesh_run(sol_context *c, int ik, double eps, sol_timeline *tl, int64_t max_s
     MeshArgs A{};
     A.systems = m.sys;
     A.parts = m.part; A.part_of = m.part_of;
-    A.sync = m.sync;
+    A.sync = reinterpret_cast<MeshSync *>(m.sync);
     A.pos = m.pos; A.gm = c->gm;
     A.tot = c->np;
     A.mass = c->mass; A.radius = c->radius;
@@ -866,13 +885,28 @@ int mesh_run(sol_context *c, int ik, double eps, sol_timeline *tl, int64_t max_s
     A.rm3 = m.rm3; A.nnd = m.nnd; A.nni = m.nni;
     A.eps2 = c->softening * c->softening;
     A.ticks = (uint64_t)(c->grid_wait_s * (double)c->rtc_hz);
-    const double per_step = 13.0 * (5.0e-6 + (double)c->n * (double)c->n * 1.0e-12);
+    QuadArgs Q{};
+    Q.system = m.sys;
+    Q.sync = reinterpret_cast<QuadSync *>(m.sync);
+    Q.sources = grid_sources(c) - 1;
+    Q.groups = groups;
+    Q.tot = A.tot;
+    Q.gm = A.gm; Q.mass = A.mass; Q.radius = A.radius;
+    Q.y0 = A.y0; Q.y = A.y; Q.acc0 = A.acc0; Q.yscale = A.yscale; Q.err = A.err;
+    Q.rm3 = A.rm3; Q.nnd = A.nnd; Q.nni = A.nni;
+    Q.ticks = A.ticks;
+    const double per_step = quad ? 2.0e-5 : 13.0 * (5.0e-6 + (double)c->n * (double)c->n * 1.0e-12);
     const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(20000, (int64_t)(0.2 / per_step)));
     A.y0_in = c->y0;
     for (;;) {
         const int64_t k = max_steps > 0 ? std::min(chunk, max_steps - S.steps) : chunk;
         const UnitLease lease(c->device, groups, c->cu_count);
-        HIPCHECK(c, launch_mesh(c->stream, ik, A, 1, groups, c->n, share, (int)k));
+        if (quad) {
+            Q.y0_in = A.y0_in;
+            HIPCHECK(c, launch_quad(c->stream, ik, Q, (int)k));
+        } else {
+            HIPCHECK(c, launch_mesh(c->stream, ik, A, 1, groups, c->n, share, (int)k));
+        }
         HIPCHECK(c, hipMemcpyAsync(c->mesh_h, m.sys, sizeof(ResSystem) + sizeof(uint32_t), hipMemcpyDeviceToHost,
                                    c->stream));
         HIPCHECK(c, hipStreamSynchronize(c->stream));
@@ -1091,7 +1125,7 @@ int sol_create(sol_context **out, const sol_nbodies *nb, int32_t barycentric, in
         const int b = std::atoi(e);
         if (b >= 64 && b <= 256 && b % 64 == 0) c->grid_block = b;
     }
-    if (const char *e = std::getenv("SOLARIS_AMD_GRID_MIN")) c->grid_min_bodies = std::max(2, std::atoi(e));
+    if (const char *e = std::getenv("SOLARIS_AMD_GRID_MIN")) c->grid_min_bodies = c->quad_min_bodies = std::max(2, std::atoi(e));
     if (const char *e = std::getenv("SOLARIS_AMD_GRID_WAIT")) c->grid_wait_s = std::max(0.0, std::atof(e));
     {
         int khz = 0;
@@ -1563,7 +1597,8 @@ int sol_integrate_until(sol_context *c, int32_t integrator, double eps, sol_time
         stats->device_ms = ms;
         int groups = 0;
         if (path == kPathMesh) (void)use_mesh(c, ik, nullptr, &groups);
-        stats->path = path == kPathMesh ? SOL_PATH_GRID : path;
+        if (path == kPathQuad) (void)use_quad(c, ik, &groups);
+        stats->path = path == kPathMesh || path == kPathQuad ? SOL_PATH_GRID : path;
         stats->slices = path == SOL_PATH_GRID ? gm.nslices : groups;
     }
     return r;

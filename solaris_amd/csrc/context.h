@@ -12,6 +12,7 @@
 #include "sol_internal.h"
 #include "resident.h"
 #include "mesh.h"
+#include "quad.h"
 
 namespace sol { struct AdjointState; }
 
@@ -68,7 +69,7 @@ struct sol_context {
     // buffers (gbuf: 111 doubles per slot, gibuf: 2 int32)
     bool grid_disabled = false;
     int grid_block = 0;           // slice threads; 0: chosen per system
-    int grid_min_bodies = 129;
+    int grid_min_bodies = 129, quad_min_bodies = 2;
     sol::ResSystem *grid_sys_d = nullptr;
     std::vector<sol::ResSystem> grid_sys_h;
     int grid_sys_cap = 0;
@@ -81,16 +82,16 @@ struct sol_context {
     int grid_failures = 0;           // grid runs that gave up; two turn the grid form off
     int grid_capacity[18] = {-1, -1, -1, -1, -1, -1, -1, -1, -1,
                              -1, -1, -1, -1, -1, -1, -1, -1, -1};   // per integrator, gas, slice size
-    // self-gravitating systems over several workgroups (mesh.hip): the arrays
-    // a run writes, which change places with the context's own at its end
+    // systems over several workgroups that exchange positions (mesh.hip) or,
+    // with few sources, step decisions only (quad.hip): the arrays a run writes, which change places with the context's own at its end
     // (a run that could not complete leaves those untouched)
     struct Mesh {
         double *y0 = nullptr, *y = nullptr, *acc0 = nullptr, *yscale = nullptr, *error = nullptr;
         double *rm3 = nullptr, *nnd = nullptr;
         int32_t *nni = nullptr;
         double *pos = nullptr;
-        sol::ResSystem *sys = nullptr;       // followed by the MeshSync
-        sol::MeshSync *sync = nullptr;
+        sol::ResSystem *sys = nullptr;       // followed by the MeshSync or QuadSync
+        unsigned char *sync = nullptr;       // (its first word: a wait gave up)
         sol::MeshPart *part = nullptr;
         int32_t *part_of = nullptr;
     } mesh;

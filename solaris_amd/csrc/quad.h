@@ -1,0 +1,47 @@
+// quad.h -- whole Driver loops of systems with few sources, four lanes per
+// body (quad.hip).
+#pragma once
+
+#include "resident.h"
+
+namespace sol {
+
+// Limits of the quad form: workgroups, and the bodies besides the star that
+// are a source of some other (every wave integrates all of them).
+constexpr int kQuadMaxGroups = 256;
+constexpr int kQuadMaxSources = 8;
+constexpr int kQuadThreads = 256;
+
+// Exchange words of one system's workgroups.  words[p][k][w] is half k of
+// workgroup w's error maximum of exchange x (p = x & 1), x | event << 31 in
+// its upper half, so that a reader needs no flag of its own.  System-scope
+// atomics only.
+struct QuadSync {
+    uint32_t error, pad[31];
+    unsigned long long words[2][2][kQuadMaxGroups];
+};
+
+struct QuadArgs {
+    ResSystem *system;
+    QuadSync *sync;
+    int32_t sources;           // bodies [1, 1 + sources) are integrated by every wave
+    int32_t groups;
+    // read: state, k^2 m and masses; written at the end (component stride tot):
+    // the state, the previous state, the Driver's arrays and the side outputs
+    int64_t tot;
+    const double *y0_in, *gm, *mass, *radius;
+    double *y0, *y, *acc0, *yscale, *err, *rm3, *nnd;
+    int32_t *nni;
+    uint64_t ticks;            // real-time-counter ticks a wait lasts before it gives up
+};
+
+// Workgroups for n bodies (0: the system does not fit).
+int quad_groups(int n, int sources, int cus);
+
+// Zeroes the exchange words and runs max_steps accepted steps of integrator
+// `integ`.  The a.groups workgroups have to be resident at once.
+hipError_t launch_quad(hipStream_t st, int integ, const QuadArgs &a, int max_steps);
+// Workgroups of that launch the device holds at once.
+int quad_capacity(int integ, int sources, int cu_count);
+
+}  // namespace sol
