@@ -122,6 +122,8 @@ PairPlan make_plan(const sol_context *c, const SegSpec *segs, int ns, double *pa
 // Bodies of the mutual block below which the one-directional sum is kept.
 constexpr int kSymMinBodies = 2048;
 
+constexpr int kBesideMinBodies = 8192;   // the neighbour search beside the pair sum (pair_sums)
+
 // A call's arrays go through pinned memory that the kernels read and write in
 // place, up to this many bodies of six doubles: it saves a copy command, its
 // wait and a kernel on each side.  Measured for set_state, get_array and a
@@ -344,11 +346,19 @@ double *ind_buf(sol_context *c, int parity) { return c->ind + (size_t)(parity & 
 // kernel, which in mixed precision also keeps the FP32 rounding of the
 // pair sums cancelling in the error estimate's F10 - F12 (RKF78) and
 // F7 - F8 (Dormand-Prince).  Sets the epilogue's plan fields.
-void pair_sums(sol_context *c, bool nn, EpiArgs &a)
+int pair_sums(sol_context *c, bool nn, EpiArgs &a)
 {
     const double eps2 = c->softening * c->softening;
     a.nn_sep = 0;
     if (c->sym.M > 0) {
+        // The nearest-neighbour search (six short launches) beside the pair
+        // sum, on the second stream, where that is long enough to pay for the
+        // events; one after the other and beside, us per force evaluation:
+        // 4,001 bodies 109 and 113..122, 6,001 132 and 131..137, 8,193 159 and
+        // 149..156, 16,385 281 and 253, 40,001 929 and 885.  (A profiled
+        // context times its launches one by one.)
+        const bool beside = nn && !c->profiling && c->n >= kBesideMinBodies;
+        if (beside) HIPCHECK(c, hipEventRecord(c->ev_fork, c->stream));
         {
             ProfScope ps(c, 3, c->sym_inter_per_launch);
             if (mixed_on(c))
@@ -356,24 +366,29 @@ void pair_sums(sol_context *c, bool nn, EpiArgs &a)
             else
                 launch_pairs_sym(c->stream, c->sym, c->J, c->apart, c->bpart, eps2);
         }
+        if (beside) HIPCHECK(c, hipStreamWaitEvent(c->stream2, c->ev_fork, 0));
+        if (nn) {
+            ProfScope ps(c, 2, 0.0);
+            launch_nn_grid(beside ? c->stream2 : c->stream, c->grid, c->plan, c->J, c->n, c->barycentric != 0);
+            a.nnr2 = c->grid.r2;
+            a.nnidx = c->grid.idx;
+            a.nn_sep = 1;
+        }
         if (c->plan_rest.total_items > 0) {
             ProfScope ps(c, 0, c->rest_inter_per_launch);
             launch_pairs(c->stream, c->plan_rest, c->J, c->part, c->nnr2, c->nnidx, false, false, mixed_on(c), eps2,
                          c->J32);
         }
-        if (nn) {
-            ProfScope ps(c, 2, 0.0);
-            launch_nn_grid(c->stream, c->grid, c->plan, c->J, c->n, c->barycentric != 0);
-            a.nnr2 = c->grid.r2;
-            a.nnidx = c->grid.idx;
-            a.nn_sep = 1;
+        if (beside) {
+            HIPCHECK(c, hipEventRecord(c->ev_join, c->stream2));
+            HIPCHECK(c, hipStreamWaitEvent(c->stream, c->ev_join, 0));
         }
         a.plan = c->plan_rest;
         a.sym = c->sym;
         a.use_sym = 1;
         a.apart = c->apart;
         a.bpart = c->bpart;
-        return;
+        return SOL_OK;
     }
     {
         ProfScope ps(c, nn ? 2 : 0, c->pair_inter_per_launch);
@@ -382,6 +397,7 @@ void pair_sums(sol_context *c, bool nn, EpiArgs &a)
     }
     a.plan = c->plan;
     a.use_sym = 0;
+    return SOL_OK;
 }
 
 // One full force evaluation of the state `st` (6 x NP) at time t, the
@@ -411,7 +427,7 @@ int evaluate_at(sol_context *c, const double *st, double t, double h, double *ou
     EpiArgs a = base_args(c);
     a.h = h;
     a.t = t;
-    pair_sums(c, last, a);
+    if (int r = pair_sums(c, last, a)) return r;
     a.kind = kind;
     a.integ = integ;
     a.stage = 0;
@@ -465,7 +481,7 @@ int run_stages(sol_context *c, int ik, double t, double h, bool read_err, double
     for (int s = 1; s <= S; ++s) {
         const bool last = (s == S);
         EpiArgs e = a;
-        pair_sums(c, last, e);
+        if (int r = pair_sums(c, last, e)) return r;
         e.stage = s;
         e.kind = last ? EPI_FINAL : EPI_MID;
         e.last = last ? 1 : 0;
@@ -1133,7 +1149,10 @@ int sol_create(sol_context **out, const sol_nbodies *nb, int32_t barycentric, in
             c->rtc_hz = (uint64_t)khz * 1000;
     }
     if (const char *e = std::getenv("SOLARIS_AMD_NO_SYM")) c->sym_disabled = e[0] == '1';
-    if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
+    if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
+        hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess) {
         c->err = "hipStreamCreate failed";
         return bail(SOL_ERR_DEVICE);
     }
@@ -1186,6 +1205,7 @@ int sol_destroy(sol_context *c)
     if (!c) return SOL_OK;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
+    if (c->stream2) (void)hipStreamSynchronize(c->stream2);
     adjoint_release(c);
     for (void *p : c->allocs) (void)hipFree(p);
     if (c->part) (void)hipFree(c->part);
@@ -1205,6 +1225,9 @@ int sol_destroy(sol_context *c)
     if (c->io_h) (void)hipHostFree(c->io_h);
     if (c->mesh_h) (void)hipHostFree(c->mesh_h);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
+    if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
+    if (c->ev_join) (void)hipEventDestroy(c->ev_join);
+    if (c->stream2) (void)hipStreamDestroy(c->stream2);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return SOL_OK;

@@ -19,6 +19,8 @@ namespace sol { struct AdjointState; }
 struct sol_context {
     int device = 0;
     hipStream_t stream = nullptr;
+    hipStream_t stream2 = nullptr;                       // the nearest-neighbour search beside the pair sum
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     sol_nbodies nb{};
     int n = 0, np = 0, nblk = 0, n_massive = 0;
     int barycentric = 0;

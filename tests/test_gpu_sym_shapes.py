@@ -1,7 +1,8 @@
 """The symmetric pair sum where its groups and workgroups change: blocks that
 end one body into, one body short of and at the end of a group of 256 (and of
 a packet of 64), the smallest block, and workgroups of one item and of
-several, whose column sums pass from item to item.
+several, whose column sums pass from item to item; and the nearest-neighbour
+search after the pair sum (up to 8,191 bodies) and beside it.
 
 FP64 against the one-directional sum (SOLARIS_AMD_NO_SYM=1): both round to a
 few 1e-16 of the sum of the terms' magnitudes, within 1e-14 of the total
@@ -52,3 +53,24 @@ def test_mixed_against_fp64(n):
     b = accelerations(scn)
     c = accelerations(scn, runtime.MIXED, SOLARIS_AMD_SYM_WAVES="3")
     assert rel(a, b) <= 1e-7 and rel(c, b) <= 1e-7
+
+
+@pytest.mark.parametrize("n", [8191, 8192])
+def test_neighbours_after_and_beside_the_pair_sum(n):
+    """Force evaluations one after another, each with its own neighbours; the
+    one-directional kernel finds the same ones."""
+    scn = S.make_c3(n=n - 1, softening=0.0)
+    os.environ["SOLARIS_AMD_NO_SYM"] = "1"
+    try:
+        plain = runtime.Context(scn)
+    finally:
+        os.environ.pop("SOLARIS_AMD_NO_SYM")
+    ctx = runtime.Context(scn)
+    for k in range(3):
+        y = scn.y0.copy()
+        y[1:, :3] = np.roll(y[1:, :3], k, axis=0)
+        a, b = ctx.compute(0.0, y), plain.compute(0.0, y)
+        sa, sb = ctx.side_outputs(), plain.side_outputs()
+        assert rel(a[1:, 3:], b[1:, 3:]) <= 1e-14
+        assert np.array_equal(sa[1], sb[1])
+        np.testing.assert_allclose(sa[2], sb[2], rtol=1e-12, atol=0)
