@@ -859,6 +859,7 @@ int mesh_buffers(sol_context *c)
     if ((r = dalloc(c, &m.y0, 6 * np)) || (r = dalloc(c, &m.y, 6 * np)) || (r = dalloc(c, &m.acc0, 6 * np)) ||
         (r = dalloc(c, &m.yscale, 6 * np)) || (r = dalloc(c, &m.error, 6 * np)) || (r = dalloc(c, &m.rm3, np)) ||
         (r = dalloc(c, &m.nnd, np)) || (r = dalloc(c, &m.nni, np)) || (r = dalloc(c, &m.part, 1)) ||
+        (r = dalloc(c, &m.sys_in, 1)) ||
         (r = dalloc(c, &m.part_of, (size_t)kMeshMaxGroups)) ||
         (r = dalloc(c, &sys, sizeof(ResSystem) + std::max(sizeof(MeshSync), sizeof(QuadSync)))))
         return r;
@@ -902,6 +903,7 @@ int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int
     A.eps2 = c->softening * c->softening;
     A.ticks = (uint64_t)(c->grid_wait_s * (double)c->rtc_hz);
     QuadArgs Q{};
+    Q.system_in = m.sys_in;
     Q.system = m.sys;
     Q.sync = reinterpret_cast<QuadSync *>(m.sync);
     Q.sources = grid_sources(c) - 1;
@@ -919,6 +921,7 @@ int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int
         const UnitLease lease(c->device, groups, c->cu_count);
         if (quad) {
             Q.y0_in = A.y0_in;
+            HIPCHECK(c, hipMemcpyAsync(m.sys_in, &S, sizeof S, hipMemcpyHostToDevice, c->stream));
             HIPCHECK(c, launch_quad(c->stream, ik, Q, (int)k));
         } else {
             HIPCHECK(c, launch_mesh(c->stream, ik, A, 1, groups, c->n, share, (int)k));
@@ -938,6 +941,12 @@ int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int
         if (S.status != RES_RUNNING) break;
         if (max_steps > 0 && S.steps >= max_steps) break;
         A.y0_in = m.y0;
+        if (quad) {
+            // (its launches do not read what they write; pos is the mesh form's)
+            HIPCHECK(c, hipMemcpyAsync(m.pos, m.y0, 6 * (size_t)c->np * sizeof(double), hipMemcpyDeviceToDevice,
+                                       c->stream));
+            A.y0_in = m.pos;
+        }
     }
     std::swap(c->y0, m.y0);
     std::swap(c->y, m.y);

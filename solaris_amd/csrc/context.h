@@ -93,6 +93,7 @@ struct sol_context {
         int32_t *nni = nullptr;
         double *pos = nullptr;
         sol::ResSystem *sys = nullptr;       // followed by the MeshSync or QuadSync
+        sol::ResSystem *sys_in = nullptr;    // the quad form's copy to read
         unsigned char *sync = nullptr;       // (its first word: a wait gave up)
         sol::MeshPart *part = nullptr;
         int32_t *part_of = nullptr;

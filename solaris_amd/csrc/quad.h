@@ -22,12 +22,15 @@ struct QuadSync {
 };
 
 struct QuadArgs {
+    // read and written at the end, not in place: without an exchange (RK4) a
+    // workgroup may be done before another has started
+    const ResSystem *system_in;
     ResSystem *system;
     QuadSync *sync;
     int32_t sources;           // bodies [1, 1 + sources) are integrated by every wave
     int32_t groups;
-    // read: state, k^2 m and masses; written at the end (component stride tot):
-    // the state, the previous state, the Driver's arrays and the side outputs
+    // read: state, k^2 m and masses; written at the end (component stride tot),
+    // none of them read by the launch: the state, the previous state, the Driver's arrays and the side outputs
     int64_t tot;
     const double *y0_in, *gm, *mass, *radius;
     double *y0, *y, *acc0, *yscale, *err, *rm3, *nnd;

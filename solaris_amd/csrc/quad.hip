@@ -220,7 +220,7 @@ __global__ __launch_bounds__(kQuadThreads) void k_quad(QuadArgs A, int max_steps
     const int quad = lane >> 2, l = lane & 3, comp = l < 3 ? l : 2;
     const int ns = A.sources, mine = kQuads - ns;
     const int gw = (int)blockIdx.x * kQuadWaves + wave;
-    ResSystem S = *A.system;
+    ResSystem S = *A.system_in;
     if (S.status != RES_RUNNING) return;      // the same in every workgroup
 
     const int n = S.n;

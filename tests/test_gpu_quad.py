@@ -141,3 +141,23 @@ def test_wait_that_gives_up_falls_back():
     assert a.driver(RKF78, 1e-10, ta)[0] == 0 and b.driver(RKF78, 1e-10, tb)[0] == 0
     assert ta.time == tb.time
     assert np.array_equal(a.get_array(runtime.Y0), b.get_array(runtime.Y0))
+
+
+def test_many_launches():
+    """More RK4 steps than one launch takes, against the same in calls of its
+    own, and every workgroup's bodies in a run of one step (without an
+    exchange a workgroup may end before another starts)."""
+    scn = system(400, 2)
+    a, b = make_ctx(scn), make_ctx(scn)
+    ta, tb = timelines(0.0, 0.05)
+    assert a.integrate(RK4, 0.0, ta, max_steps=21000)[0] == 0
+    for k in (9000, 12000):
+        assert b.integrate(RK4, 0.0, tb, max_steps=k)[0] == 0
+    assert ta.time == tb.time
+    assert np.array_equal(a.get_array(runtime.Y0), b.get_array(runtime.Y0))
+    scn = system(14339, 2)
+    a, b = make_ctx(scn), other(scn)
+    ta, tb = timelines(0.0, 0.05)
+    for _ in range(20):
+        assert a.driver(RK4, 0.0, ta)[0] == 0 and b.driver(RK4, 0.0, tb)[0] == 0
+    assert np.abs(a.get_array(runtime.Y0) - b.get_array(runtime.Y0)).max() <= 20 * 1e-13
