@@ -93,7 +93,7 @@ int amalloc(sol_context *c, AdjointState *A, double **p, size_t count)
 {
     void *q = nullptr;
     HIPCHECK(c, hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(double)));
-    HIPCHECK(c, hipMemset(q, 0, std::max<size_t>(count, 1) * sizeof(double)));
+    HIPCHECK(c, hipMemsetAsync(q, 0, std::max<size_t>(count, 1) * sizeof(double), c->stream));
     A->allocs.push_back(q);
     *p = static_cast<double *>(q);
     return SOL_OK;

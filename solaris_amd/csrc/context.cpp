@@ -1191,6 +1191,11 @@ int sol_create(sol_context **out, const sol_nbodies *nb, int32_t barycentric, in
             return bail(SOL_ERR_DEVICE);
         }
     }
+    // the copies below are made on the default stream
+    if (hipStreamSynchronize(c->stream) != hipSuccess) {
+        c->err = "filling the context's arrays failed";
+        return bail(SOL_ERR_DEVICE);
+    }
     std::vector<double> coef;
     fill_coefficients(coef);
     if (hipMemcpy(c->coef, coef.data(), coef.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {

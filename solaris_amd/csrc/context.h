@@ -151,7 +151,9 @@ int dalloc(sol_context *c, T **p, size_t count)
 {
     void *q = nullptr;
     HIPCHECK(c, hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T)));
-    HIPCHECK(c, hipMemset(q, 0, std::max<size_t>(count, 1) * sizeof(T)));
+    // on the context's stream: a fill on the default stream is not waited for,
+    // and would not be ordered before the kernels of a non-blocking one
+    HIPCHECK(c, hipMemsetAsync(q, 0, std::max<size_t>(count, 1) * sizeof(T), c->stream));
     c->allocs.push_back(q);
     *p = static_cast<T *>(q);
     return SOL_OK;

@@ -138,7 +138,8 @@ int ealloc(sol_ensemble *e, T **p, size_t n)
 {
     void *q = nullptr;
     ECHECK(e, hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(T)));
-    ECHECK(e, hipMemset(q, 0, std::max<size_t>(n, 1) * sizeof(T)));
+    // (on the ensemble's stream, which is not ordered after the default one)
+    ECHECK(e, hipMemsetAsync(q, 0, std::max<size_t>(n, 1) * sizeof(T), e->stream));
     *p = static_cast<T *>(q);
     return SOL_OK;
 }
