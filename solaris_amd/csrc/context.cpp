@@ -547,12 +547,11 @@ int grid_capacity_of(sol_context *c, int ik, int block)
 // that needs at most 160 slices (every attempt's grid-wide decision costs
 // more with more slices; a step's latency is that of one body per thread
 // whatever the slice), else 256 (grid_block > 0 fixes it).
-bool use_grid(sol_context *c, int ik, SliceMap *m)
+bool grid_slices(sol_context *c, int ik, SliceMap *m)
 {
     if (c->resident_disabled || c->grid_disabled) return false;
     if (c->has_gas && !c->gas_dead && c->barycentric) return false;
     if (c->precision != SOL_PRECISION_FP64 || c->softening != 0.0) return false;
-    if (c->n < c->grid_min_bodies) return false;
     const int src = grid_sources(c);
     int block = c->grid_block;
     if (block == 0) {
@@ -567,6 +566,8 @@ bool use_grid(sol_context *c, int ik, SliceMap *m)
     if (m) *m = sm;
     return true;
 }
+
+bool use_grid(sol_context *c, int ik, SliceMap *m) { return c->n >= c->grid_min_bodies && grid_slices(c, ik, m); }
 
 // The resident arrays of the context's own (system-layout) buffers.
 ResArrays resident_arrays(sol_context *c)
@@ -687,19 +688,35 @@ bool use_mesh(sol_context *c, int ik, int *share_out = nullptr, int *groups_out 
 }
 
 // The quad form (quad.hip) takes the systems of the grid form, and smaller
-// ones, that have at most eight sources besides the star, no live gas, and
-// bodies for at most a workgroup per CU (14,339 with two planets).  The Sun,
-// two planets and test particles, us per RKF78 attempt in one workgroup or in
-// slices, and in quads: 4 bodies 15 and 5.4, 128 15 and 5.2, 515 17.6 and 5.6,
-// 5,001 18.6 and 6.1, 14,338 20.4 and 6.9.
-bool use_quad(sol_context *c, int ik, int *groups_out = nullptr)
+// ones, that have at most eight sources besides the star and bodies for at
+// most a workgroup per CU (14,339 with two planets).  The Sun, two planets and
+// test particles, us per RKF78 attempt in one workgroup or in slices, and in
+// quads: 4 bodies 15 and 5.4, 128 15 and 5.2, 515 17.6 and 5.6, 5,001 18.6 and
+// 6.1, 14,338 20.4 and 6.9.  With live gas: the grid form's slices of 64 and
+// 128 places, us per RKF78 attempt: 125 bodies 64 (one workgroup) and 31, 505
+// 51 and 31, 16,389 56 and 38.
+struct QuadShape { int sources, own, groups, places; };   // places: bodies of a workgroup with gas (0: no gas)
+
+bool use_quad(sol_context *c, int ik, QuadShape *out = nullptr)
 {
     if (c->resident_disabled || c->grid_disabled || c->barycentric || c->grid_block != 0) return false;
-    if (c->has_gas && !c->gas_dead) return false;
     if (c->precision != SOL_PRECISION_FP64 || c->softening != 0.0 || c->n < c->quad_min_bodies) return false;
-    const int sources = grid_sources(c) - 1, groups = quad_groups(c->n, sources, c->cu_count);
-    if (groups == 0 || quad_capacity(ik, sources, c->cu_count) < groups) return false;
-    if (groups_out) *groups_out = groups;
+    QuadShape q{};
+    q.sources = grid_sources(c) - 1;
+    if (q.sources < 1 || q.sources > kQuadMaxSources) return false;
+    if (c->has_gas && !c->gas_dead) {
+        SliceMap m{};
+        if (!grid_slices(c, ik, &m) || m.stride > kQuadGasBodies || m.nslices < 1 ||
+            m.nslices > std::min(c->cu_count, kQuadMaxGroups))
+            return false;
+        q.own = m.per; q.groups = m.nslices; q.places = m.stride;
+        if (quad_gas_capacity(ik, q.sources, q.places, c->cu_count) < q.groups) return false;
+    } else {
+        q.own = 16 - q.sources;
+        q.groups = quad_groups(c->n, q.sources, c->cu_count);
+        if (q.groups == 0 || quad_capacity(ik, q.sources, c->cu_count) < q.groups) return false;
+    }
+    if (out) *out = q;
     return true;
 }
 
@@ -872,6 +889,18 @@ int mesh_buffers(sol_context *c)
     return dalloc(c, &m.pos, 6 * np);
 }
 
+int mesh_gas_buffers(sol_context *c)
+{
+    sol_context::Mesh &m = c->mesh;
+    if (m.dragc) return SOL_OK;
+    const size_t np = c->np;
+    int r;
+    if ((r = dalloc(c, &m.migt, np)) || (r = dalloc(c, &m.migc, 3 * np)) || (r = dalloc(c, &m.migt_prev, np)) ||
+        (r = dalloc(c, &m.migc_prev, 3 * np)))
+        return r;
+    return dalloc(c, &m.dragc, 3 * np);
+}
+
 // resident_run on the mesh or the quad form: accepted steps of integrator ik
 // with the system's bodies shared out over workgroups, about 0.2 s of work per
 // launch.  The context's arrays are replaced by the run's at its end only.
@@ -880,7 +909,9 @@ int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int
 {
     const bool quad = path == kPathQuad;
     int share = 0, groups = 0;
-    if (quad ? !use_quad(c, ik, &groups) : !use_mesh(c, ik, &share, &groups)) return kGridRetry;
+    QuadShape shape{};
+    if (quad ? !use_quad(c, ik, &shape) : !use_mesh(c, ik, &share, &groups)) return kGridRetry;
+    if (quad) groups = shape.groups;
     int r = mesh_buffers(c);
     if (r) return r;
     sol_context::Mesh &m = c->mesh;
@@ -906,14 +937,25 @@ int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int
     Q.system_in = m.sys_in;
     Q.system = m.sys;
     Q.sync = reinterpret_cast<QuadSync *>(m.sync);
-    Q.sources = grid_sources(c) - 1;
+    Q.sources = shape.sources;
     Q.groups = groups;
+    Q.own = shape.own;
     Q.tot = A.tot;
     Q.gm = A.gm; Q.mass = A.mass; Q.radius = A.radius;
     Q.y0 = A.y0; Q.y = A.y; Q.acc0 = A.acc0; Q.yscale = A.yscale; Q.err = A.err;
     Q.rm3 = A.rm3; Q.nnd = A.nnd; Q.nni = A.nni;
     Q.ticks = A.ticks;
-    const double per_step = quad ? 2.0e-5 : 13.0 * (5.0e-6 + (double)c->n * (double)c->n * 1.0e-12);
+    if (shape.places) {
+        if ((r = mesh_gas_buffers(c))) return r;
+        Q.gas = c->gasdev;
+        Q.density = c->density; Q.cd = c->cd; Q.gs = c->gs; Q.ge = c->ge; Q.stop = c->stop;
+        Q.migt_in = c->migt; Q.migc_in = c->migc;
+        Q.migt = m.migt; Q.migc = m.migc; Q.dragc = m.dragc;
+        // the Driver turns both migration switches on for its first evaluation
+        Q.mig_do1 = c->nb.proto_planet > 0;
+        Q.mig_do2 = c->nb.giant_planet > 0;
+    }
+    const double per_step = quad ? 5.0e-5 : 13.0 * (5.0e-6 + (double)c->n * (double)c->n * 1.0e-12);
     const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(20000, (int64_t)(0.2 / per_step)));
     A.y0_in = c->y0;
     for (;;) {
@@ -922,7 +964,8 @@ int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int
         if (quad) {
             Q.y0_in = A.y0_in;
             HIPCHECK(c, hipMemcpyAsync(m.sys_in, &S, sizeof S, hipMemcpyHostToDevice, c->stream));
-            HIPCHECK(c, launch_quad(c->stream, ik, Q, (int)k));
+            HIPCHECK(c, shape.places ? launch_quad_gas(c->stream, ik, Q, shape.places, (int)k)
+                                     : launch_quad(c->stream, ik, Q, (int)k));
         } else {
             HIPCHECK(c, launch_mesh(c->stream, ik, A, 1, groups, c->n, share, (int)k));
         }
@@ -947,6 +990,20 @@ int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int
                                        c->stream));
             A.y0_in = m.pos;
         }
+        if (shape.places) {
+            // the next launch reads what this one left; a lost one still leaves the context's
+            HIPCHECK(c, hipMemcpyAsync(m.migt_prev, m.migt, c->np * sizeof(int32_t), hipMemcpyDeviceToDevice,
+                                       c->stream));
+            HIPCHECK(c, hipMemcpyAsync(m.migc_prev, m.migc, 3 * (size_t)c->np * sizeof(double),
+                                       hipMemcpyDeviceToDevice, c->stream));
+            Q.migt_in = m.migt_prev;
+            Q.migc_in = m.migc_prev;
+        }
+    }
+    if (shape.places) {
+        std::swap(c->migt, m.migt);
+        std::swap(c->migc, m.migc);
+        std::swap(c->dragc, m.dragc);
     }
     std::swap(c->y0, m.y0);
     std::swap(c->y, m.y);
@@ -1634,7 +1691,11 @@ int sol_integrate_until(sol_context *c, int32_t integrator, double eps, sol_time
         stats->device_ms = ms;
         int groups = 0;
         if (path == kPathMesh) (void)use_mesh(c, ik, nullptr, &groups);
-        if (path == kPathQuad) (void)use_quad(c, ik, &groups);
+        if (path == kPathQuad) {
+            QuadShape q{};
+            (void)use_quad(c, ik, &q);
+            groups = q.groups;
+        }
         stats->path = path == kPathMesh || path == kPathQuad ? SOL_PATH_GRID : path;
         stats->slices = path == SOL_PATH_GRID ? gm.nslices : groups;
     }

@@ -92,6 +92,9 @@ struct sol_context {
         double *rm3 = nullptr, *nnd = nullptr;
         int32_t *nni = nullptr;
         double *pos = nullptr;
+        // with gas: migration and drag (prev: as the run's last launch left them)
+        int32_t *migt = nullptr, *migt_prev = nullptr;
+        double *migc = nullptr, *migc_prev = nullptr, *dragc = nullptr;
         sol::ResSystem *sys = nullptr;       // followed by the MeshSync or QuadSync
         sol::ResSystem *sys_in = nullptr;    // the quad form's copy to read
         unsigned char *sync = nullptr;       // (its first word: a wait gave up)

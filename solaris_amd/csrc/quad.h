@@ -11,6 +11,7 @@ namespace sol {
 constexpr int kQuadMaxGroups = 256;
 constexpr int kQuadMaxSources = 8;
 constexpr int kQuadThreads = 256;
+constexpr int kQuadGasBodies = 128;     // places of a workgroup with gas, at most: four threads each
 
 // Exchange words of one system's workgroups.  words[p][k][w] is half k of
 // workgroup w's error maximum of exchange x (p = x & 1), x | event << 31 in
@@ -27,8 +28,9 @@ struct QuadArgs {
     const ResSystem *system_in;
     ResSystem *system;
     QuadSync *sync;
-    int32_t sources;           // bodies [1, 1 + sources) are integrated by every wave
+    int32_t sources;           // bodies [1, 1 + sources) are integrated by every wave (with gas: workgroup)
     int32_t groups;
+    int32_t own;               // bodies of its own a wave (with gas: a workgroup) has
     // read: state, k^2 m and masses; written at the end (component stride tot),
     // none of them read by the launch: the state, the previous state, the Driver's arrays and the side outputs
     int64_t tot;
@@ -36,6 +38,15 @@ struct QuadArgs {
     double *y0, *y, *acc0, *yscale, *err, *rm3, *nnd;
     int32_t *nni;
     uint64_t ticks;            // real-time-counter ticks a wait lasts before it gives up
+    // gas: the drag bodies' parameters, and migration (read, written at the
+    // end): types, and the caches of the Driver's first evaluation and of the
+    // last evaluation's drag
+    GasDev gas;
+    const double *density, *cd, *gs, *ge, *stop, *migc_in;
+    const int32_t *migt_in;
+    int32_t *migt;
+    double *migc, *dragc;
+    int32_t mig_do1, mig_do2;
 };
 
 // Workgroups for n bodies (0: the system does not fit).
@@ -44,7 +55,10 @@ int quad_groups(int n, int sources, int cus);
 // Zeroes the exchange words and runs max_steps accepted steps of integrator
 // `integ`.  The a.groups workgroups have to be resident at once.
 hipError_t launch_quad(hipStream_t st, int integ, const QuadArgs &a, int max_steps);
-// Workgroups of that launch the device holds at once.
+// The same with gas: workgroups of `places` bodies (the sources and a.own).
+hipError_t launch_quad_gas(hipStream_t st, int integ, const QuadArgs &a, int places, int max_steps);
+// Workgroups of these launches the device holds at once.
 int quad_capacity(int integ, int sources, int cu_count);
+int quad_gas_capacity(int integ, int sources, int places, int cu_count);
 
 }  // namespace sol

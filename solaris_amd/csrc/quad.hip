@@ -28,11 +28,13 @@
 // and after, us: RKF78 of 4 bodies 15.2 and 5.4, 515 17.6 and 5.6, 5,001 18.6
 // and 6.1, 14,338 20.4 and 6.9; Dormand-Prince of 515 13.9 and 4.9; RK4 of 515
 // 4.4 and 1.2.  An evaluation of 85 to 100 instructions takes 0.28 us, the
-// exchange 1.9 us.
+// exchange 1.9 us.  With gas, RKF78 of 505 bodies 51.6 and 31.1, 4,005 52.0 and
+// 30.2, 16,389 55.8 and 38.3.
 #include <float.h>
 
 #include <algorithm>
 
+#include "gasdev.h"
 #include "lane_pairs.h"
 #include "quad.h"
 #include "static_for.h"
@@ -41,6 +43,7 @@
 namespace sol {
 namespace {
 
+#define QUAD_LDS __attribute__((address_space(3)))
 #define QUAD_SCOPE __HIP_MEMORY_SCOPE_SYSTEM
 
 constexpr int kQuadWaves = kQuadThreads / kWave;
@@ -88,15 +91,21 @@ struct QSide {
 };
 
 // Acceleration component of this lane for the position whose component it
-// holds.  tab: the wave's source records (x, y, z), [0] the origin.
-template <int NA, bool SIDE>
+// holds.  tab: the source records (x, y, z), [0] the origin; the wave's own,
+// or with BLOCK the workgroup's (two sets in turn, so that one barrier between
+// writing and reading suffices).
+template <int NA, bool SIDE, bool BLOCK = false>
 __device__ __forceinline__ double quad_force(const QPulls<NA> &P, double (*tab)[4], int src, int l, double pos,
                                              QSide &side)
 {
     if (src > 0) tab[src][l] = pos;
     const double x = dpp_mov<0x00>(pos), y = dpp_mov<0x55>(pos), z = dpp_mov<0xAA>(pos);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    if (BLOCK) {
+        __syncthreads();
+    } else {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
     const double c15 = 1.5, c1875 = 1.875;
     double f[3] = {0.0, 0.0, 0.0};
     if (SIDE) { side.best = DBL_MAX; side.idx = 0x7fffffff; }
@@ -139,22 +148,45 @@ __device__ __forceinline__ double quad_force(const QPulls<NA> &P, double (*tab)[
     return keep + dpp_mov<0xB1>(send);
 }
 
-// One component of a body: state, previous state, stage derivatives
-// (velocities V, accelerations F), scale and error.
+// Stage derivatives of one component: velocities V and accelerations F, in
+// registers, or (LDS) in columns of the workgroup's LDS, column = thread.
+template <bool LDS>
+struct QStages {
+    double V_[13], F_[13];
+    __device__ __forceinline__ double V(int l) const { return V_[l]; }
+    __device__ __forceinline__ double F(int l) const { return F_[l]; }
+    __device__ __forceinline__ void put(int l, double v, double f) { V_[l] = v; F_[l] = f; }
+};
+template <>
+struct QStages<true> {
+    QUAD_LDS double *col;      // this thread's column
+    int stride;                // threads
+    __device__ __forceinline__ double V(int l) const { return col[2 * l * stride]; }
+    __device__ __forceinline__ double F(int l) const { return col[(2 * l + 1) * stride]; }
+    __device__ __forceinline__ void put(int l, double v, double f)
+    {
+        col[2 * l * stride] = v;
+        col[(2 * l + 1) * stride] = f;
+    }
+};
+
+// One component of a body: state, previous state, stage derivatives, scale
+// and error.
+template <bool LDS>
 struct QBody {
     double p, v, po, vo;
-    double V[13], F[13];
+    QStages<LDS> d;
     double sp, sv, ep, ev;
 };
 
 // State of stage S in tableau order, as resident.hip's stage_state.
-template <int INTEG, int S>
-__device__ __forceinline__ void quad_stage(const QBody &B, double h, double &pos, double &vel)
+template <int INTEG, int S, bool LDS>
+__device__ __forceinline__ void quad_stage(const QBody<LDS> &B, double h, double &pos, double &vel)
 {
     if constexpr (INTEG == INTEG_DP) {
-        double var = tab::kDpA[S][0] * B.F[0];
+        double var = tab::kDpA[S][0] * B.d.F(0);
         static_for<1, S>([&](auto L) {
-            if constexpr (tab::kDpA[S][L] != 0.0) var += tab::kDpA[S][L] * B.F[L];
+            if constexpr (tab::kDpA[S][L] != 0.0) var += tab::kDpA[S][L] * B.d.F(L);
         });
         pos = B.p + tab::kDpC[S] * h * B.v + h * h * (var);
         vel = B.v + h * (var);
@@ -164,7 +196,7 @@ __device__ __forceinline__ void quad_stage(const QBody &B, double h, double &pos
         static_for<0, S>([&](auto L) {
             constexpr double d = INTEG == INTEG_RKF78 ? tab::kRkfD[S][L] : tab::kRk4A[S][L];
             if constexpr (d != 0.0) {
-                const double x = d * B.V[L], y = d * B.F[L];
+                const double x = d * B.d.V(L), y = d * B.d.F(L);
                 ap = first ? x : ap + x;
                 av = first ? y : av + y;
                 first = false;
@@ -177,60 +209,154 @@ __device__ __forceinline__ void quad_stage(const QBody &B, double h, double &pos
 
 // Final state and error estimate (kept in B); returns this lane's part of the
 // error maximum.
-template <int INTEG>
-__device__ __forceinline__ double quad_final(QBody &B, double h, double &pos, double &vel)
+template <int INTEG, bool LDS>
+__device__ __forceinline__ double quad_final(QBody<LDS> &B, double h, double &pos, double &vel)
 {
     if constexpr (INTEG == INTEG_RKF78) {
         constexpr double b0 = 41.0 / 840.0, b5 = 34.0 / 105.0, b6 = 9.0 / 35.0, b8 = 9.0 / 280.0, b10 = 41.0 / 840.0;
-        auto sum = [&](const double *F) {
-            return b0 * F[0] + b5 * F[5] + b6 * (F[6] + F[7]) + b8 * (F[8] + F[9]) + b10 * F[10];
+        auto sum = [&](auto F) {
+            return b0 * F(0) + b5 * F(5) + b6 * (F(6) + F(7)) + b8 * (F(8) + F(9)) + b10 * F(10);
         };
-        pos = B.p + h * sum(B.V);
-        vel = B.v + h * sum(B.F);
-        B.ep = h * fabs(B.V[0] + B.V[10] - B.V[11] - B.V[12]) * 41.0 / 840.0;
-        B.ev = h * fabs(B.F[0] + B.F[10] - B.F[11] - B.F[12]) * 41.0 / 840.0;
+        auto V = [&](int l) { return B.d.V(l); };
+        auto F = [&](int l) { return B.d.F(l); };
+        pos = B.p + h * sum(V);
+        vel = B.v + h * sum(F);
+        B.ep = h * fabs(V(0) + V(10) - V(11) - V(12)) * 41.0 / 840.0;
+        B.ev = h * fabs(F(0) + F(10) - F(11) - F(12)) * 41.0 / 840.0;
         return fmax(fabs(B.ep / B.sp), fabs(B.ev / B.sv));
     } else if constexpr (INTEG == INTEG_RK4) {
-        auto sum = [&](const double *F) {
-            return tab::kRk4B[0] * F[0] + tab::kRk4B[1] * F[1] + tab::kRk4B[2] * F[2] + tab::kRk4B[3] * F[3];
+        auto sum = [&](auto F) {
+            return tab::kRk4B[0] * F(0) + tab::kRk4B[1] * F(1) + tab::kRk4B[2] * F(2) + tab::kRk4B[3] * F(3);
         };
-        pos = B.p + h * sum(B.V);
-        vel = B.v + h * sum(B.F);
+        pos = B.p + h * sum([&](int l) { return B.d.V(l); });
+        vel = B.v + h * sum([&](int l) { return B.d.F(l); });
         return 0.0;
     } else {
         constexpr const double *b = tab::kDpB, *d = tab::kDpBdh;
-        const double *F = B.F;
+        auto F = [&](int l) { return B.d.F(l); };
         const double h2 = h * h;
-        pos = B.p + h * B.v + h2 * (b[0] * F[0] + b[4] * F[4] + b[5] * F[5] + b[6] * F[6] + b[7] * F[7] + b[8] * F[8]);
-        vel = B.v + h * (d[0] * F[0] + d[4] * F[4] + d[5] * F[5] + d[6] * F[6] + d[7] * F[7]);
-        B.ep = h2 * fabs(F[7] - F[8]) / 20.0;
+        pos = B.p + h * B.v + h2 * (b[0] * F(0) + b[4] * F(4) + b[5] * F(5) + b[6] * F(6) + b[7] * F(7) + b[8] * F(8));
+        vel = B.v + h * (d[0] * F(0) + d[4] * F(4) + d[5] * F(5) + d[6] * F(6) + d[7] * F(7));
+        B.ep = h2 * fabs(F(7) - F(8)) / 20.0;
         B.ev = 0.0;
         return B.ep;
     }
 }
 
-template <int INTEG, int NA>
-__global__ __launch_bounds__(kQuadThreads) void k_quad(QuadArgs A, int max_steps)
+// ---- gas -------------------------------------------------------------------
+
+// What the drag reads, in LDS: the nebula, derived constants (mu = k^2 m0; edge
+// = rho_c inner_edge^(rho_i - 4); thermal: the factor of sqrt(r) in the mean
+// thermal speed), the exponent each lane of a quad takes, and the parameters
+// of the bodies.
+struct QGas {
+    GasDev g;
+    double mu, edge, thermal, idx[4];
+    int32_t quarters[4], by_quarters;      // 4 idx, where all four are whole and at most 16
+    double R[kQuadGasBodies], rho_b[kQuadGasBodies], cd[kQuadGasBodies], gs[kQuadGasBodies], ge[kQuadGasBodies];
+};
+
+// x^(k / 4), |k| <= 16, from square roots and products (r1 = sqrt(x)): a third
+// of the operations of pow.
+__device__ __forceinline__ double quad_quarters(double x, double r1, int k)
 {
-    __shared__ __attribute__((aligned(16))) double records[kQuadWaves][4 * NA][4];
-    __shared__ double sh_max[2][kQuadWaves], sh_val;
-    __shared__ int sh_any[2][kQuadWaves], sh_ev, sh_ok;
+    const int a = k < 0 ? -k : k, n = a >> 2;
+    const double r2 = sqrt(r1), x2 = x * x;
+    double p = (a & 1 ? r2 : 1.0) * (a & 2 ? r1 : 1.0);
+    p *= (n & 1 ? x : 1.0) * (n & 2 ? x2 : 1.0);
+    p = n & 4 ? p * (x2 * x2) : p;
+    return k < 0 ? 1.0 / p : p;
+}
+
+// GasDragAC (gas_drag in gasdev.h, with the same branches), component of this
+// lane of the drag at (x, y, z, vx, vy, vz).  What bounds an evaluation with gas
+// is this function's operations: a pow costs some 250 and a body needs three to
+// five, one division or root 12 to 25.  So the lanes of a quad take one power
+// each, of the cylindrical radius for the scale height, the density and eta and
+// of the spherical one for the mean free path; exponents in quarters go without
+// pow; and the circular velocity is (-y, x) sqrt(mu / rc^3).  The relative error
+// of the drag against 80 bits over 0.5 to 3 AU, most of it cancellation in the
+// velocity against the gas, is 1.6e-14 rms (before: 1.8e-14).  A call rather
+// than inlined code, whose constants would be held through the loop.
+__device__ __attribute__((noinline)) double quad_drag(const QUAD_LDS QGas *c, double factor, double x, double y, double z,
+                                                      double vx, double vy, double vz)
+{
+    const int l = threadIdx.x & 3, place = threadIdx.x >> 2;
+    const double idx = c->idx[l], R = c->R[place];
+    const double q = SQR(x) + SQR(y);
+    const double base = sqrt(l == 2 ? q + SQR(z) : q);
+    const double rc = dpp_mov<0x00>(base), r = dpp_mov<0xAA>(base);
+    const double r1 = sqrt(base);
+    // as pl() in gasdev.h: the exponents 1 and 1/2 (and here all quarters) without pow
+    double p = idx == 1.0 ? base : r1;
+    if (c->by_quarters) p = quad_quarters(base, r1, c->quarters[l]);
+    else if (idx != 1.0 && idx != 0.5) p = pow(base, idx);
+    const double h = c->g.sh_c * dpp_mov<0x00>(p), rho_p = dpp_mov<0x55>(p);
+    const double lambda = c->g.mfp_c * dpp_mov<0xAA>(p), eta = c->g.eta_c * dpp_mov<0xFF>(p);
+    const double s = (q > 0.0 ? sqrt(c->mu / (q * rc)) : 0.0) * sqrt(1.0 - 2.0 * eta);
+    const double ux = vx + y * s, uy = vy - x * s, uz = vz;
+    const double w = exp(-SQR(z / h));
+    const double rho = factor * (c->g.inner_edge < rc ? c->g.rho_c * rho_p * w : c->edge * SQR(SQR(rc)) * w);
+    double C;
+    if (R <= 0.1 * lambda) {                                  // Epstein
+        C = c->ge[place] * (c->thermal * sqrt(r)) * rho;
+    } else if (R >= 10.0 * lambda) {                          // Stokes
+        C = c->gs[place] * sqrt(ux * ux + uy * uy + uz * uz) * rho;
+    } else {                                                    // transition
+        const double l1 = 0.1 * lambda, l2 = 10.0 * lambda;
+        const double ge = 1.0 / (c->rho_b[place] * l1);
+        const double gsk = 3.0 / 8.0 * c->cd[place] / (c->rho_b[place] * l2);
+        const double vth = c->thermal * sqrt(r);
+        const double K = gsk * sqrt(ux * ux + uy * uy + uz * uz) / (ge * vth);
+        // one logarithm and one power per lane again
+        const double lg = log10(l & 1 ? l2 / l1 : K);
+        const double kappa = dpp_mov<0x00>(lg) / dpp_mov<0x55>(lg);
+        const double pk = l & 1 ? pow(R, kappa) : pow(l1, -kappa);
+        C = ge * vth * dpp_mov<0x00>(pk) * dpp_mov<0x55>(pk) * rho;
+    }
+    return -C * (l == 0 ? ux : l == 1 ? uy : uz);
+}
+
+__device__ __attribute__((noinline)) void quad_migration(const GasDev &g, bool giant, double x, double y, double z,
+                                                         double vx, double vy, double vz, double m, double mc,
+                                                         double stop, int32_t &type, double t, double (&o)[3])
+{
+    migration_accel(giant, x, y, z, vx, vy, vz, m, mc, stop, type, g, 0, t, o[0], o[1], o[2]);
+}
+
+// The Driver loop.  Without gas a wave is on its own but for the exchange
+// (its sources, its 16 - sources bodies, its records); with gas the workgroup
+// is: the sources once, `own` bodies, a barrier per evaluation, and the stages
+// in a loop with their derivatives in LDS, as the drag is too long to unroll.
+template <int INTEG, int NA, bool GAS>
+__device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, double *columns, QGas *gas)
+{
+    constexpr int kWaves = GAS ? 4 * kQuadGasBodies / kWave : kQuadWaves;
+    __shared__ __attribute__((aligned(16))) double records[GAS ? 2 : kQuadWaves][4 * NA][4];
+    __shared__ double sh_max[2][kWaves], sh_val;
+    __shared__ int sh_any[2][kWaves], sh_ev, sh_ok;
     constexpr int nst = q_stages<INTEG>();
+    const int nwaves = GAS ? (int)blockDim.x / kWave : kQuadWaves;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = uniform(tid / kWave);
-    const int quad = lane >> 2, l = lane & 3, comp = l < 3 ? l : 2;
-    const int ns = A.sources, mine = kQuads - ns;
-    const int gw = (int)blockIdx.x * kQuadWaves + wave;
+    const int quad = (GAS ? tid : lane) >> 2, l = lane & 3, comp = l < 3 ? l : 2;
+    const int ns = A.sources;
+    const int unit = GAS ? (int)blockIdx.x : (int)blockIdx.x * kQuadWaves + wave;   // that has the sources once
     ResSystem S = *A.system_in;
     if (S.status != RES_RUNNING) return;      // the same in every workgroup
 
     const int n = S.n;
-    int i = quad < ns ? 1 + quad : 1 + ns + gw * mine + (quad - ns);
-    const bool valid = i < n;
+    int i = quad < ns ? 1 + quad : 1 + ns + unit * A.own + (quad - ns);
+    const bool valid = i < n && quad - ns < A.own;
     if (!valid) i = 1;         // the first source once more; nothing of it is kept
-    const bool keeps = valid && (quad >= ns || gw == 0);
+    const bool keeps = valid && (quad >= ns || unit == 0);
     const int src = quad < ns && l < 3 ? 1 + quad : 0;
-    double (*tab)[4] = records[wave];
-    tab[lane >> 2 < 4 * NA ? lane >> 2 : 0][l] = 0.0;     // 16 quads, at most 12 records
+    double (*tab)[4] = records[GAS ? 0 : wave];
+    if (GAS) {
+        if (tid < 2 * 4 * NA * 4) (&records[0][0][0])[tid] = 0.0;
+        __syncthreads();
+    } else {
+        tab[quad < 4 * NA ? quad : 0][l] = 0.0;     // 16 quads, at most 12 records
+    }
 
     QPulls<NA> P;
     {
@@ -245,41 +371,146 @@ __global__ __launch_bounds__(kQuadThreads) void k_quad(QuadArgs A, int max_steps
             P.near[t] = is;
         }
     }
-    QBody B;
+    QBody<GAS> B;
+    if constexpr (GAS) { B.d.col = (QUAD_LDS double *)columns + tid; B.d.stride = (int)blockDim.x; }
     B.p = B.po = A.y0_in[comp * A.tot + i];
     B.v = B.vo = A.y0_in[(3 + comp) * A.tot + i];
     B.sp = B.sv = B.ep = B.ev = 0.0;
-    static_for<0, 13>([&](auto L) { B.V[L] = B.F[L] = 0.0; });
+    static_for<0, 13>([&](auto L) { B.d.put(L, 0.0, 0.0); });
     QSide side{0.0, 0.0, 0}, none;
     const bool events = S.clip && (S.stop_mask & SOL_STOP_EVENT) && (S.e3 > 0.0 || S.h3 > 0.0 || S.coll > 0.0);
     const bool combine = INTEG != INTEG_RK4 || events;
     bool flushed = false;      // small numbers were flushed in this launch
     int x = 0;                 // exchanges
+
+    // Gas: the drag body's parameters, the migration of a massive one (types
+    // and accelerations are this thread's until the end).
+    bool drags = false;
+    double mig = 0.0, mig_next = 0.0, drag = 0.0, migc = 0.0;
+    int32_t mt = 0, mt_next = 0;
+    bool migrates = false, giant = false, fresh = false, fresh_next = false;
+    const double m0 = A.mass[0];
+    if constexpr (GAS) {
+        drags = i >= S.drag_lo && i < S.drag_hi;
+        const GasDev &g = A.gas;
+        if (tid == 0) {
+            // MeanThermalSpeed_CMU and Temperature_CMU, as gas_drag in gasdev.h
+            const double kb = 1.3806488e-23 * ((1.0 / 1.98911e30) * SQR(1.0 / 1.495978707e11)) / SQR(1.0 / 86400.0);
+            const double mp = 1.672621777e-27 * (1.0 / 1.98911e30);
+            const double cvth = sqrt((8.0 * kb) / (3.14159265358979323846 * g.mmw * mp));
+            const double ctp = kGauss2 * (1.0 / (kb / mp));
+            gas->g = g;
+            gas->mu = kGauss2 * m0;
+            gas->edge = g.rho_c * pow(g.inner_edge, g.rho_i - 4.0);
+            gas->thermal = cvth * sqrt(SQR(g.sh_c) * g.mmw * ctp * pow(m0, 2.0 * g.sh_i - 3.0));
+            gas->idx[0] = g.sh_i; gas->idx[1] = g.rho_i; gas->idx[2] = g.mfp_i; gas->idx[3] = g.eta_i;
+            gas->by_quarters = 1;
+            for (int k = 0; k < 4; ++k) {
+                const double v = 4.0 * gas->idx[k];
+                const bool whole = fabs(v) <= 16.0 && v == trunc(v);
+                gas->quarters[k] = whole ? (int)v : 0;
+                if (!whole) gas->by_quarters = 0;
+            }
+        }
+        if (l == 0) {
+            gas->R[quad] = A.radius[i]; gas->rho_b[quad] = A.density[i]; gas->cd[quad] = A.cd[i];
+            gas->gs[quad] = A.gs[i]; gas->ge[quad] = A.ge[i];
+        }
+        __syncthreads();
+        mt = A.migt_in[i];
+        migc = A.migc_in[comp * A.tot + i];
+        giant = i < S.giant_end;
+        migrates = i >= S.mig_lo && i < S.nm && (giant ? A.mig_do2 : A.mig_do1) != 0;
+    }
+    // Migration of the Driver's first evaluation at (pos, vel, t) for this
+    // thread's component; type: the body's, which it may end.
+    auto migration = [&](double t, double pos, double vel, int32_t &type, bool &is) -> double {
+        is = migrates && type == (giant ? SOL_MIGRATION_TYPE_II : SOL_MIGRATION_TYPE_I);
+        double o[3] = {0.0, 0.0, 0.0};
+        if (is)
+            quad_migration(gas->g, giant, dpp_mov<0x00>(pos), dpp_mov<0x55>(pos), dpp_mov<0xAA>(pos), dpp_mov<0x00>(vel),
+                           dpp_mov<0x55>(vel), dpp_mov<0xAA>(vel), A.mass[i], m0, A.stop[i], type, t, o);
+        return l == 0 ? o[0] : l == 1 ? o[1] : o[2];
+    };
+    // Acceleration at (pos, vel) with the gas's factor and the migration m.
+    auto accelerate = [&](double pos, double vel, double factor, double m, QSide &sd) -> double {
+        double f = quad_force<NA, true, true>(P, tab, src, l, pos, sd);
+        tab = tab == records[0] ? records[1] : records[0];
+        if (drags) {
+            drag = quad_drag((const QUAD_LDS QGas *)gas, factor, dpp_mov<0x00>(pos), dpp_mov<0x55>(pos), dpp_mov<0xAA>(pos),
+                             dpp_mov<0x00>(vel), dpp_mov<0x55>(vel), dpp_mov<0xAA>(vel));
+            f += drag;
+        }
+        return f + m;
+    };
+
     // f0 of the next step: the acceleration at (p, v)
-    double f0 = quad_force<NA, false>(P, tab, src, l, B.p, none);
+    double f0 = 0.0;
+    bool again = GAS;          // with gas f0 is formed at the step's start: the first one, and after a flush
+    if constexpr (!GAS) f0 = quad_force<NA, false>(P, tab, src, l, B.p, none);
 
     for (int step = 0; step < max_steps; ++step) {
         const double t0 = S.t;
         double h = S.h_next, errmax = 0.0;
         int iter = 0, outcome = 0;             // outcome: 0 accept, 2 underflow, 3 maxiter
         bool event = false;
-        B.V[0] = B.v;
-        B.F[0] = f0;
+        if constexpr (GAS) {
+            if (again) {
+                mt_next = mt;
+                mig_next = migration(t0, B.p, B.v, mt_next, fresh_next);
+                f0 = accelerate(B.p, B.v, reduction_factor(A.gas, t0), mig_next, none);
+                again = false;
+            }
+            mig = mig_next;
+            mt = mt_next;
+            fresh = fresh_next;
+            if (fresh) migc = mig;
+        }
+        B.d.put(0, B.v, f0);
         if (INTEG == INTEG_RKF78) {
-            B.sp = fabs(B.p) + fabs(h * B.V[0]) + 1.0e-30;
-            B.sv = fabs(B.v) + fabs(h * B.F[0]) + 1.0e-30;
+            B.sp = fabs(B.p) + fabs(h * B.v) + 1.0e-30;
+            B.sv = fabs(B.v) + fabs(h * f0) + 1.0e-30;
         }
         double pos, vel;
         for (;;) {
             ++iter;
-            static_for<1, nst + 1>([&](auto T) {
-                quad_stage<INTEG, T>(B, h, pos, vel);
-                B.V[T] = vel;
-                if constexpr (T < nst) B.F[T] = quad_force<NA, false>(P, tab, src, l, pos, none);
-                else B.F[T] = quad_force<NA, true>(P, tab, src, l, pos, side);
-            });
+            double last_drag = 0.0;
+            if constexpr (GAS) {
+                for (int q = 1; q <= nst; ++q) {
+                    static_for<1, nst + 1>([&](auto T) {
+                        if (q == T) quad_stage<INTEG, T>(B, h, pos, vel);
+                    });
+                    // RK4 and Dormand-Prince pass t + c h, RKF78 passes t to every stage
+                    double ts = t0;
+                    if (INTEG != INTEG_RKF78)
+                        static_for<1, nst + 1>([&](auto T) {
+                            if (q == T) ts = t0 + (INTEG == INTEG_RK4 ? tab::kRk4C[T < 4 ? T : 0] : tab::kDpC[T < 9 ? T : 0]) * h;
+                        });
+                    const double f = accelerate(pos, vel, reduction_factor(A.gas, ts), mig, side);
+                    B.d.put(q, vel, f);
+                }
+                last_drag = drag;
+            } else {
+                static_for<1, nst + 1>([&](auto T) {
+                    quad_stage<INTEG, T>(B, h, pos, vel);
+                    if constexpr (T < nst) B.d.put(T, vel, quad_force<NA, false>(P, tab, src, l, pos, none));
+                    else B.d.put(T, vel, quad_force<NA, true>(P, tab, src, l, pos, side));
+                });
+            }
             const double ratio = quad_final<INTEG>(B, h, pos, vel);
             double raw = 0.0;
+            // f0 of the next step, should this one be accepted
+            auto next_f0 = [&]() {
+                if constexpr (GAS) {
+                    const double tn = t0 + h;
+                    mt_next = mt;
+                    mig_next = migration(tn, pos, vel, mt_next, fresh_next);
+                    f0 = accelerate(pos, vel, reduction_factor(A.gas, tn), mig_next, none);
+                    drag = last_drag;
+                } else {
+                    f0 = quad_force<NA, false>(P, tab, src, l, pos, none);
+                }
+            };
             if (combine) {
                 ++x;
                 // the side outputs' events and the workgroup's error maximum
@@ -298,7 +529,7 @@ __global__ __launch_bounds__(kQuadThreads) void k_quad(QuadArgs A, int max_steps
                 __syncthreads();
                 double g = sh_max[par][0];
                 int any = sh_any[par][0];
-                for (int w = 1; w < kQuadWaves; ++w) { g = fmax(g, sh_max[par][w]); any |= sh_any[par][w]; }
+                for (int w = 1; w < nwaves; ++w) { g = fmax(g, sh_max[par][w]); any |= sh_any[par][w]; }
                 unsigned long long *mw = A.sync->words[x & 1][0], *lw = A.sync->words[x & 1][1];
                 if (tid == 0 && A.groups > 1) {
                     // a NaN has its sign bit cleared and is passed over below
@@ -307,8 +538,7 @@ __global__ __launch_bounds__(kQuadThreads) void k_quad(QuadArgs A, int max_steps
                     __hip_atomic_store(mw + blockIdx.x, tag | (e >> 32), __ATOMIC_RELAXED, QUAD_SCOPE);
                     __hip_atomic_store(lw + blockIdx.x, tag | (e & 0xffffffffull), __ATOMIC_RELAXED, QUAD_SCOPE);
                 }
-                // meanwhile f0 of the next step, should this one be accepted
-                f0 = quad_force<NA, false>(P, tab, src, l, pos, none);
+                next_f0();             // meanwhile
                 if (A.groups > 1 && wave == 0) {
                     constexpr int kPolls = kQuadMaxGroups / kWave;
                     const uint64_t c0 = __builtin_amdgcn_s_memrealtime();
@@ -362,7 +592,7 @@ __global__ __launch_bounds__(kQuadThreads) void k_quad(QuadArgs A, int max_steps
                 raw = uniform(fabs(g));
                 event = uniform(any) != 0;
             } else {
-                f0 = quad_force<NA, false>(P, tab, src, l, pos, none);
+                next_f0();
             }
             S.attempts += 1;
             B.po = pos;                       // the attempt's final state, as the Driver's second array
@@ -442,7 +672,8 @@ __global__ __launch_bounds__(kQuadThreads) void k_quad(QuadArgs A, int max_steps
             if (fabs(B.v) < 1.0e-50) B.v = 0.0;
             if (fabs(B.po) < 1.0e-50) B.po = 0.0;
             if (fabs(B.vo) < 1.0e-50) B.vo = 0.0;
-            f0 = quad_force<NA, false>(P, tab, src, l, B.p, none);
+            if constexpr (GAS) again = true;
+            else f0 = quad_force<NA, false>(P, tab, src, l, B.p, none);
         }
         if (S.status != RES_RUNNING) break;
     }
@@ -453,12 +684,17 @@ __global__ __launch_bounds__(kQuadThreads) void k_quad(QuadArgs A, int max_steps
         A.y0[v] = B.v;
         A.y[p] = B.po;
         A.y[v] = B.vo;
-        A.acc0[p] = B.V[0];
-        A.acc0[v] = B.F[0];
+        A.acc0[p] = B.d.V(0);
+        A.acc0[v] = B.d.F(0);
+        if constexpr (GAS) {
+            A.migc[p] = migc;
+            A.dragc[p] = drag;
+        }
         if (INTEG == INTEG_RKF78) { A.yscale[p] = B.sp; A.yscale[v] = B.sv; }
         if (INTEG != INTEG_RK4) { A.err[p] = B.ep; A.err[v] = B.ev; }
     }
     if (keeps && l == 0) {
+        if constexpr (GAS) A.migt[i] = mt;
         const bool has = side.best < DBL_MAX;
         A.rm3[i] = side.rm3;
         A.nnd[i] = has ? sqrt(side.best) : 0.0;
@@ -476,12 +712,27 @@ __global__ __launch_bounds__(kQuadThreads) void k_quad(QuadArgs A, int max_steps
             if (INTEG != INTEG_RK4) A.err[o] = 0.0;
         }
         if (tid == 0) {
+            if constexpr (GAS) A.migt[0] = A.migt_in[0];
             A.rm3[0] = 0.0;
             A.nnd[0] = 0.0;
             A.nni[0] = -1;
             *A.system = S;
         }
     }
+}
+
+template <int INTEG, int NA>
+__global__ __launch_bounds__(kQuadThreads) void k_quad(QuadArgs A, int max_steps)
+{
+    quad_run<INTEG, NA, false>(A, max_steps, nullptr, nullptr);
+}
+
+template <int INTEG, int NA>
+__global__ __launch_bounds__(4 * kQuadGasBodies) void k_quad_gas(QuadArgs A, int max_steps)
+{
+    extern __shared__ __attribute__((aligned(16))) double quad_columns[];
+    __shared__ QGas gas;
+    quad_run<INTEG, NA, true>(A, max_steps, quad_columns, &gas);
 }
 
 __global__ __launch_bounds__(kQuadMaxGroups) void k_quad_zero(QuadSync *s)
@@ -499,11 +750,27 @@ const void *quad_kernel_of(int sources)
                           : (const void *)k_quad<INTEG, 3>;
 }
 
-const void *quad_kernel(int integ, int sources)
+template <int INTEG>
+const void *quad_gas_kernel_of(int sources)
 {
-    return integ == INTEG_RKF78 ? quad_kernel_of<INTEG_RKF78>(sources)
-         : integ == INTEG_RK4   ? quad_kernel_of<INTEG_RK4>(sources)
-                                : quad_kernel_of<INTEG_DP>(sources);
+    return sources <= 3   ? (const void *)k_quad_gas<INTEG, 1>
+           : sources <= 7 ? (const void *)k_quad_gas<INTEG, 2>
+                          : (const void *)k_quad_gas<INTEG, 3>;
+}
+
+const void *quad_kernel(int integ, int sources, bool gas)
+{
+    return integ == INTEG_RKF78 ? (gas ? quad_gas_kernel_of<INTEG_RKF78>(sources) : quad_kernel_of<INTEG_RKF78>(sources))
+         : integ == INTEG_RK4   ? (gas ? quad_gas_kernel_of<INTEG_RK4>(sources) : quad_kernel_of<INTEG_RK4>(sources))
+                                : (gas ? quad_gas_kernel_of<INTEG_DP>(sources) : quad_kernel_of<INTEG_DP>(sources));
+}
+
+template <int INTEG>
+size_t column_bytes_of(int places) { return (size_t)(2 * (q_stages<INTEG>() + 1)) * 4 * places * sizeof(double); }
+size_t column_bytes(int integ, int places)
+{
+    return integ == INTEG_RKF78 ? column_bytes_of<INTEG_RKF78>(places)
+         : integ == INTEG_RK4   ? column_bytes_of<INTEG_RK4>(places) : column_bytes_of<INTEG_DP>(places);
 }
 
 }  // namespace
@@ -520,20 +787,48 @@ int quad_groups(int n, int sources, int cus)
 int quad_capacity(int integ, int sources, int cu_count)
 {
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, quad_kernel(integ, sources), kQuadThreads, 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, quad_kernel(integ, sources, false), kQuadThreads, 0) !=
         hipSuccess)
+        return 0;
+    return per_cu * cu_count;
+}
+
+int quad_gas_capacity(int integ, int sources, int places, int cu_count)
+{
+    const void *f = quad_kernel(integ, sources, true);
+    const int lds = (int)column_bytes(integ, places);
+    int per_cu = 0;
+    if (sources < 1 || sources > kQuadMaxSources || places <= sources || places > kQuadGasBodies ||
+        hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, 4 * places, lds) != hipSuccess)
         return 0;
     return per_cu * cu_count;
 }
 
 hipError_t launch_quad(hipStream_t st, int integ, const QuadArgs &a, int max_steps)
 {
-    if (a.groups < 1 || a.groups > kQuadMaxGroups || a.sources < 1 || a.sources > kQuadMaxSources)
+    if (a.groups < 1 || a.groups > kQuadMaxGroups || a.sources < 1 || a.sources > kQuadMaxSources ||
+        a.own != kQuads - a.sources)
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_quad_zero, dim3(1), dim3(kQuadMaxGroups), 0, st, a.sync);
     QuadArgs args = a;
     void *kargs[] = {&args, &max_steps};
-    return hipLaunchKernel(quad_kernel(integ, a.sources), dim3(a.groups), dim3(kQuadThreads), kargs, 0, st);
+    return hipLaunchKernel(quad_kernel(integ, a.sources, false), dim3(a.groups), dim3(kQuadThreads), kargs, 0, st);
+}
+
+hipError_t launch_quad_gas(hipStream_t st, int integ, const QuadArgs &a, int places, int max_steps)
+{
+    if (a.groups < 1 || a.groups > kQuadMaxGroups || a.sources < 1 || a.sources > kQuadMaxSources || a.own < 1 ||
+        a.sources + a.own > places || places > kQuadGasBodies || places % kQuads != 0)
+        return hipErrorInvalidValue;
+    const void *f = quad_kernel(integ, a.sources, true);
+    const size_t lds = column_bytes(integ, places);
+    hipError_t r = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (r != hipSuccess) return r;
+    hipLaunchKernelGGL(k_quad_zero, dim3(1), dim3(kQuadMaxGroups), 0, st, a.sync);
+    QuadArgs args = a;
+    void *kargs[] = {&args, &max_steps};
+    return hipLaunchKernel(f, dim3(a.groups), dim3(4 * places), kargs, lds, st);
 }
 
 }  // namespace sol
