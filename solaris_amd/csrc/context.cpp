@@ -177,9 +177,18 @@ void build_plan(sol_context *c)
     // reads.  k = 1, 2, 3, 4, 5: at 32,769 bodies 482, 460, 450, 481 (k = 4)
     // and 509 us for FP64 with 2 or 3 items in a workgroup; at 65,537 1,604
     // (k = 5) to 1,697 (k = 8) and 1,683 (k = 1), the epilogue 54, 49 and 90.
+    // Mixed precision, whose pairs take half the time, splits the items of small
+    // systems into units: pair sum and epilogue of 3,001 bodies 43 + 14 us with
+    // whole items, 25 + 15 with two units and 16 + 18 with four, 5,001 44 + 15,
+    // 28 + 17 and 22 + 21, 8,193 54 + 16, 40 + 20 and 34 + 26, 12,001 71 + 19,
+    // 57 + 23 and 54 + 32, 16,385 94 + 20, 85 + 27 and 113 + 40; FP64 gains
+    // what its epilogue loses (8,193 bodies 48 + 16, 45 + 19).
     // SOLARIS_AMD_SYM_WAVES overrides the count (tests use it to give each
     // workgroup many items).
-    const int64_t groups = (M - 1 + kSymGroup - 1) / kSymGroup, items = groups * (groups + 1) / 2;
+    const int64_t groups = (M - 1 + kSymGroup - 1) / kSymGroup;
+    int64_t items = groups * (groups + 1) / 2;
+    const int shift = !mixed_on(c) ? 0 : items <= 400 ? 2 : items <= 1600 ? 1 : 0;
+    items <<= shift;
     const int64_t most = (int64_t)c->cu_count * 26;
     const int64_t per = (items + most - 1) / most;
     int64_t waves = (items + per - 1) / per;
@@ -187,7 +196,7 @@ void build_plan(sol_context *c)
         const long v = std::atol(e);
         if (v > 0) waves = v;
     }
-    sym_plan_make(c->sym, M, waves);
+    sym_plan_make(c->sym, M, waves, shift);
     c->sym_inter_per_launch = (double)(M - 1) * (double)(M - 2);
     SegSpec rest[kMaxSeg];
     int nr = 0;
@@ -216,7 +225,7 @@ int ensure_partials(sol_context *c)
         g.max_cells = (int32_t)mc;
     }
     if (c->sym.M > 0) {
-        const size_t na = (size_t)c->sym.nitems * 3 * kSymGroup;
+        const size_t na = (size_t)sym_units(c->sym) * 3 * kSymGroup;
         const size_t nb = (size_t)c->sym.nwaves * c->sym.slots_per_wave * 3 * kSymGroup;
         if (na > c->apart_cap) {
             if (c->apart) (void)hipFree(c->apart);
@@ -666,6 +675,11 @@ SliceArrays system_arrays(sol_context *c)
 // From 32 sources on: an RKF78 attempt of 33 bodies takes 48 us on the mesh
 // and 58 in one workgroup, of 17 bodies 47 and 35.
 constexpr int kMeshMinSources = 32;
+// ... and to 23 bodies per workgroup, 5,889 bodies: RKF78 and Dormand-Prince, us
+// per attempt in the mesh form and with one launch per stage: 3,501 287 and 451,
+// 207 and 330; 5,001 464 and 465, 331 and 342; with 31 per workgroup 6,001 627
+// and 580, 452 and 426; 7,937 801 and 626, 582 and 461.
+constexpr int kMeshContextShare = 23;
 constexpr int kPathMesh = 100, kPathQuad = 101;     // reported as SOL_PATH_GRID
 
 bool use_mesh(sol_context *c, int ik, int *share_out = nullptr, int *groups_out = nullptr)
@@ -679,7 +693,7 @@ bool use_mesh(sol_context *c, int ik, int *share_out = nullptr, int *groups_out 
     source_ends(c, ea, eb);
     if (std::max(ea, eb) < kMeshMinSources) return false;
     const int share = mesh_share(c->n, c->n_massive, ea, eb, c->cu_count);
-    if (share == 0) return false;
+    if (share == 0 || share > kMeshContextShare) return false;
     const int groups = mesh_groups(c->n, c->n_massive, ea, eb, share);
     if (mesh_capacity(ik, c->n, share, c->cu_count) < groups) return false;
     if (share_out) *share_out = share;
@@ -1380,8 +1394,14 @@ int sol_set_precision(sol_context *c, int32_t precision, double softening)
         int r = dalloc(c, &c->J32, (size_t)c->np);
         if (r) return r;
     }
+    const bool plan = c->precision != precision;
     c->precision = precision;
     c->softening = softening;
+    if (plan) {
+        HIPCHECK(c, hipStreamSynchronize(c->stream));
+        build_plan(c);
+        return ensure_partials(c);
+    }
     return SOL_OK;
 }
 

@@ -500,9 +500,13 @@ __device__ __forceinline__ float rot_lane_f(float v)
 // (positions from J) to FP64 sums that travel with the packet.  As in the
 // FP64 kernel the packet's (x, y, z, k^2 m) are read from the wave's LDS
 // slice, one 16-byte read per step, and only its three FP32 sums rotate.
-// Per pair: 17 FP32 VALU operations and one v_rsq_f32.  Four waves per SIMD.
-// Measured before (whole items per wave) and after, us: 5,001 bodies 82 and
-// 44, 16,385 110 and 93, 32,769 339 and 277, 65,537 1,070 and 868.
+// Per pair: 17 FP32 VALU operations and one v_rsq_f32, 27 ns per wave's pair at
+// the rates under this load (1.4 and 4.4 ns), which bounds it from some 16,000
+// bodies on; below, a wave's 256 pairs per lane in turn do, so the plan splits
+// an item's steps over two or four units (context.cpp).  Four waves per SIMD.
+// Measured before (whole items per wave) and after, us: 3,001 bodies 81 and 16,
+// 5,001 82 and 22, 8,193 85 and 40, 16,385 110 and 93, 32,769 339 and 277,
+// 65,537 1,070 and 868.
 template <bool SOFT>
 __global__ __launch_bounds__(256, 4) void k_pairs_sym_mixed(SymPlan sp, const float4 *__restrict__ J32,
                                                          const double4 *__restrict__ J, double *__restrict__ apart,
@@ -517,7 +521,8 @@ __global__ __launch_bounds__(256, 4) void k_pairs_sym_mixed(SymPlan sp, const fl
     const int64_t lo = sym_wave_lo(sp, w), hi = sym_wave_lo(sp, w + 1);
     if (lo >= hi) return;
     int ag, hg;
-    sym_decode(lo, ag, hg);
+    sym_decode(lo >> sp.shift, ag, hg);
+    const int parts = 1 << sp.shift, len = kWave >> sp.shift;     // steps of a unit
     const float e2 = SOFT ? eps2 : 0.0f;
     float4 *pk = pk_lds[j];
     double *record = bpart + (int64_t)w * sp.slots_per_wave * (3 * kSymGroup);
@@ -543,6 +548,7 @@ __global__ __launch_bounds__(256, 4) void k_pairs_sym_mixed(SymPlan sp, const fl
     load_col();
     for (int64_t it = lo;; ) {
         const bool diag = (ag == hg);
+        const int part = (int)it & (parts - 1), k0 = part * len;
         const int ib = 1 + ag * kSymGroup + j * kWave + lane;
         const float4 v = ib < sp.M ? J32[ib] : make_float4(-1.0e18f, 0.0f, 0.0f, 0.0f);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -583,8 +589,8 @@ __global__ __launch_bounds__(256, 4) void k_pairs_sym_mixed(SymPlan sp, const fl
         // two steps per iteration, each packet body read one step ahead
         // (entry lane + k + 2 <= 127 stays in the slice)
         auto fp32_pass = [&](auto diag_c) {
-            float4 qa = pk[lane];
-            for (int k = 0; k < kWave; k += 2) {
+            float4 qa = pk[lane + k0];
+            for (int k = k0; k < k0 + len; k += 2) {
                 const float4 qb = pk[lane + k + 1];
                 step(qa, k, diag_c);
                 qa = pk[lane + k + 2];
@@ -602,7 +608,7 @@ __global__ __launch_bounds__(256, 4) void k_pairs_sym_mixed(SymPlan sp, const fl
         if (wave_far != ~0ull) {
             // replay the packet's steps for the close pairs, in FP64
             double hx = 0.0, hy = 0.0, hz = 0.0;
-            for (int k = 0; k < kWave; ++k) {
+            for (int k = k0; k < k0 + len; ++k) {
                 const float4 q = pk[lane + k];
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
@@ -633,12 +639,14 @@ __global__ __launch_bounds__(256, 4) void k_pairs_sym_mixed(SymPlan sp, const fl
             }
             cx += hx; cy += hy; cz += hz;
         }
-        double *r = apart + it * (3 * kSymGroup) + j * kWave + lane;
+        // after step k0 + len - 1 lane l has the sums of packet body l + k0 + len
+        double *r = apart + it * (3 * kSymGroup) + j * kWave + ((lane + k0 + len) & (kWave - 1));
         r[0] = cx;
         r[kSymGroup] = cy;
         r[2 * kSymGroup] = cz;
         ++it;
         const bool last = it >= hi;
+        if (part + 1 < parts && !last) continue;
         if (last || diag) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) {

@@ -225,22 +225,34 @@ __device__ bool gather_pairs(const EpiArgs &a, int i, double &px, double &py, do
         const SymPlan &sp = a.sym;
         const int g = (i - 1) / kSymGroup, r = (i - 1) - g * kSymGroup;
         // row records: independent loads, unrolled so that many are in flight
+        if (sp.shift == 0) {
+            const double *row = a.apart + (sym_col_start(g) + g) * (3 * kSymGroup) + r;
 #pragma unroll 8
-        for (int h = g; h < sp.ngroups; ++h) {
-            const double *q = a.apart + (sym_col_start(h) + g) * (3 * kSymGroup);
-            px += q[r];
-            py += q[kSymGroup + r];
-            pz += q[2 * kSymGroup + r];
+            for (int h = g; h < sp.ngroups; ++h) {
+                px += row[0];
+                py += row[kSymGroup];
+                pz += row[2 * kSymGroup];
+                row += (int64_t)(h + 1) * (3 * kSymGroup);
+            }
+        } else {
+#pragma unroll 8
+            for (int k = g << sp.shift; k < sp.ngroups << sp.shift; ++k) {
+                const int h = k >> sp.shift, unit = k & ((1 << sp.shift) - 1);
+                const double *row = a.apart + (((sym_col_start(h) + g) << sp.shift) + unit) * (3 * kSymGroup) + r;
+                px += row[0];
+                py += row[kSymGroup];
+                pz += row[2 * kSymGroup];
+            }
         }
-        // column records of the waves w0..w1 that cover column g's items
+        // column records of the waves w0..w1 that cover column g's units
         // [A, B).  The waves hold contiguous non-empty ranges, so every wave
         // after w0 starts inside the column (its slot 0): only w0's first
         // column is decoded, and the other loads are independent.
-        const int64_t A = sym_col_start(g), B = A + g + 1;
+        const int64_t A = sym_col_start(g) << sp.shift, B = sym_col_start(g + 1) << sp.shift;
         const int64_t w0 = sym_wave_of(sp, A), w1 = sym_wave_of(sp, B - 1);
         {
             int a0, h0;
-            sym_decode(sym_wave_lo(sp, w0), a0, h0);
+            sym_decode(sym_wave_lo(sp, w0) >> sp.shift, a0, h0);
             const double *q = a.bpart + (w0 * sp.slots_per_wave + (g - h0)) * (3 * kSymGroup);
             px += q[r];
             py += q[kSymGroup + r];

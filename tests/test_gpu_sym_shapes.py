@@ -2,7 +2,9 @@
 end one body into, one body short of and at the end of a group of 256 (and of
 a packet of 64), the smallest block, and workgroups of one item and of
 several, whose column sums pass from item to item; and the nearest-neighbour
-search after the pair sum (up to 8,191 bodies) and beside it.
+search after the pair sum (up to 8,191 bodies) and beside it.  In mixed
+precision also items of four, two and one units, and a change of the precision
+of a context, which changes its plan.
 
 FP64 against the one-directional sum (SOLARIS_AMD_NO_SYM=1): both round to a
 few 1e-16 of the sum of the terms' magnitudes, within 1e-14 of the total
@@ -46,7 +48,7 @@ def test_fp64_against_one_directional(n, waves):
     assert rel(a, b) <= 1e-14
 
 
-@pytest.mark.parametrize("n", [2048, 2049, 2113, 2305, 6337])
+@pytest.mark.parametrize("n", [2048, 2049, 2113, 2305, 6337, 7168, 7169, 14336, 14337])
 def test_mixed_against_fp64(n):
     scn = S.make_c3(n=n)
     a = accelerations(scn, runtime.MIXED)
@@ -74,3 +76,16 @@ def test_neighbours_after_and_beside_the_pair_sum(n):
         assert rel(a[1:, 3:], b[1:, 3:]) <= 1e-14
         assert np.array_equal(sa[1], sb[1])
         np.testing.assert_allclose(sa[2], sb[2], rtol=1e-12, atol=0)
+
+
+def test_change_of_precision():
+    scn = S.make_c3(n=6337)
+    ctx = runtime.Context(scn, precision=runtime.MIXED)
+    ctx.set_side_outputs(False)
+    out = []
+    for precision in (runtime.MIXED, 0, runtime.MIXED):
+        ctx.set_precision(precision, scn.softening)
+        out.append(ctx.compute(0.0, scn.y0)[1:, 3:])
+    assert np.array_equal(out[0], out[2])
+    assert np.array_equal(out[1], accelerations(scn))
+    assert rel(out[0], out[1]) <= 1e-7
