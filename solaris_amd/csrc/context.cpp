@@ -705,8 +705,8 @@ bool use_mesh(sol_context *c, int ik, int *share_out = nullptr, int *groups_out 
 // ones, that have at most eight sources besides the star and bodies for at
 // most a workgroup per CU (14,339 with two planets).  The Sun, two planets and
 // test particles, us per RKF78 attempt in one workgroup or in slices, and in
-// quads: 4 bodies 15 and 5.4, 128 15 and 5.2, 515 17.6 and 5.6, 5,001 18.6 and
-// 6.1, 14,338 20.4 and 6.9.  With live gas: the grid form's slices of 64 and
+// quads: 4 bodies 15 and 7.0, 128 15 and 6.6, 515 17.7 and 6.9, 5,001 18.8 and
+// 7.4, 14,338 20.4 and 8.1.  With live gas: the grid form's slices of 64 and
 // 128 places, us per RKF78 attempt: 125 bodies 64 (one workgroup) and 31, 505
 // 51 and 31, 16,389 56 and 38.
 struct QuadShape { int sources, own, groups, places; };   // places: bodies of a workgroup with gas (0: no gas)

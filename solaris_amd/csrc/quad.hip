@@ -9,10 +9,9 @@
 // 17 us per RKF78 attempt for 1.3 us per stage.  What bounds it is thus the
 // number of operations in one lane, and here four lanes share a body:
 //
-//   pulls       lane l takes the pulls of bodies l, l + 4, ... (the star, body
-//               0, as a source at the origin with weight k^2 (m0 + mi)), and
-//               each source's indirect term with its direct one; the sums are
-//               reduced over the quad so that lane c (c < 3) has component c;
+//   pulls       lane l takes the pulls of sources l, l + 4, ..., each with its
+//               indirect term, and lane 0 the body's own 1 / r^3; lane c
+//               (c < 3) gathers and adds component c;
 //   state       lane c keeps component c of position and velocity and of all
 //               stage derivatives in registers (the stages are unrolled) and
 //               forms only that component of the next state.
@@ -25,9 +24,9 @@
 // accepted with.
 //
 // Per attempt, before (slices of resident.hip, below 129 bodies one workgroup)
-// and after, us: RKF78 of 4 bodies 15.2 and 5.4, 515 17.6 and 5.6, 5,001 18.6
-// and 6.1, 14,338 20.4 and 6.9; Dormand-Prince of 515 13.9 and 4.9; RK4 of 515
-// 4.4 and 1.2.  An evaluation of 85 to 100 instructions takes 0.28 us, the
+// and after, us: RKF78 of 4 bodies 15.2 and 7.0, 515 17.7 and 6.9, 5,001 18.8
+// and 7.4, 14,338 20.4 and 8.1; Dormand-Prince of 515 13.7 and 5.7; RK4 of 515
+// 4.4 and 1.5.  An evaluation of about 120 instructions takes 0.38 us, the
 // exchange 1.9 us.  With gas, RKF78 of 505 bodies 51.6 and 31.1, 4,005 52.0 and
 // 30.2, 16,389 55.8 and 38.3.
 #include <float.h>
@@ -62,90 +61,154 @@ __device__ __forceinline__ double quad_wmax(double v)
     return v;
 }
 
-// What a lane needs for the pulls on its body: NA of them, l, l + 4, ...
+// What a lane needs for the pulls on its body.
 template <int NA>
 struct QPulls {
-    double w[NA], u[NA];       // weights of the direct and the indirect term (0: not a source of this body)
-    int slot[NA];              // the source's record
+    double mu;                 // k^2 (m0 + mi)
+    double w[4 * NA];          // k^2 m of source a (0: not a source of this body); with gas w[t] of
+                               // this lane's (mu for the star, source 0)
+    int slot[NA];              // the records of this lane's sources l, l + 4, ...
     bool near[NA];             // a candidate for the nearest neighbour
 };
 
 // |d|^-3 from r2 = |d|^2: the hardware's reciprocal square root and its
-// second-order correction.  Its cap is above 1 / |d| of any two distinct
-// bodies, so that a body's own record and the star's indirect term (d = 0)
-// come out as exactly 0.
-__device__ __forceinline__ double quad_rm3(double r2, double c15, double c1875)
+// second-order correction, as pair_range in resident.hip.  Its cap is above
+// 1 / |d| of any two distinct bodies, so that a body's own record (d = 0, weight
+// 0) comes out finite.
+__device__ __forceinline__ double quad_rm3(double r2)
 {
     const double y = fmin(__builtin_amdgcn_rsq(r2), 1.0e50);
     const double tt = y * y;
     const double e = __builtin_fma(-r2, tt, 1.0);
     const double y3 = tt * y;
-    return __builtin_fma(y3, e * __builtin_fma(c1875, e, c15), y3);
+    return __builtin_fma(y3, e * __builtin_fma(1.875, e, 1.5), y3);
 }
 
-// Side outputs of a body: 1 / |r|^3 (lane 0), distance squared and index of
-// the nearest source.
+// x^2 + y^2 + z^2, the first or the second square rounded first.
+template <bool SECOND>
+__device__ __forceinline__ double quad_sq(double x, double y, double z)
+{
+    return __builtin_fma(z, z, SECOND ? __builtin_fma(x, x, y * y) : __builtin_fma(y, y, x * x));
+}
+
+// The value of lane LANE of the quad in all four.
+template <int LANE>
+__device__ __forceinline__ double quad_from(double v) { return dpp_mov<LANE * 0x55>(v); }
+
+// Side outputs of a body: 1 / |r|^3, distance squared and index of the nearest
+// source.
 struct QSide {
     double rm3, best;
     int idx;
 };
 
+// The nearest of the quad's four lanes, the smaller index of equals.
+__device__ __forceinline__ void quad_nearest(QSide &side)
+{
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const double ob = s == 0 ? dpp_mov<0xB1>(side.best) : dpp_mov<0x4E>(side.best);
+        const int oi = s == 0 ? __builtin_amdgcn_mov_dpp(side.idx, 0xB1, 0xF, 0xF, false)
+                              : __builtin_amdgcn_mov_dpp(side.idx, 0x4E, 0xF, 0xF, false);
+        const bool take = ob < side.best || (ob == side.best && oi < side.idx);
+        side.best = take ? ob : side.best;
+        side.idx = take ? oi : side.idx;
+    }
+}
+
 // Acceleration component of this lane for the position whose component it
-// holds.  tab: the source records (x, y, z), [0] the origin; the wave's own,
-// or with BLOCK the workgroup's (two sets in turn, so that one barrier between
-// writing and reading suffices).
-template <int NA, bool SIDE, bool BLOCK = false>
-__device__ __forceinline__ double quad_force(const QPulls<NA> &P, double (*tab)[4], int src, int l, double pos,
+// holds.  tab: the wave's source records (x, y, z), [0] the origin.
+//
+// Lane l forms d_a / |d_a|^3 - r_a / |r_a|^3 of its sources a and lane 0 the
+// body's own 1 / |r|^3; lane c gathers component c of all and adds the weighted
+// terms in the sources' order.  Every operation is that of resident.hip on the
+// same operands, fused as the compiler fuses it there (FIRST: a step's first
+// evaluation, which it fuses in another order than the stages'), so a run has
+// the same bits in quads, in slices and in one workgroup.  (Weights in the
+// lanes and a reduction over the quad take 85 instead of 120 operations, 5.6
+// instead of 7.0 us per RKF78 attempt of 515 bodies, but round otherwise, and a
+// particle's encounters over some years grow that to 1e-7.)
+template <int NA, bool SIDE, bool FIRST>
+__device__ __forceinline__ double quad_force(const QPulls<NA> &P, double (*tab)[4], int ns, int src, int l, double pos,
                                              QSide &side)
 {
     if (src > 0) tab[src][l] = pos;
-    const double x = dpp_mov<0x00>(pos), y = dpp_mov<0x55>(pos), z = dpp_mov<0xAA>(pos);
-    if (BLOCK) {
-        __syncthreads();
-    } else {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    }
-    const double c15 = 1.5, c1875 = 1.875;
-    double f[3] = {0.0, 0.0, 0.0};
+    const double x = quad_from<0>(pos), y = quad_from<1>(pos), z = quad_from<2>(pos);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
     if (SIDE) { side.best = DBL_MAX; side.idx = 0x7fffffff; }
+    double rm3 = 0.0, sum = 0.0;
+    static_for<0, NA>([&](auto T) {
+        constexpr int t = T;
+        const double *rec = tab[P.slot[t]];
+        double rx = rec[0], ry = rec[1], rz = rec[2];
+        const double dx = rx - x, dy = ry - y, dz = rz - z;
+        const double d2 = quad_sq<true>(dx, dy, dz);
+        const double wd = quad_rm3(d2);
+        if (t == 0) {                          // lane 0: the body itself
+            rx = l == 0 ? x : rx;
+            ry = l == 0 ? y : ry;
+            rz = l == 0 ? z : rz;
+        }
+        const double r2 = quad_sq<FIRST>(rx, ry, rz);
+        const double r = sqrt(r2);
+        const double m3 = 1.0 / (r2 * r);
+        if (t == 0) rm3 = quad_from<0>(m3);
+        const double gx = __builtin_fma(dx, wd, -(rx * m3)), gy = __builtin_fma(dy, wd, -(ry * m3)),
+                     gz = __builtin_fma(dz, wd, -(rz * m3));
+        if (SIDE && P.near[t] && d2 < side.best) { side.best = d2; side.idx = P.slot[t]; }
+        static_for<(t == 0 ? 1 : 0), 4>([&](auto L) {
+            constexpr int a = 4 * t + L;
+            if (a <= ns) {
+                const double u = quad_from<L>(gx), v = quad_from<L>(gy), w = quad_from<L>(gz);
+                sum = __builtin_fma(P.w[a], l == 0 ? u : l == 1 ? v : w, sum);
+            }
+        });
+    });
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (SIDE) {
+        side.rm3 = rm3;
+        quad_nearest(side);
+    }
+    return __builtin_fma(-P.mu * rm3, pos, sum);
+}
+
+// The same with gas, whose drag outweighs the rest: weights in the lanes (the
+// star as a source at the origin), a reduction over the quad, and no root or
+// division.  tab: the workgroup's records, two sets in turn, so that one barrier
+// between writing and reading suffices.  38 instead of 44 us per RKF78 attempt
+// of 16,389 bodies.
+template <int NA>
+__device__ __forceinline__ double quad_force_gas(const QPulls<NA> &P, double (*tab)[4], int src, int l, double pos,
+                                                 QSide &side)
+{
+    if (src > 0) tab[src][l] = pos;
+    const double x = quad_from<0>(pos), y = quad_from<1>(pos), z = quad_from<2>(pos);
+    __syncthreads();
+    double f[3] = {0.0, 0.0, 0.0};
+    side.best = DBL_MAX;
+    side.idx = 0x7fffffff;
 #pragma unroll
     for (int t = 0; t < NA; ++t) {
         const double *r = tab[P.slot[t]];
         const double rx = r[0], ry = r[1], rz = r[2];
         const double dx = rx - x, dy = ry - y, dz = rz - z;
         const double d2 = dx * dx + dy * dy + dz * dz;
-        const double s2 = rx * rx + ry * ry + rz * rz;
-        const double wd = quad_rm3(d2, c15, c1875), ws = quad_rm3(s2, c15, c1875);
-        const double g = P.w[t] * wd, k = P.u[t] * ws;
+        const double wd = quad_rm3(d2), ws = quad_rm3(rx * rx + ry * ry + rz * rz);
+        const double g = P.w[t] * wd, k = t == 0 && l == 0 ? 0.0 : P.w[t] * ws;
         f[0] += g * dx - k * rx;
         f[1] += g * dy - k * ry;
         f[2] += g * dz - k * rz;
-        if (SIDE) {
-            if (t == 0) side.rm3 = wd;          // lane 0: the star
-            if (P.near[t] && d2 < side.best) { side.best = d2; side.idx = P.slot[t]; }
-        }
+        if (t == 0) side.rm3 = quad_from<0>(wd);
+        if (P.near[t] && d2 < side.best) { side.best = d2; side.idx = P.slot[t]; }
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    quad_nearest(side);
     // lanes 0, 1 keep components 0, 1 and lanes 2, 3 component 2
     const bool hi = l >= 2;
     const double a = (hi ? f[2] : f[0]) + dpp_mov<0x4E>(hi ? f[0] : f[2]);
     const double b = f[1] + dpp_mov<0x4E>(f[1]);
-    const double keep = l == 1 ? b : a, send = l == 0 ? b : a;
-    if (SIDE) {
-        // the smaller index of equals
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const double ob = s == 0 ? dpp_mov<0xB1>(side.best) : dpp_mov<0x4E>(side.best);
-            const int oi = s == 0 ? __builtin_amdgcn_mov_dpp(side.idx, 0xB1, 0xF, 0xF, false)
-                                  : __builtin_amdgcn_mov_dpp(side.idx, 0x4E, 0xF, 0xF, false);
-            const bool take = ob < side.best || (ob == side.best && oi < side.idx);
-            side.best = take ? ob : side.best;
-            side.idx = take ? oi : side.idx;
-        }
-    }
-    return keep + dpp_mov<0xB1>(send);
+    return (l == 1 ? b : a) + dpp_mov<0xB1>(l == 0 ? b : a);
 }
 
 // Stage derivatives of one component: velocities V and accelerations F, in
@@ -179,32 +242,56 @@ struct QBody {
     double sp, sv, ep, ev;
 };
 
-// State of stage S in tableau order, as resident.hip's stage_state.
+// Coefficient L of stage S, and the first two stages l with a nonzero one (S
+// if there is none).
+template <int INTEG, int S>
+constexpr double q_coef(int l)
+{
+    return INTEG == INTEG_RKF78 ? tab::kRkfD[S][l] : INTEG == INTEG_RK4 ? tab::kRk4A[S][l] : tab::kDpA[S][l];
+}
+template <int INTEG, int S>
+constexpr int q_nonzero(int from)
+{
+    for (int l = from; l < S; ++l)
+        if (q_coef<INTEG, S>(l) != 0.0) return l;
+    return S;
+}
+
+// c0 f0 + c1 f1, the first or the second product rounded first.
+template <bool SECOND>
+__device__ __forceinline__ double quad_two(double c0, double f0, double c1, double f1)
+{
+    return SECOND ? __builtin_fma(c0, f0, c1 * f1) : __builtin_fma(c1, f1, c0 * f0);
+}
+
+// The sum of coefficient times derivative over the nonzero coefficients of
+// stage S in tableau order, fused as the compiler fuses it in resident.hip.
+template <int INTEG, int S, typename Get>
+__device__ __forceinline__ double quad_sum(Get f)
+{
+    constexpr int l0 = q_nonzero<INTEG, S>(0), l1 = q_nonzero<INTEG, S>(l0 + 1);
+    if constexpr (l1 >= S) {
+        return q_coef<INTEG, S>(l0) * f(l0);
+    } else {
+        constexpr double c0 = q_coef<INTEG, S>(l0), c1 = q_coef<INTEG, S>(l1);
+        double acc = quad_two<!(l1 == S - 1 || (c0 < 0.0 && c1 > 0.0))>(c0, f(l0), c1, f(l1));
+        static_for<l1 + 1, S>([&](auto L) {
+            if constexpr (q_coef<INTEG, S>(L) != 0.0) acc = __builtin_fma(q_coef<INTEG, S>(L), f(L), acc);
+        });
+        return acc;
+    }
+}
+
+// State of stage S, as resident.hip's stage_state.
 template <int INTEG, int S, bool LDS>
 __device__ __forceinline__ void quad_stage(const QBody<LDS> &B, double h, double &pos, double &vel)
 {
-    if constexpr (INTEG == INTEG_DP) {
-        double var = tab::kDpA[S][0] * B.d.F(0);
-        static_for<1, S>([&](auto L) {
-            if constexpr (tab::kDpA[S][L] != 0.0) var += tab::kDpA[S][L] * B.d.F(L);
-        });
-        pos = B.p + tab::kDpC[S] * h * B.v + h * h * (var);
-        vel = B.v + h * (var);
-    } else {
-        double ap = 0.0, av = 0.0;
-        bool first = true;
-        static_for<0, S>([&](auto L) {
-            constexpr double d = INTEG == INTEG_RKF78 ? tab::kRkfD[S][L] : tab::kRk4A[S][L];
-            if constexpr (d != 0.0) {
-                const double x = d * B.d.V(L), y = d * B.d.F(L);
-                ap = first ? x : ap + x;
-                av = first ? y : av + y;
-                first = false;
-            }
-        });
-        pos = B.p + h * ap;
-        vel = B.v + h * av;
-    }
+    const double av = quad_sum<INTEG, S>([&](int l) { return B.d.F(l); });
+    if constexpr (INTEG == INTEG_DP)
+        pos = __builtin_fma(h * h, av, __builtin_fma(tab::kDpC[S] * h, B.v, B.p));
+    else
+        pos = __builtin_fma(h, quad_sum<INTEG, S>([&](int l) { return B.d.V(l); }), B.p);
+    vel = __builtin_fma(h, av, B.v);
 }
 
 // Final state and error estimate (kept in B); returns this lane's part of the
@@ -212,31 +299,42 @@ __device__ __forceinline__ void quad_stage(const QBody<LDS> &B, double h, double
 template <int INTEG, bool LDS>
 __device__ __forceinline__ double quad_final(QBody<LDS> &B, double h, double &pos, double &vel)
 {
+    auto V = [&](int l) { return B.d.V(l); };
+    auto F = [&](int l) { return B.d.F(l); };
     if constexpr (INTEG == INTEG_RKF78) {
         constexpr double b0 = 41.0 / 840.0, b5 = 34.0 / 105.0, b6 = 9.0 / 35.0, b8 = 9.0 / 280.0, b10 = 41.0 / 840.0;
-        auto sum = [&](auto F) {
-            return b0 * F(0) + b5 * F(5) + b6 * (F(6) + F(7)) + b8 * (F(8) + F(9)) + b10 * F(10);
+        auto sum = [&](auto f) {
+            double s = quad_two<true>(b0, f(0), b5, f(5));
+            s = __builtin_fma(b6, f(6) + f(7), s);
+            s = __builtin_fma(b8, f(8) + f(9), s);
+            return __builtin_fma(b10, f(10), s);
         };
-        auto V = [&](int l) { return B.d.V(l); };
-        auto F = [&](int l) { return B.d.F(l); };
-        pos = B.p + h * sum(V);
-        vel = B.v + h * sum(F);
+        pos = __builtin_fma(h, sum(V), B.p);
+        vel = __builtin_fma(h, sum(F), B.v);
         B.ep = h * fabs(V(0) + V(10) - V(11) - V(12)) * 41.0 / 840.0;
         B.ev = h * fabs(F(0) + F(10) - F(11) - F(12)) * 41.0 / 840.0;
         return fmax(fabs(B.ep / B.sp), fabs(B.ev / B.sv));
     } else if constexpr (INTEG == INTEG_RK4) {
-        auto sum = [&](auto F) {
-            return tab::kRk4B[0] * F(0) + tab::kRk4B[1] * F(1) + tab::kRk4B[2] * F(2) + tab::kRk4B[3] * F(3);
+        constexpr const double *b = tab::kRk4B;
+        auto sum = [&](auto f) {
+            return __builtin_fma(b[3], f(3), __builtin_fma(b[2], f(2), quad_two<true>(b[0], f(0), b[1], f(1))));
         };
-        pos = B.p + h * sum([&](int l) { return B.d.V(l); });
-        vel = B.v + h * sum([&](int l) { return B.d.F(l); });
+        pos = __builtin_fma(h, sum(V), B.p);
+        vel = __builtin_fma(h, sum(F), B.v);
         return 0.0;
     } else {
         constexpr const double *b = tab::kDpB, *d = tab::kDpBdh;
-        auto F = [&](int l) { return B.d.F(l); };
         const double h2 = h * h;
-        pos = B.p + h * B.v + h2 * (b[0] * F(0) + b[4] * F(4) + b[5] * F(5) + b[6] * F(6) + b[7] * F(7) + b[8] * F(8));
-        vel = B.v + h * (d[0] * F(0) + d[4] * F(4) + d[5] * F(5) + d[6] * F(6) + d[7] * F(7));
+        double s = quad_two<false>(b[0], F(0), b[4], F(4)), u = quad_two<false>(d[0], F(0), d[4], F(4));
+        s = __builtin_fma(b[5], F(5), s);
+        u = __builtin_fma(d[5], F(5), u);
+        s = __builtin_fma(b[6], F(6), s);
+        u = __builtin_fma(d[6], F(6), u);
+        s = __builtin_fma(b[7], F(7), s);
+        u = __builtin_fma(d[7], F(7), u);
+        s = __builtin_fma(b[8], F(8), s);
+        pos = __builtin_fma(h2, s, __builtin_fma(h, B.v, B.p));
+        vel = __builtin_fma(h, u, B.v);
         B.ep = h2 * fabs(F(7) - F(8)) / 20.0;
         B.ev = 0.0;
         return B.ep;
@@ -361,14 +459,15 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
     QPulls<NA> P;
     {
         const int end = i < S.nm ? S.end_a : S.end_b;
+        P.mu = kGauss2 * (A.mass[0] + A.mass[i]);
+#pragma unroll
+        for (int a = 0; a < (GAS ? 0 : 4 * NA); ++a) P.w[a] = a >= 1 && a <= ns && a < end && a != i ? A.gm[a] : 0.0;
 #pragma unroll
         for (int t = 0; t < NA; ++t) {
             const int a = l + 4 * t;
-            const bool is = a >= 1 && a <= ns && a < end && a != i;
             P.slot[t] = a <= ns ? a : 0;
-            P.u[t] = is ? A.gm[a] : 0.0;
-            P.w[t] = a == 0 ? kGauss2 * (A.mass[0] + A.mass[i]) : P.u[t];
-            P.near[t] = is;
+            P.near[t] = a >= 1 && a <= ns && a < end && a != i;
+            if (GAS) P.w[t] = a == 0 ? P.mu : P.near[t] ? A.gm[a] : 0.0;
         }
     }
     QBody<GAS> B;
@@ -434,7 +533,7 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
     };
     // Acceleration at (pos, vel) with the gas's factor and the migration m.
     auto accelerate = [&](double pos, double vel, double factor, double m, QSide &sd) -> double {
-        double f = quad_force<NA, true, true>(P, tab, src, l, pos, sd);
+        double f = quad_force_gas<NA>(P, tab, src, l, pos, sd);
         tab = tab == records[0] ? records[1] : records[0];
         if (drags) {
             drag = quad_drag((const QUAD_LDS QGas *)gas, factor, dpp_mov<0x00>(pos), dpp_mov<0x55>(pos), dpp_mov<0xAA>(pos),
@@ -447,7 +546,7 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
     // f0 of the next step: the acceleration at (p, v)
     double f0 = 0.0;
     bool again = GAS;          // with gas f0 is formed at the step's start: the first one, and after a flush
-    if constexpr (!GAS) f0 = quad_force<NA, false>(P, tab, src, l, B.p, none);
+    if constexpr (!GAS) f0 = quad_force<NA, false, true>(P, tab, ns, src, l, B.p, none);
 
     for (int step = 0; step < max_steps; ++step) {
         const double t0 = S.t;
@@ -493,8 +592,8 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
             } else {
                 static_for<1, nst + 1>([&](auto T) {
                     quad_stage<INTEG, T>(B, h, pos, vel);
-                    if constexpr (T < nst) B.d.put(T, vel, quad_force<NA, false>(P, tab, src, l, pos, none));
-                    else B.d.put(T, vel, quad_force<NA, true>(P, tab, src, l, pos, side));
+                    if constexpr (T < nst) B.d.put(T, vel, quad_force<NA, false, false>(P, tab, ns, src, l, pos, none));
+                    else B.d.put(T, vel, quad_force<NA, true, false>(P, tab, ns, src, l, pos, side));
                 });
             }
             const double ratio = quad_final<INTEG>(B, h, pos, vel);
@@ -508,7 +607,7 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
                     f0 = accelerate(pos, vel, reduction_factor(A.gas, tn), mig_next, none);
                     drag = last_drag;
                 } else {
-                    f0 = quad_force<NA, false>(P, tab, src, l, pos, none);
+                    f0 = quad_force<NA, false, true>(P, tab, ns, src, l, pos, none);
                 }
             };
             if (combine) {
@@ -673,7 +772,7 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
             if (fabs(B.po) < 1.0e-50) B.po = 0.0;
             if (fabs(B.vo) < 1.0e-50) B.vo = 0.0;
             if constexpr (GAS) again = true;
-            else f0 = quad_force<NA, false>(P, tab, src, l, B.p, none);
+            else f0 = quad_force<NA, false, true>(P, tab, ns, src, l, B.p, none);
         }
         if (S.status != RES_RUNNING) break;
     }

@@ -6,7 +6,8 @@ the sizes where it changes: one to three, four to seven and eight sources (one,
 two and three pulls per lane); waves with one body of their own and full ones;
 one workgroup and two; the largest system; sink classes of their own source
 ranges; events, outputs and the small-number flush; a step that underflows; and
-a wait that gives up.
+a wait that gives up.  Runs have the same bits as in slices
+(SOLARIS_AMD_GRID_BLOCK=64), whose sums the quads follow.
 
 Tolerances as in test_gpu_mesh.py: both sums round to a few 1e-16 per term, so
 accelerations agree within the 1e-12 of the force tests, and a state after one
@@ -161,3 +162,20 @@ def test_many_launches():
     for _ in range(20):
         assert a.driver(RK4, 0.0, ta)[0] == 0 and b.driver(RK4, 0.0, tb)[0] == 0
     assert np.abs(a.get_array(runtime.Y0) - b.get_array(runtime.Y0)).max() <= 20 * 1e-13
+
+
+@pytest.mark.parametrize("n,sources", [(515, 2), (1033, 3), (300, 7), (300, 8)])
+@pytest.mark.parametrize("integrator", [RKF78, RK4, DP])
+def test_same_bits_as_slices(n, sources, integrator):
+    scn = system(n, sources)
+    out = []
+    for env in ({}, {"SOLARIS_AMD_GRID_BLOCK": "64"}):
+        ctx = make_ctx(scn, **env)
+        tl = _abi.timeline(0.0, 0.01, 1000.0, output=300.0)
+        r, st = ctx.integrate(integrator, 1e-10, tl, max_steps=400)
+        assert r == 0 and st.path == _abi.PATH_GRID
+        out.append([ctx.get_array(w) for w in (runtime.Y0, runtime.Y, runtime.ACCEL, runtime.ERROR)] +
+                   list(ctx.side_outputs()) + [tl.time, tl.hNext, st.attempts])
+    print(f"[quad bits, {n} bodies, {sources} sources, integrator {integrator}] {out[0][-1]} attempts", flush=True)
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
