@@ -159,8 +159,9 @@ typedef struct sol_run_stats {
 
 /* sol_run_stats.path: one launch per stage (gravity, gas and stage-combine
  * kernels); whole Driver loops in one workgroup (small systems); whole
- * Driver loops in slices of the system, one workgroup each, with the step
- * decisions combined over a cooperative grid (systems with few sources). */
+ * Driver loops over several workgroups of one launch, which exchange step
+ * decisions (systems with few sources) or also positions (self-gravitating
+ * systems of 32 to 5,889 bodies). */
 enum { SOL_PATH_MULTI_KERNEL = 0, SOL_PATH_RESIDENT = 1, SOL_PATH_GRID = 2 };
 
 typedef struct sol_context sol_context;
