@@ -27,11 +27,12 @@
 // and after, us: RKF78 of 4 bodies 15.2 and 7.0, 515 17.7 and 6.9, 5,001 18.8
 // and 7.4, 14,338 20.4 and 8.1; Dormand-Prince of 515 13.7 and 5.7; RK4 of 515
 // 4.4 and 1.5.  An evaluation of about 120 instructions takes 0.38 us, the
-// exchange 1.9 us.  With gas, RKF78 of 505 bodies 51.6 and 31.1, 4,005 52.0 and
-// 30.2, 16,389 55.8 and 38.3.
+// exchange 1.9 us.  With gas, RKF78 of 125 bodies 63.7 and 34.3, 505 50.6 and
+// 34.3, 16,389 55.9 and 41.3.
 #include <float.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "gasdev.h"
 #include "lane_pairs.h"
@@ -65,8 +66,7 @@ __device__ __forceinline__ double quad_wmax(double v)
 template <int NA>
 struct QPulls {
     double mu;                 // k^2 (m0 + mi)
-    double w[4 * NA];          // k^2 m of source a (0: not a source of this body); with gas w[t] of
-                               // this lane's (mu for the star, source 0)
+    double w[4 * NA];          // k^2 m of source a (0: not a source of this body)
     int slot[NA];              // the records of this lane's sources l, l + 4, ...
     bool near[NA];             // a candidate for the nearest neighbour
 };
@@ -174,41 +174,72 @@ __device__ __forceinline__ double quad_force(const QPulls<NA> &P, double (*tab)[
     return __builtin_fma(-P.mu * rm3, pos, sum);
 }
 
-// The same with gas, whose drag outweighs the rest: weights in the lanes (the
-// star as a source at the origin), a reduction over the quad, and no root or
-// division.  tab: the workgroup's records, two sets in turn, so that one barrier
-// between writing and reading suffices.  38 instead of 44 us per RKF78 attempt
-// of 16,389 bodies.
-template <int NA>
-__device__ __forceinline__ double quad_force_gas(const QPulls<NA> &P, double (*tab)[4], int src, int l, double pos,
-                                                 QSide &side)
+// The same with gas, in two halves: the sources' quads publish r_a and r_a /
+// |r_a|^3, and after a barrier every quad forms its pulls, so that a quad takes
+// one root and one division for its own |r|^-3 and none per record.  The lanes
+// share that root and division with the drag's: base is the cylindrical radius
+// rc (lane 2: the spherical one), over_rc3 mu / rc^3.  tab: the workgroup's
+// records (x, y, z, -, and those times |r|^-3), two sets in turn, so that one
+// barrier between writing and reading suffices.
+//
+// The operations are those of quad_force, so what differs from resident.hip is
+// the drag's last bits alone, which rarely reach an acceleration some 1e7 times
+// as large.  (A root of each record's own and sums over the lanes take 39.8
+// instead of 41.3 us per RKF78 attempt of 16,389 bodies, but round otherwise,
+// and over 100 days a planetesimal's encounters grow that to 1e-8; with
+// quad_force itself 44.)
+struct QGasPlace {
+    double x, y, z, base, rm3, over_rc3;
+};
+
+template <bool FIRST>
+__device__ __forceinline__ QGasPlace quad_publish(double (*tab)[8], int src, int l, double pos, double mu)
 {
-    if (src > 0) tab[src][l] = pos;
-    const double x = quad_from<0>(pos), y = quad_from<1>(pos), z = quad_from<2>(pos);
-    __syncthreads();
-    double f[3] = {0.0, 0.0, 0.0};
+    QGasPlace W;
+    W.x = quad_from<0>(pos);
+    W.y = quad_from<1>(pos);
+    W.z = quad_from<2>(pos);
+    const double r2 = quad_sq<FIRST>(W.x, W.y, W.z), q = SQR(W.x) + SQR(W.y);
+    W.base = sqrt(l == 2 ? r2 : q);
+    const double rc = quad_from<0>(W.base), r = quad_from<2>(W.base);
+    const double part = (l < 2 ? 1.0 : mu) / (l < 2 ? r2 * r : q * rc);
+    W.rm3 = quad_from<0>(part);
+    W.over_rc3 = quad_from<2>(part);
+    if (src > 0) {
+        tab[src][l] = pos;
+        tab[src][4 + l] = pos * W.rm3;
+    }
+    return W;
+}
+
+// Acceleration component of this lane; last: the nearest source too.
+template <int NA>
+__device__ __forceinline__ double quad_force_gas(const QPulls<NA> &P, double (*tab)[8], int ns, int l, double pos,
+                                                 const QGasPlace &W, bool last, QSide &side)
+{
+    side.rm3 = W.rm3;
     side.best = DBL_MAX;
     side.idx = 0x7fffffff;
-#pragma unroll
-    for (int t = 0; t < NA; ++t) {
-        const double *r = tab[P.slot[t]];
-        const double rx = r[0], ry = r[1], rz = r[2];
-        const double dx = rx - x, dy = ry - y, dz = rz - z;
-        const double d2 = dx * dx + dy * dy + dz * dz;
-        const double wd = quad_rm3(d2), ws = quad_rm3(rx * rx + ry * ry + rz * rz);
-        const double g = P.w[t] * wd, k = t == 0 && l == 0 ? 0.0 : P.w[t] * ws;
-        f[0] += g * dx - k * rx;
-        f[1] += g * dy - k * ry;
-        f[2] += g * dz - k * rz;
-        if (t == 0) side.rm3 = quad_from<0>(wd);
+    double sum = 0.0;
+    static_for<0, NA>([&](auto T) {
+        constexpr int t = T;
+        const double *rec = tab[P.slot[t]];
+        const double dx = rec[0] - W.x, dy = rec[1] - W.y, dz = rec[2] - W.z;
+        const double d2 = quad_sq<true>(dx, dy, dz);
+        const double wd = quad_rm3(d2);
+        const double gx = __builtin_fma(dx, wd, -rec[4]), gy = __builtin_fma(dy, wd, -rec[5]),
+                     gz = __builtin_fma(dz, wd, -rec[6]);
         if (P.near[t] && d2 < side.best) { side.best = d2; side.idx = P.slot[t]; }
-    }
-    quad_nearest(side);
-    // lanes 0, 1 keep components 0, 1 and lanes 2, 3 component 2
-    const bool hi = l >= 2;
-    const double a = (hi ? f[2] : f[0]) + dpp_mov<0x4E>(hi ? f[0] : f[2]);
-    const double b = f[1] + dpp_mov<0x4E>(f[1]);
-    return (l == 1 ? b : a) + dpp_mov<0xB1>(l == 0 ? b : a);
+        static_for<(t == 0 ? 1 : 0), 4>([&](auto L) {
+            constexpr int a = 4 * t + L;
+            if (a <= ns) {
+                const double u = quad_from<L>(gx), v = quad_from<L>(gy), w = quad_from<L>(gz);
+                sum = __builtin_fma(P.w[a], l == 0 ? u : l == 1 ? v : w, sum);
+            }
+        });
+    });
+    if (last) quad_nearest(side);
+    return __builtin_fma(-P.mu * W.rm3, pos, sum);
 }
 
 // Stage derivatives of one component: velocities V and accelerations F, in
@@ -376,13 +407,11 @@ __device__ __forceinline__ double quad_quarters(double x, double r1, int k)
 // of the drag against 80 bits over 0.5 to 3 AU, most of it cancellation in the
 // velocity against the gas, is 1.6e-14 rms (before: 1.8e-14).  A call rather
 // than inlined code, whose constants would be held through the loop.
-__device__ __attribute__((noinline)) double quad_drag(const QUAD_LDS QGas *c, double factor, double x, double y, double z,
-                                                      double vx, double vy, double vz)
+__device__ __attribute__((noinline)) double quad_drag(const QUAD_LDS QGas *c, double factor, double base, double over_rc3,
+                                                      double x, double y, double z, double vx, double vy, double vz)
 {
     const int l = threadIdx.x & 3, place = threadIdx.x >> 2;
     const double idx = c->idx[l], R = c->R[place];
-    const double q = SQR(x) + SQR(y);
-    const double base = sqrt(l == 2 ? q + SQR(z) : q);
     const double rc = dpp_mov<0x00>(base), r = dpp_mov<0xAA>(base);
     const double r1 = sqrt(base);
     // as pl() in gasdev.h: the exponents 1 and 1/2 (and here all quarters) without pow
@@ -391,7 +420,7 @@ __device__ __attribute__((noinline)) double quad_drag(const QUAD_LDS QGas *c, do
     else if (idx != 1.0 && idx != 0.5) p = pow(base, idx);
     const double h = c->g.sh_c * dpp_mov<0x00>(p), rho_p = dpp_mov<0x55>(p);
     const double lambda = c->g.mfp_c * dpp_mov<0xAA>(p), eta = c->g.eta_c * dpp_mov<0xFF>(p);
-    const double s = (q > 0.0 ? sqrt(c->mu / (q * rc)) : 0.0) * sqrt(1.0 - 2.0 * eta);
+    const double s = (rc > 0.0 ? sqrt(over_rc3) : 0.0) * sqrt(1.0 - 2.0 * eta);
     const double ux = vx + y * s, uy = vy - x * s, uz = vz;
     const double w = exp(-SQR(z / h));
     const double rho = factor * (c->g.inner_edge < rc ? c->g.rho_c * rho_p * w : c->edge * SQR(SQR(rc)) * w);
@@ -430,7 +459,7 @@ template <int INTEG, int NA, bool GAS>
 __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, double *columns, QGas *gas)
 {
     constexpr int kWaves = GAS ? 4 * kQuadGasBodies / kWave : kQuadWaves;
-    __shared__ __attribute__((aligned(16))) double records[GAS ? 2 : kQuadWaves][4 * NA][4];
+    __shared__ __attribute__((aligned(16))) double records[GAS ? 2 : kQuadWaves][4 * NA][GAS ? 8 : 4];
     __shared__ double sh_max[2][kWaves], sh_val;
     __shared__ int sh_any[2][kWaves], sh_ev, sh_ok;
     constexpr int nst = q_stages<INTEG>();
@@ -448,9 +477,9 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
     if (!valid) i = 1;         // the first source once more; nothing of it is kept
     const bool keeps = valid && (quad >= ns || unit == 0);
     const int src = quad < ns && l < 3 ? 1 + quad : 0;
-    double (*tab)[4] = records[GAS ? 0 : wave];
+    double (*tab)[GAS ? 8 : 4] = records[GAS ? 0 : wave];
     if (GAS) {
-        if (tid < 2 * 4 * NA * 4) (&records[0][0][0])[tid] = 0.0;
+        for (int k = tid; k < 2 * 4 * NA * 8; k += (int)blockDim.x) (&records[0][0][0])[k] = 0.0;
         __syncthreads();
     } else {
         tab[quad < 4 * NA ? quad : 0][l] = 0.0;     // 16 quads, at most 12 records
@@ -461,13 +490,12 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
         const int end = i < S.nm ? S.end_a : S.end_b;
         P.mu = kGauss2 * (A.mass[0] + A.mass[i]);
 #pragma unroll
-        for (int a = 0; a < (GAS ? 0 : 4 * NA); ++a) P.w[a] = a >= 1 && a <= ns && a < end && a != i ? A.gm[a] : 0.0;
+        for (int a = 0; a < 4 * NA; ++a) P.w[a] = a >= 1 && a <= ns && a < end && a != i ? A.gm[a] : 0.0;
 #pragma unroll
         for (int t = 0; t < NA; ++t) {
             const int a = l + 4 * t;
             P.slot[t] = a <= ns ? a : 0;
             P.near[t] = a >= 1 && a <= ns && a < end && a != i;
-            if (GAS) P.w[t] = a == 0 ? P.mu : P.near[t] ? A.gm[a] : 0.0;
         }
     }
     QBody<GAS> B;
@@ -532,15 +560,19 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
         return l == 0 ? o[0] : l == 1 ? o[1] : o[2];
     };
     // Acceleration at (pos, vel) with the gas's factor and the migration m.
-    auto accelerate = [&](double pos, double vel, double factor, double m, QSide &sd) -> double {
-        double f = quad_force_gas<NA>(P, tab, src, l, pos, sd);
-        tab = tab == records[0] ? records[1] : records[0];
-        if (drags) {
-            drag = quad_drag((const QUAD_LDS QGas *)gas, factor, dpp_mov<0x00>(pos), dpp_mov<0x55>(pos), dpp_mov<0xAA>(pos),
-                             dpp_mov<0x00>(vel), dpp_mov<0x55>(vel), dpp_mov<0xAA>(vel));
-            f += drag;
+    // first: a step's first evaluation (as in quad_force), last: its last.
+    auto accelerate = [&](auto first, bool last, double pos, double vel, double factor, double m, QSide &sd) -> double {
+        if constexpr (GAS) {
+            const QGasPlace W = quad_publish<decltype(first)::value>(tab, src, l, pos, gas->mu);
+            if (drags)
+                drag = quad_drag((const QUAD_LDS QGas *)gas, factor, W.base, W.over_rc3, W.x, W.y, W.z,
+                                 dpp_mov<0x00>(vel), dpp_mov<0x55>(vel), dpp_mov<0xAA>(vel));
+            __syncthreads();
+            const double f = quad_force_gas<NA>(P, tab, ns, l, pos, W, last, sd);
+            tab = tab == records[0] ? records[1] : records[0];
+            return (drags ? f + drag : f) + m;
         }
-        return f + m;
+        return 0.0;
     };
 
     // f0 of the next step: the acceleration at (p, v)
@@ -557,7 +589,7 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
             if (again) {
                 mt_next = mt;
                 mig_next = migration(t0, B.p, B.v, mt_next, fresh_next);
-                f0 = accelerate(B.p, B.v, reduction_factor(A.gas, t0), mig_next, none);
+                f0 = accelerate(std::true_type(), false, B.p, B.v, reduction_factor(A.gas, t0), mig_next, none);
                 again = false;
             }
             mig = mig_next;
@@ -585,7 +617,7 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
                         static_for<1, nst + 1>([&](auto T) {
                             if (q == T) ts = t0 + (INTEG == INTEG_RK4 ? tab::kRk4C[T < 4 ? T : 0] : tab::kDpC[T < 9 ? T : 0]) * h;
                         });
-                    const double f = accelerate(pos, vel, reduction_factor(A.gas, ts), mig, side);
+                    const double f = accelerate(std::false_type(), q == nst, pos, vel, reduction_factor(A.gas, ts), mig, side);
                     B.d.put(q, vel, f);
                 }
                 last_drag = drag;
@@ -604,7 +636,7 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
                     const double tn = t0 + h;
                     mt_next = mt;
                     mig_next = migration(tn, pos, vel, mt_next, fresh_next);
-                    f0 = accelerate(pos, vel, reduction_factor(A.gas, tn), mig_next, none);
+                    f0 = accelerate(std::true_type(), false, pos, vel, reduction_factor(A.gas, tn), mig_next, none);
                     drag = last_drag;
                 } else {
                     f0 = quad_force<NA, false, true>(P, tab, ns, src, l, pos, none);

@@ -108,3 +108,21 @@ def test_split_run_is_the_same():
     assert ta.time == tb.time
     for which in (runtime.Y0, runtime.Y, runtime.ACCEL):
         assert np.array_equal(a.get_array(which), b.get_array(which))
+
+
+@pytest.mark.parametrize("n_pl,planets", [(128, 1), (178, 4), (500, 8), (9600, 4)])
+@pytest.mark.parametrize("integrator", [RKF78, RK4, DP])
+def test_same_bits_as_slices_in_a_thin_nebula(n_pl, planets, integrator):
+    """A drag too weak to change any sum leaves the pulls, with the slices' bits."""
+    scn = S.make_c2(n_pl=n_pl, n_proto=planets)
+    scn.gas = copy.deepcopy(scn.gas)
+    scn.gas.update(density=(1e-60, -2.75))
+    out = []
+    for env in ({}, dict(SOLARIS_AMD_GRID_BLOCK="128")):
+        ctx = make_ctx(scn, **env)
+        tl = _abi.timeline(0.0, 0.25, 1e12)
+        r, st = ctx.integrate(integrator, 1e-10, tl, max_steps=12)
+        assert r == 0 and st.path == _abi.PATH_GRID
+        out.append([ctx.get_array(w) for w in (runtime.Y0, runtime.Y, runtime.ACCEL)] + [*ctx.side_outputs()[:3], tl.hNext])
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
