@@ -707,8 +707,8 @@ bool use_mesh(sol_context *c, int ik, int *share_out = nullptr, int *groups_out 
 // test particles, us per RKF78 attempt in one workgroup or in slices, and in
 // quads: 4 bodies 15 and 7.0, 128 15 and 6.6, 515 17.7 and 6.9, 5,001 18.8 and
 // 7.4, 14,338 20.4 and 8.1.  With live gas: the grid form's slices of 64 and
-// 128 places, us per RKF78 attempt: 125 bodies 64 (one workgroup) and 34, 505
-// 51 and 34, 16,389 56 and 41.
+// 128 places, us per RKF78 attempt: 125 bodies 64 (one workgroup) and 33, 505
+// 51 and 33, 16,389 56 and 39.
 struct QuadShape { int sources, own, groups, places; };   // places: bodies of a workgroup with gas (0: no gas)
 
 bool use_quad(sol_context *c, int ik, QuadShape *out = nullptr)

@@ -27,8 +27,8 @@
 // and after, us: RKF78 of 4 bodies 15.2 and 7.0, 515 17.7 and 6.9, 5,001 18.8
 // and 7.4, 14,338 20.4 and 8.1; Dormand-Prince of 515 13.7 and 5.7; RK4 of 515
 // 4.4 and 1.5.  An evaluation of about 120 instructions takes 0.38 us, the
-// exchange 1.9 us.  With gas, RKF78 of 125 bodies 63.7 and 34.3, 505 50.6 and
-// 34.3, 16,389 55.9 and 41.3.
+// exchange 1.9 us.  With gas, RKF78 of 125 bodies 63.7 and 32.6, 505 51.3 and
+// 33.3, 16,389 55.9 and 39.
 #include <float.h>
 
 #include <algorithm>
@@ -184,10 +184,9 @@ __device__ __forceinline__ double quad_force(const QPulls<NA> &P, double (*tab)[
 //
 // The operations are those of quad_force, so what differs from resident.hip is
 // the drag's last bits alone, which rarely reach an acceleration some 1e7 times
-// as large.  (A root of each record's own and sums over the lanes take 39.8
-// instead of 41.3 us per RKF78 attempt of 16,389 bodies, but round otherwise,
-// and over 100 days a planetesimal's encounters grow that to 1e-8; with
-// quad_force itself 44.)
+// as large.  (Weights in the lanes and sums over the quad took 39.8 us per RKF78
+// attempt of 16,389 bodies, this 38.5, and rounded otherwise: over 100 days a
+// planetesimal's encounters grew that to 1e-8.)
 struct QGasPlace {
     double x, y, z, base, rm3, over_rc3;
 };
@@ -374,13 +373,13 @@ __device__ __forceinline__ double quad_final(QBody<LDS> &B, double h, double &po
 
 // ---- gas -------------------------------------------------------------------
 
-// What the drag reads, in LDS: the nebula, derived constants (mu = k^2 m0; edge
-// = rho_c inner_edge^(rho_i - 4); thermal: the factor of sqrt(r) in the mean
+// What the drag reads, in LDS: the nebula, derived constants (edge =
+// rho_c inner_edge^(rho_i - 4); thermal: the factor of sqrt(r) in the mean
 // thermal speed), the exponent each lane of a quad takes, and the parameters
 // of the bodies.
 struct QGas {
     GasDev g;
-    double mu, edge, thermal, idx[4];
+    double edge, thermal, idx[4];
     int32_t quarters[4], by_quarters;      // 4 idx, where all four are whole and at most 16
     double R[kQuadGasBodies], rho_b[kQuadGasBodies], cd[kQuadGasBodies], gs[kQuadGasBodies], ge[kQuadGasBodies];
 };
@@ -527,7 +526,6 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
             const double cvth = sqrt((8.0 * kb) / (3.14159265358979323846 * g.mmw * mp));
             const double ctp = kGauss2 * (1.0 / (kb / mp));
             gas->g = g;
-            gas->mu = kGauss2 * m0;
             gas->edge = g.rho_c * pow(g.inner_edge, g.rho_i - 4.0);
             gas->thermal = cvth * sqrt(SQR(g.sh_c) * g.mmw * ctp * pow(m0, 2.0 * g.sh_i - 3.0));
             gas->idx[0] = g.sh_i; gas->idx[1] = g.rho_i; gas->idx[2] = g.mfp_i; gas->idx[3] = g.eta_i;
@@ -563,12 +561,18 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
     // first: a step's first evaluation (as in quad_force), last: its last.
     auto accelerate = [&](auto first, bool last, double pos, double vel, double factor, double m, QSide &sd) -> double {
         if constexpr (GAS) {
-            const QGasPlace W = quad_publish<decltype(first)::value>(tab, src, l, pos, gas->mu);
-            if (drags)
-                drag = quad_drag((const QUAD_LDS QGas *)gas, factor, W.base, W.over_rc3, W.x, W.y, W.z,
-                                 dpp_mov<0x00>(vel), dpp_mov<0x55>(vel), dpp_mov<0xAA>(vel));
+            const QGasPlace W = quad_publish<decltype(first)::value>(tab, src, l, pos, kGauss2 * m0);
+            auto resist = [&] {
+                if (drags)
+                    drag = quad_drag((const QUAD_LDS QGas *)gas, factor, W.base, W.over_rc3, W.x, W.y, W.z,
+                                     dpp_mov<0x00>(vel), dpp_mov<0x55>(vel), dpp_mov<0xAA>(vel));
+            };
+            // the drag before the barrier hides its wait (505 bodies, us per attempt: Dormand-Prince 24.7 and
+            // 23.7, RK4 11.7 and 11.0); in RKF78 its call would hold too much (16,389 bodies 38.5 and 41.1)
+            if constexpr (INTEG != INTEG_RKF78) resist();
             __syncthreads();
             const double f = quad_force_gas<NA>(P, tab, ns, l, pos, W, last, sd);
+            if constexpr (INTEG == INTEG_RKF78) resist();
             tab = tab == records[0] ? records[1] : records[0];
             return (drags ? f + drag : f) + m;
         }
