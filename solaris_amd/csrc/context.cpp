@@ -1230,9 +1230,10 @@ int sol_create(sol_context **out, const sol_nbodies *nb, int32_t barycentric, in
     }
     if (const char *e = std::getenv("SOLARIS_AMD_NO_SYM")) c->sym_disabled = e[0] == '1';
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess) {
+        (c->n >= kBesideMinBodies &&
+         (hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking) != hipSuccess ||
+          hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
+          hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess))) {
         c->err = "hipStreamCreate failed";
         return bail(SOL_ERR_DEVICE);
     }
