@@ -37,13 +37,13 @@
 #include "gasdev.h"
 #include "lane_pairs.h"
 #include "quad.h"
+#include "quad_stages.h"
 #include "static_for.h"
 #include "tableaux.h"
 
 namespace sol {
 namespace {
 
-#define QUAD_LDS __attribute__((address_space(3)))
 #define QUAD_SCOPE __HIP_MEMORY_SCOPE_SYSTEM
 
 constexpr int kQuadWaves = kQuadThreads / kWave;
@@ -51,6 +51,9 @@ constexpr int kQuads = kWave / 4;
 
 template <int INTEG>
 constexpr int q_stages() { return INTEG == INTEG_RKF78 ? 12 : INTEG == INTEG_RK4 ? 3 : 8; }
+// rows of stage derivatives: the step's first evaluation and its stages
+template <int INTEG>
+constexpr int q_rows() { return q_stages<INTEG>() + 1; }
 
 // A call rather than inlined code: its registers would be held through the stages.
 __device__ __attribute__((noinline)) double quad_pow(double x, double y) { return pow(x, y); }
@@ -241,34 +244,12 @@ __device__ __forceinline__ double quad_force_gas(const QPulls<NA> &P, double (*t
     return __builtin_fma(-P.mu * W.rm3, pos, sum);
 }
 
-// Stage derivatives of one component: velocities V and accelerations F, in
-// registers, or (LDS) in columns of the workgroup's LDS, column = thread.
-template <bool LDS>
-struct QStages {
-    double V_[13], F_[13];
-    __device__ __forceinline__ double V(int l) const { return V_[l]; }
-    __device__ __forceinline__ double F(int l) const { return F_[l]; }
-    __device__ __forceinline__ void put(int l, double v, double f) { V_[l] = v; F_[l] = f; }
-};
-template <>
-struct QStages<true> {
-    QUAD_LDS double *col;      // this thread's column
-    int stride;                // threads
-    __device__ __forceinline__ double V(int l) const { return col[2 * l * stride]; }
-    __device__ __forceinline__ double F(int l) const { return col[(2 * l + 1) * stride]; }
-    __device__ __forceinline__ void put(int l, double v, double f)
-    {
-        col[2 * l * stride] = v;
-        col[(2 * l + 1) * stride] = f;
-    }
-};
-
 // One component of a body: state, previous state, stage derivatives, scale
 // and error.
-template <bool LDS>
+template <int INTEG, bool LDS>
 struct QBody {
     double p, v, po, vo;
-    QStages<LDS> d;
+    QStages<q_rows<INTEG>(), LDS> d;
     double sp, sv, ep, ev;
 };
 
@@ -314,7 +295,7 @@ __device__ __forceinline__ double quad_sum(Get f)
 
 // State of stage S, as resident.hip's stage_state.
 template <int INTEG, int S, bool LDS>
-__device__ __forceinline__ void quad_stage(const QBody<LDS> &B, double h, double &pos, double &vel)
+__device__ __forceinline__ void quad_stage(const QBody<INTEG, LDS> &B, double h, double &pos, double &vel)
 {
     const double av = quad_sum<INTEG, S>([&](int l) { return B.d.F(l); });
     if constexpr (INTEG == INTEG_DP)
@@ -327,7 +308,7 @@ __device__ __forceinline__ void quad_stage(const QBody<LDS> &B, double h, double
 // Final state and error estimate (kept in B); returns this lane's part of the
 // error maximum.
 template <int INTEG, bool LDS>
-__device__ __forceinline__ double quad_final(QBody<LDS> &B, double h, double &pos, double &vel)
+__device__ __forceinline__ double quad_final(QBody<INTEG, LDS> &B, double h, double &pos, double &vel)
 {
     auto V = [&](int l) { return B.d.V(l); };
     auto F = [&](int l) { return B.d.F(l); };
@@ -497,12 +478,12 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
             P.near[t] = a >= 1 && a <= ns && a < end && a != i;
         }
     }
-    QBody<GAS> B;
+    QBody<INTEG, GAS> B;
     if constexpr (GAS) { B.d.col = (QUAD_LDS double *)columns + tid; B.d.stride = (int)blockDim.x; }
     B.p = B.po = A.y0_in[comp * A.tot + i];
     B.v = B.vo = A.y0_in[(3 + comp) * A.tot + i];
     B.sp = B.sv = B.ep = B.ev = 0.0;
-    static_for<0, 13>([&](auto L) { B.d.put(L, 0.0, 0.0); });
+    B.d.clear();
     QSide side{0.0, 0.0, 0}, none;
     const bool events = S.clip && (S.stop_mask & SOL_STOP_EVENT) && (S.e3 > 0.0 || S.h3 > 0.0 || S.coll > 0.0);
     const bool combine = INTEG != INTEG_RK4 || events;
@@ -900,12 +881,11 @@ const void *quad_kernel(int integ, int sources, bool gas)
                                 : (gas ? quad_gas_kernel_of<INTEG_DP>(sources) : quad_kernel_of<INTEG_DP>(sources));
 }
 
-template <int INTEG>
-size_t column_bytes_of(int places) { return (size_t)(2 * (q_stages<INTEG>() + 1)) * 4 * places * sizeof(double); }
 size_t column_bytes(int integ, int places)
 {
-    return integ == INTEG_RKF78 ? column_bytes_of<INTEG_RKF78>(places)
-         : integ == INTEG_RK4   ? column_bytes_of<INTEG_RK4>(places) : column_bytes_of<INTEG_DP>(places);
+    const int rows = integ == INTEG_RKF78 ? q_rows<INTEG_RKF78>()
+                   : integ == INTEG_RK4   ? q_rows<INTEG_RK4>() : q_rows<INTEG_DP>();
+    return quad_column_bytes(rows, 4 * places);
 }
 
 }  // namespace
