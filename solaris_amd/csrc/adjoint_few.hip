@@ -43,6 +43,19 @@ __device__ __forceinline__ double few_rsqrt(double r2)
     return __builtin_fma(y, e * __builtin_fma(0.375, e, 0.5), y);
 }
 
+// r2^(-3/2) for the forward pass: the hardware's reciprocal square root cubed,
+// corrected once, as the pair sums form it (resident.hip).  Errors over r2 of
+// 1e-2 to 1e2 in units of 2^-53, rms and largest: 0.64 and 2.4, where 1 / (r2
+// sqrt(r2)) has 0.74 and 2.4 and the cube of few_rsqrt 1.55 and 5.4.
+__device__ __forceinline__ double few_rm3(double r2)
+{
+    const double y = __builtin_amdgcn_rsq(r2);
+    const double t = y * y;
+    const double e = __builtin_fma(-r2, t, 1.0);
+    const double y3 = t * y;
+    return __builtin_fma(y3, e * __builtin_fma(1.875, e, 1.5), y3);
+}
+
 // This thread's body and its share of the sources.
 struct Few {
     int i, sub, end;        // body; lane among its eight; its sources are [1, end)
@@ -83,15 +96,13 @@ __device__ __forceinline__ void few_accel(const Few &f, int src, const few_rec *
             const double dx = r.x - p[0], dy = r.y - p[1], dz = r.z - p[2];
             double r2 = dx * dx + dy * dy + dz * dz;
             if (j == f.i || j >= f.end) r2 = 1.0;
-            const double v = few_rsqrt(r2);
-            const double w = v * v * v;
+            const double w = few_rm3(r2);
             t[0] += f.gj[q] * (dx * w - r.x * r.w);
             t[1] += f.gj[q] * (dy * w - r.y * r.w);
             t[2] += f.gj[q] * (dz * w - r.z * r.w);
         }
     }
-    const double v = few_rsqrt(p[0] * p[0] + p[1] * p[1] + p[2] * p[2]);
-    const double c = -f.mu * (v * v * v);
+    const double c = -f.mu * few_rm3(p[0] * p[0] + p[1] * p[1] + p[2] * p[2]);
     sum8(t);
 #pragma unroll
     for (int k = 0; k < 3; ++k) a[k] = c * p[k] + t[k];
@@ -156,8 +167,7 @@ __global__ __launch_bounds__(256) void k_few_forward(FewArgs a)
                 // form it beside their distances, the chain is 15% slower (it
                 // is bound by the instructions of one wave)
                 if (mine) {
-                    const double r = few_rsqrt(p[0] * p[0] + p[1] * p[1] + p[2] * p[2]);
-                    const few_rec rec = {p[0], p[1], p[2], r * r * r};
+                    const few_rec rec = {p[0], p[1], p[2], few_rm3(p[0] * p[0] + p[1] * p[1] + p[2] * p[2])};
                     s[q][f.i] = rec;
                     reinterpret_cast<few_rec *>(a.sp_out)[((size_t)(step - n0) * 4 + q) * a.src + f.i] = rec;
                 }
