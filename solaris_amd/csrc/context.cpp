@@ -695,7 +695,9 @@ bool use_mesh(sol_context *c, int ik, int *share_out = nullptr, int *groups_out 
     const int share = mesh_share(c->n, c->n_massive, ea, eb, c->cu_count);
     if (share == 0 || share > kMeshContextShare) return false;
     const int groups = mesh_groups(c->n, c->n_massive, ea, eb, share);
-    if (mesh_capacity(ik, c->n, share, c->cu_count) < groups) return false;
+    int &cap = c->mesh_caps[ik][share / 8];
+    if (cap < 0) cap = mesh_capacity(ik, c->n, share, c->cu_count);
+    if (cap < groups) return false;
     if (share_out) *share_out = share;
     if (groups_out) *groups_out = groups;
     return true;
@@ -724,11 +726,16 @@ bool use_quad(sol_context *c, int ik, QuadShape *out = nullptr)
             m.nslices > std::min(c->cu_count, kQuadMaxGroups))
             return false;
         q.own = m.per; q.groups = m.nslices; q.places = m.stride;
-        if (quad_gas_capacity(ik, q.sources, q.places, c->cu_count) < q.groups) return false;
+        int &cap = c->quad_gas_caps[ik][q.sources / 4][q.places / kQuadGasBodies];
+        if (cap < 0) cap = quad_gas_capacity(ik, q.sources, q.places, c->cu_count);
+        if (cap < q.groups) return false;
     } else {
         q.own = 16 - q.sources;
         q.groups = quad_groups(c->n, q.sources, c->cu_count);
-        if (q.groups == 0 || quad_capacity(ik, q.sources, c->cu_count) < q.groups) return false;
+        if (q.groups == 0) return false;
+        int &cap = c->quad_caps[ik][q.sources / 4];
+        if (cap < 0) cap = quad_capacity(ik, q.sources, c->cu_count);
+        if (cap < q.groups) return false;
     }
     if (out) *out = q;
     return true;
@@ -880,39 +887,27 @@ int resident_run(sol_context *c, int ik, double eps, sol_timeline *tl, int64_t m
 }
 
 // Arrays and exchange words of the mesh and the quad form.
-int mesh_buffers(sol_context *c)
+int mesh_buffers(sol_context *c, bool gas)
 {
     sol_context::Mesh &m = c->mesh;
-    if (m.pos) return SOL_OK;
     const size_t np = c->np;
-    unsigned char *sys = nullptr;
-    int r;
-    if ((r = dalloc(c, &m.y0, 6 * np)) || (r = dalloc(c, &m.y, 6 * np)) || (r = dalloc(c, &m.acc0, 6 * np)) ||
-        (r = dalloc(c, &m.yscale, 6 * np)) || (r = dalloc(c, &m.error, 6 * np)) || (r = dalloc(c, &m.rm3, np)) ||
-        (r = dalloc(c, &m.nnd, np)) || (r = dalloc(c, &m.nni, np)) || (r = dalloc(c, &m.part, 1)) ||
-        (r = dalloc(c, &m.sys_in, 1)) ||
-        (r = dalloc(c, &m.part_of, (size_t)kMeshMaxGroups)) ||
-        (r = dalloc(c, &sys, sizeof(ResSystem) + std::max(sizeof(MeshSync), sizeof(QuadSync)))))
-        return r;
-    m.sys = reinterpret_cast<ResSystem *>(sys);
-    m.sync = sys + sizeof(ResSystem);
-    if (!c->mesh_h && hipHostMalloc((void **)&c->mesh_h, sizeof(ResSystem) + 8 + sizeof(MeshPart), hipHostMallocDefault) != hipSuccess) {
-        c->mesh_h = nullptr;
-        return c->fail(SOL_ERR_DEVICE, "hipHostMalloc failed");
+    if (!m.pos) {
+        ArrayBlock b;
+        b.add(&m.y0, 6 * np); b.add(&m.y, 6 * np); b.add(&m.acc0, 6 * np);
+        b.add(&m.yscale, 6 * np); b.add(&m.error, 6 * np);
+        b.add(&m.rm3, np); b.add(&m.nnd, np); b.add(&m.nni, np);
+        b.add(&m.run, 1); b.add(&m.part_of, (size_t)kMeshMaxGroups);
+        b.add(&m.pos, 6 * np);
+        if (int r = b.make(c)) return r;
     }
-    return dalloc(c, &m.pos, 6 * np);
-}
-
-int mesh_gas_buffers(sol_context *c)
-{
-    sol_context::Mesh &m = c->mesh;
-    if (m.dragc) return SOL_OK;
-    const size_t np = c->np;
-    int r;
-    if ((r = dalloc(c, &m.migt, np)) || (r = dalloc(c, &m.migc, 3 * np)) || (r = dalloc(c, &m.migt_prev, np)) ||
-        (r = dalloc(c, &m.migc_prev, 3 * np)))
-        return r;
-    return dalloc(c, &m.dragc, 3 * np);
+    if (gas && !m.dragc) {
+        ArrayBlock b;
+        b.add(&m.migt, np); b.add(&m.migc, 3 * np);
+        b.add(&m.migt_prev, np); b.add(&m.migc_prev, 3 * np);
+        b.add(&m.dragc, 3 * np);
+        if (int r = b.make(c)) return r;
+    }
+    return SOL_OK;
 }
 
 // resident_run on the mesh or the quad form: accepted steps of integrator ik
@@ -926,20 +921,22 @@ int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int
     QuadShape shape{};
     if (quad ? !use_quad(c, ik, &shape) : !use_mesh(c, ik, &share, &groups)) return kGridRetry;
     if (quad) groups = shape.groups;
-    int r = mesh_buffers(c);
-    if (r) return r;
+    if (int r = mesh_buffers(c, shape.places != 0)) return r;
     sol_context::Mesh &m = c->mesh;
-    ResSystem &S = *reinterpret_cast<ResSystem *>(c->mesh_h);
-    uint32_t &lost = *reinterpret_cast<uint32_t *>(c->mesh_h + sizeof(ResSystem));
+    MeshRun &to = c->mesh_h[0], &back = c->mesh_h[1];
+    ResSystem &S = back.system;
     S = resident_system(c, eps, tl, clip, stop_mask);
-    HIPCHECK(c, hipMemcpyAsync(m.sys, &S, sizeof S, hipMemcpyHostToDevice, c->stream));
-    MeshPart &P = *reinterpret_cast<MeshPart *>(c->mesh_h + sizeof(ResSystem) + 8);
-    P = MeshPart{0, 0, groups, share};
-    HIPCHECK(c, hipMemcpyAsync(m.part, &P, sizeof P, hipMemcpyHostToDevice, c->stream));
+    if (!quad) {
+        // (the words are zero)
+        to.system = S;
+        to.part = MeshPart{0, 0, groups, share};
+        HIPCHECK(c, hipMemcpyAsync(m.run, &to, offsetof(MeshRun, words) + sizeof(MeshSync), hipMemcpyHostToDevice,
+                                   c->stream));
+    }
     MeshArgs A{};
-    A.systems = m.sys;
-    A.parts = m.part; A.part_of = m.part_of;
-    A.sync = reinterpret_cast<MeshSync *>(m.sync);
+    A.systems = &m.run->system;
+    A.parts = &m.run->part; A.part_of = m.part_of;
+    A.sync = &m.run->words.mesh;
     A.pos = m.pos; A.gm = c->gm;
     A.tot = c->np;
     A.mass = c->mass; A.radius = c->radius;
@@ -948,9 +945,8 @@ int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int
     A.eps2 = c->softening * c->softening;
     A.ticks = (uint64_t)(c->grid_wait_s * (double)c->rtc_hz);
     QuadArgs Q{};
-    Q.system_in = m.sys_in;
-    Q.system = m.sys;
-    Q.sync = reinterpret_cast<QuadSync *>(m.sync);
+    Q.system = &m.run->system;
+    Q.sync = &m.run->words.quad;
     Q.sources = shape.sources;
     Q.groups = groups;
     Q.own = shape.own;
@@ -960,7 +956,6 @@ int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int
     Q.rm3 = A.rm3; Q.nnd = A.nnd; Q.nni = A.nni;
     Q.ticks = A.ticks;
     if (shape.places) {
-        if ((r = mesh_gas_buffers(c))) return r;
         Q.gas = c->gasdev;
         Q.density = c->density; Q.cd = c->cd; Q.gs = c->gs; Q.ge = c->ge; Q.stop = c->stop;
         Q.migt_in = c->migt; Q.migc_in = c->migc;
@@ -972,21 +967,22 @@ int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int
     const double per_step = quad ? 5.0e-5 : 13.0 * (5.0e-6 + (double)c->n * (double)c->n * 1.0e-12);
     const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(20000, (int64_t)(0.2 / per_step)));
     A.y0_in = c->y0;
-    for (;;) {
+    for (bool first = true;; first = false) {
         const int64_t k = max_steps > 0 ? std::min(chunk, max_steps - S.steps) : chunk;
         const UnitLease lease(c->device, groups, c->cu_count);
         if (quad) {
             Q.y0_in = A.y0_in;
-            HIPCHECK(c, hipMemcpyAsync(m.sys_in, &S, sizeof S, hipMemcpyHostToDevice, c->stream));
+            Q.system_in = S;
             HIPCHECK(c, shape.places ? launch_quad_gas(c->stream, ik, Q, shape.places, (int)k)
                                      : launch_quad(c->stream, ik, Q, (int)k));
         } else {
-            HIPCHECK(c, launch_mesh(c->stream, ik, A, 1, groups, c->n, share, (int)k));
+            HIPCHECK(c, launch_mesh(c->stream, ik, A, 1, groups, c->n, share, (int)k, first));
         }
-        HIPCHECK(c, hipMemcpyAsync(c->mesh_h, m.sys, sizeof(ResSystem) + sizeof(uint32_t), hipMemcpyDeviceToHost,
-                                   c->stream));
+        HIPCHECK(c, hipMemcpyAsync(&back, m.run, kMeshRunBack, hipMemcpyDeviceToHost, c->stream));
         HIPCHECK(c, hipStreamSynchronize(c->stream));
-        if (lost != 0 || S.status == RES_SYNC_ERROR) {
+        // (without an exchange the quad form leaves its words alone)
+        const bool lost = back.words.mesh.error != 0 && (!quad || quad_exchanges(ik, Q));
+        if (lost || S.status == RES_SYNC_ERROR) {
             // a workgroup that was not resident: as for the grid form, the
             // call runs again from its unchanged start
             if (++c->grid_failures >= 2) c->grid_disabled = true;
@@ -1229,6 +1225,9 @@ int sol_create(sol_context **out, const sol_nbodies *nb, int32_t barycentric, in
             c->rtc_hz = (uint64_t)khz * 1000;
     }
     if (const char *e = std::getenv("SOLARIS_AMD_NO_SYM")) c->sym_disabled = e[0] == '1';
+    std::fill_n(&c->mesh_caps[0][0], 3 * 4, -1);
+    std::fill_n(&c->quad_caps[0][0], 3 * 3, -1);
+    std::fill_n(&c->quad_gas_caps[0][0][0], 3 * 3 * 2, -1);
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         (c->n >= kBesideMinBodies &&
          (hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking) != hipSuccess ||
@@ -1251,17 +1250,21 @@ int sol_create(sol_context **out, const sol_nbodies *nb, int32_t barycentric, in
         (r = dalloc(c, &c->errblk, c->nblk)) || (r = dalloc(c, &c->scal, 8)) || (r = dalloc(c, &c->coef, 275)) ||
         (r = dalloc(c, &c->integ, 11 * np)) || (r = dalloc(c, &c->res_d, 1)))
         return bail(r);
-    if (hipHostMalloc((void **)&c->h_scal, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void **)&c->res_h, sizeof(ResSystem), hipHostMallocDefault) != hipSuccess) {
-        c->err = "hipHostMalloc failed";
-        return bail(SOL_ERR_DEVICE);
-    }
-    if (c->n <= 2 * kIoBodies) {
-        c->io_bytes = 6 * sizeof(double) * (size_t)std::min(c->n, kIoBodies);
-        if (hipHostMalloc((void **)&c->io_h, c->io_bytes, hipHostMallocDefault) != hipSuccess) {
+    // pinned, in one allocation (each took 15 us)
+    {
+        if (c->n <= 2 * kIoBodies) c->io_bytes = 6 * sizeof(double) * (size_t)std::min(c->n, kIoBodies);
+        const size_t runs = 2 * sizeof(MeshRun), scal = 8 * sizeof(double);
+        const size_t res = (sizeof(ResSystem) + 127) / 128 * 128;
+        if (hipHostMalloc((void **)&c->pinned, runs + res + scal + c->io_bytes, hipHostMallocDefault) != hipSuccess) {
+            c->pinned = nullptr;
             c->err = "hipHostMalloc failed";
             return bail(SOL_ERR_DEVICE);
         }
+        std::memset(c->pinned, 0, runs + res + scal);
+        c->mesh_h = reinterpret_cast<MeshRun *>(c->pinned);
+        c->res_h = reinterpret_cast<ResSystem *>(c->pinned + runs);
+        c->h_scal = reinterpret_cast<double *>(c->pinned + runs + res);
+        if (c->io_bytes) c->io_h = reinterpret_cast<double *>(c->pinned + runs + res + scal);
     }
     // the copies below are made on the default stream
     if (hipStreamSynchronize(c->stream) != hipSuccess) {
@@ -1305,11 +1308,8 @@ int sol_destroy(sol_context *c)
         for (void *q : gp)
             if (q) (void)hipFree(q);
     }
-    if (c->h_scal) (void)hipHostFree(c->h_scal);
-    if (c->res_h) (void)hipHostFree(c->res_h);
+    if (c->pinned) (void)hipHostFree(c->pinned);
     if (c->integ_h) (void)hipHostFree(c->integ_h);
-    if (c->io_h) (void)hipHostFree(c->io_h);
-    if (c->mesh_h) (void)hipHostFree(c->mesh_h);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
     if (c->ev_join) (void)hipEventDestroy(c->ev_join);

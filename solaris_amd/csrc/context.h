@@ -5,7 +5,9 @@
 
 #include <algorithm>
 #include <cstdarg>
+#include <cstddef>
 #include <cstdio>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -14,7 +16,20 @@
 #include "mesh.h"
 #include "quad.h"
 
-namespace sol { struct AdjointState; }
+namespace sol {
+struct AdjointState;
+
+// What a run of the mesh form reads first, in one copy, and what comes back
+// of it and of the quad form: the descriptor up to the exchange's error word
+// (the first of either form's words: a wait gave up).
+struct MeshRun {
+    ResSystem system;
+    MeshPart part;
+    union Words { MeshSync mesh; QuadSync quad; };
+    alignas(128) Words words;
+};
+constexpr size_t kMeshRunBack = offsetof(MeshRun, words) + sizeof(uint32_t);
+}  // namespace sol
 
 struct sol_context {
     int device = 0;
@@ -54,6 +69,7 @@ struct sol_context {
     int32_t *nni = nullptr;
     double *migc = nullptr, *dragc = nullptr;
     double *errblk = nullptr, *scal = nullptr, *coef = nullptr, *integ = nullptr;
+    unsigned char *pinned = nullptr;   // one allocation: mesh_h, res_h, h_scal, io_h
     double *h_scal = nullptr;   // pinned: [0] h, [1] t, [2] error max
     double *integ_h = nullptr;  // pinned, 12 * np: the integrals' rows and the masses (made on first use)
     // pinned: the arrays of a call, which the kernels read and write in place
@@ -95,13 +111,13 @@ struct sol_context {
         // with gas: migration and drag (prev: as the run's last launch left them)
         int32_t *migt = nullptr, *migt_prev = nullptr;
         double *migc = nullptr, *migc_prev = nullptr, *dragc = nullptr;
-        sol::ResSystem *sys = nullptr;       // followed by the MeshSync or QuadSync
-        sol::ResSystem *sys_in = nullptr;    // the quad form's copy to read
-        unsigned char *sync = nullptr;       // (its first word: a wait gave up)
-        sol::MeshPart *part = nullptr;
+        sol::MeshRun *run = nullptr;
         int32_t *part_of = nullptr;
     } mesh;
-    unsigned char *mesh_h = nullptr;         // pinned: ResSystem and the error word
+    sol::MeshRun *mesh_h = nullptr;          // pinned: a run's words to the device ([0]) and back ([1])
+    // workgroups the device holds (-1: not asked yet): mesh form by integrator
+    // and share, quad form by integrator and pulls per lane, with gas also places
+    int mesh_caps[3][4], quad_caps[3][3], quad_gas_caps[3][3][2];
     // profiling (sol_profile)
     bool profiling = false;
     std::vector<hipEvent_t> ev_pool;
@@ -161,6 +177,34 @@ int dalloc(sol_context *c, T **p, size_t count)
     *p = static_cast<T *>(q);
     return SOL_OK;
 }
+
+// Arrays of a context in one allocation, zeroed by one fill: each of its own
+// took 15 us (30 arrays of 515 bodies: context 600 us, in one 250).
+class ArrayBlock {
+public:
+    template <typename T>
+    void add(T **p, size_t count)
+    {
+        items_.push_back({p, bytes_});
+        bytes_ += (std::max<size_t>(count, 1) * sizeof(T) + 255) / 256 * 256;
+    }
+    // Leaves the pointers alone when it fails.
+    int make(sol_context *c)
+    {
+        unsigned char *q = nullptr;
+        if (int r = dalloc(c, &q, bytes_)) return r;
+        for (const Item &i : items_) {
+            void *at = q + i.at;
+            std::memcpy(i.p, &at, sizeof at);
+        }
+        return SOL_OK;
+    }
+
+private:
+    struct Item { void *p; size_t at; };       // the pointer's place
+    std::vector<Item> items_;
+    size_t bytes_ = 0;
+};
 
 // Source range ends of the two astrocentric sink classes.
 void source_ends(const sol_context *c, int &ea, int &eb);

@@ -53,11 +53,12 @@ struct MeshArgs {
 int mesh_share(int n, int nm, int end_a, int end_b, int cus);
 int mesh_groups(int n, int nm, int end_a, int end_b, int share);
 
-// Zeroes the parts' exchange words and runs max_steps accepted steps of
-// integrator `integ` for every part.  The grid is the sum of the parts'
-// groups and has to be resident at once.
+// Zeroes the parts' exchange words (unless they are `zeroed`) and runs
+// max_steps accepted steps of integrator `integ` for every part.  The grid is
+// the sum of the parts' groups and has to be resident at once; mesh_capacity has
+// to have been asked for this device.
 hipError_t launch_mesh(hipStream_t st, int integ, const MeshArgs &a, int nparts, int ngroups, int max_n,
-                       int max_share, int max_steps);
+                       int max_share, int max_steps, bool zeroed = false);
 // After that launch: the state of every part that ran to its end (no wait
 // timed out) into y0 (component stride tot) and its descriptor into systems.
 // The mesh launch itself may have written some workgroups' rows of a part

@@ -815,10 +815,10 @@ int mesh_capacity(int integ, int n, int share, int cu_count)
 }
 
 hipError_t launch_mesh(hipStream_t st, int integ, const MeshArgs &a, int nparts, int ngroups, int max_n,
-                       int max_share, int max_steps)
+                       int max_share, int max_steps, bool zeroed)
 {
     if (nparts < 1 || ngroups < 1 || max_share < 1 || max_share > kMeshMaxShare) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_mesh_zero, dim3(nparts), dim3(256), 0, st, a.sync);
+    if (!zeroed) hipLaunchKernelGGL(k_mesh_zero, dim3(nparts), dim3(256), 0, st, a.sync);
     MeshArgs args = a;
     int records = 0;
     const size_t lds = mesh_tile_bytes(max_n, &records);

@@ -23,9 +23,9 @@ struct QuadSync {
 };
 
 struct QuadArgs {
-    // read and written at the end, not in place: without an exchange (RK4) a
-    // workgroup may be done before another has started
-    const ResSystem *system_in;
+    // the descriptor, and where it goes at the end.  By value: a copy to the
+    // device of its own cost 3.5 us of a Driver call
+    ResSystem system_in;
     ResSystem *system;
     QuadSync *sync;
     int32_t sources;           // bodies [1, 1 + sources) are integrated by every wave (with gas: workgroup)
@@ -52,8 +52,13 @@ struct QuadArgs {
 // Workgroups for n bodies (0: the system does not fit).
 int quad_groups(int n, int sources, int cus);
 
+// Whether the workgroups of that launch exchange words: several of them, and
+// decisions to combine (RK4 has events only).  Only then are the words zeroed
+// and A.sync->error has a meaning.
+bool quad_exchanges(int integ, const QuadArgs &a);
 // Zeroes the exchange words and runs max_steps accepted steps of integrator
-// `integ`.  The a.groups workgroups have to be resident at once.
+// `integ`.  The a.groups workgroups have to be resident at once, and
+// quad_capacity (quad_gas_capacity) asked for this device before.
 hipError_t launch_quad(hipStream_t st, int integ, const QuadArgs &a, int max_steps);
 // The same with gas: workgroups of `places` bodies (the sources and a.own).
 hipError_t launch_quad_gas(hipStream_t st, int integ, const QuadArgs &a, int places, int max_steps);

@@ -55,6 +55,12 @@ constexpr int q_stages() { return INTEG == INTEG_RKF78 ? 12 : INTEG == INTEG_RK4
 template <int INTEG>
 constexpr int q_rows() { return q_stages<INTEG>() + 1; }
 
+// Whether a run stops at events of the side outputs.
+__host__ __device__ __forceinline__ bool quad_events(const ResSystem &S)
+{
+    return S.clip && (S.stop_mask & SOL_STOP_EVENT) && (S.e3 > 0.0 || S.h3 > 0.0 || S.coll > 0.0);
+}
+
 // A call rather than inlined code: its registers would be held through the stages.
 __device__ __attribute__((noinline)) double quad_pow(double x, double y) { return pow(x, y); }
 
@@ -448,9 +454,7 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
     const int quad = (GAS ? tid : lane) >> 2, l = lane & 3, comp = l < 3 ? l : 2;
     const int ns = A.sources;
     const int unit = GAS ? (int)blockIdx.x : (int)blockIdx.x * kQuadWaves + wave;   // that has the sources once
-    ResSystem S = *A.system_in;
-    if (S.status != RES_RUNNING) return;      // the same in every workgroup
-
+    ResSystem S = A.system_in;
     const int n = S.n;
     int i = quad < ns ? 1 + quad : 1 + ns + unit * A.own + (quad - ns);
     const bool valid = i < n && quad - ns < A.own;
@@ -485,7 +489,7 @@ __device__ __forceinline__ void quad_run(const QuadArgs &A, int max_steps, doubl
     B.sp = B.sv = B.ep = B.ev = 0.0;
     B.d.clear();
     QSide side{0.0, 0.0, 0}, none;
-    const bool events = S.clip && (S.stop_mask & SOL_STOP_EVENT) && (S.e3 > 0.0 || S.h3 > 0.0 || S.coll > 0.0);
+    const bool events = quad_events(S);
     const bool combine = INTEG != INTEG_RK4 || events;
     bool flushed = false;      // small numbers were flushed in this launch
     int x = 0;                 // exchanges
@@ -911,13 +915,19 @@ int quad_capacity(int integ, int sources, int cu_count)
 int quad_gas_capacity(int integ, int sources, int places, int cu_count)
 {
     const void *f = quad_kernel(integ, sources, true);
-    const int lds = (int)column_bytes(integ, places);
     int per_cu = 0;
+    // (the attribute for the most places, so that it holds for every launch)
     if (sources < 1 || sources > kQuadMaxSources || places <= sources || places > kQuadGasBodies ||
-        hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, 4 * places, lds) != hipSuccess)
+        hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)column_bytes(integ, kQuadGasBodies)) !=
+            hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, 4 * places, column_bytes(integ, places)) != hipSuccess)
         return 0;
     return per_cu * cu_count;
+}
+
+bool quad_exchanges(int integ, const QuadArgs &a)
+{
+    return a.groups > 1 && (integ != INTEG_RK4 || quad_events(a.system_in));
 }
 
 hipError_t launch_quad(hipStream_t st, int integ, const QuadArgs &a, int max_steps)
@@ -925,7 +935,8 @@ hipError_t launch_quad(hipStream_t st, int integ, const QuadArgs &a, int max_ste
     if (a.groups < 1 || a.groups > kQuadMaxGroups || a.sources < 1 || a.sources > kQuadMaxSources ||
         a.own != kQuads - a.sources)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_quad_zero, dim3(1), dim3(kQuadMaxGroups), 0, st, a.sync);
+    if (quad_exchanges(integ, a))
+        hipLaunchKernelGGL(k_quad_zero, dim3(1), dim3(kQuadMaxGroups), 0, st, a.sync);
     QuadArgs args = a;
     void *kargs[] = {&args, &max_steps};
     return hipLaunchKernel(quad_kernel(integ, a.sources, false), dim3(a.groups), dim3(kQuadThreads), kargs, 0, st);
@@ -936,14 +947,12 @@ hipError_t launch_quad_gas(hipStream_t st, int integ, const QuadArgs &a, int pla
     if (a.groups < 1 || a.groups > kQuadMaxGroups || a.sources < 1 || a.sources > kQuadMaxSources || a.own < 1 ||
         a.sources + a.own > places || places > kQuadGasBodies || places % kQuads != 0)
         return hipErrorInvalidValue;
-    const void *f = quad_kernel(integ, a.sources, true);
-    const size_t lds = column_bytes(integ, places);
-    hipError_t r = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (r != hipSuccess) return r;
-    hipLaunchKernelGGL(k_quad_zero, dim3(1), dim3(kQuadMaxGroups), 0, st, a.sync);
+    if (quad_exchanges(integ, a))
+        hipLaunchKernelGGL(k_quad_zero, dim3(1), dim3(kQuadMaxGroups), 0, st, a.sync);
     QuadArgs args = a;
     void *kargs[] = {&args, &max_steps};
-    return hipLaunchKernel(f, dim3(a.groups), dim3(4 * places), kargs, lds, st);
+    return hipLaunchKernel(quad_kernel(integ, a.sources, true), dim3(a.groups), dim3(4 * places), kargs,
+                           column_bytes(integ, places), st);
 }
 
 }  // namespace sol
