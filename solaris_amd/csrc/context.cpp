@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "context.h"
+#include "stream_pool.h"
 #include "tableaux.h"
 #include "unit_lease.h"
 
@@ -213,41 +214,51 @@ int ensure_partials(sol_context *c)
         // the nearest-neighbour search that goes with the symmetric sum
         NNGrid &g = c->grid;
         const size_t mc = nn_grid_max_cells(c->n), np = (size_t)c->np;
-        HIPCHECK(c, hipMalloc(&g.params, sizeof(GridParams)));
-        HIPCHECK(c, hipMalloc(&g.bbox, kGridBboxBlocks * 6 * sizeof(double)));
-        HIPCHECK(c, hipMalloc(&g.count, (mc + 1) * sizeof(int32_t)));
-        HIPCHECK(c, hipMalloc(&g.start, (mc + 1) * sizeof(int32_t)));
-        HIPCHECK(c, hipMalloc(&g.cellof, np * sizeof(int32_t)));
-        HIPCHECK(c, hipMalloc(&g.rank, np * sizeof(int32_t)));
-        HIPCHECK(c, hipMalloc(&g.spos, np * sizeof(double4)));
-        HIPCHECK(c, hipMalloc(&g.r2, np * sizeof(double)));
-        HIPCHECK(c, hipMalloc(&g.idx, np * sizeof(int32_t)));
+        ArrayBlock b;
+        b.add(&g.params, 1); b.add(&g.bbox, kGridBboxBlocks * 6);
+        b.add(&g.count, mc + 1); b.add(&g.start, mc + 1);
+        b.add(&g.cellof, np); b.add(&g.rank, np); b.add(&g.spos, np);
+        b.add(&g.r2, np); b.add(&g.idx, np);
+        if (int r = b.make(c)) return r;
         g.max_cells = (int32_t)mc;
+    }
+    if (c->sym.M > 0 && c->n >= kBesideMinBodies && !c->stream2) {
+        // for the search beside the sum (pair_sums)
+        HIPCHECK(c, StreamPool::take(c->device, &c->stream2));
+        HIPCHECK(c, hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
+        HIPCHECK(c, hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
     }
     if (c->sym.M > 0) {
         const size_t na = (size_t)sym_units(c->sym) * 3 * kSymGroup;
         const size_t nb = (size_t)c->sym.nwaves * c->sym.slots_per_wave * 3 * kSymGroup;
-        if (na > c->apart_cap) {
+        if (na > c->apart_cap || nb > c->bpart_cap) {
+            const size_t ca = std::max(na, c->apart_cap), cb = std::max(nb, c->bpart_cap);
             if (c->apart) (void)hipFree(c->apart);
-            c->apart = nullptr; c->apart_cap = 0;
-            HIPCHECK(c, hipMalloc(&c->apart, na * sizeof(double)));
-            c->apart_cap = na;
-        }
-        if (nb > c->bpart_cap) {
-            if (c->bpart) (void)hipFree(c->bpart);
-            c->bpart = nullptr; c->bpart_cap = 0;
-            HIPCHECK(c, hipMalloc(&c->bpart, nb * sizeof(double)));
-            c->bpart_cap = nb;
+            c->apart = c->bpart = nullptr;
+            c->apart_cap = c->bpart_cap = 0;
+            ArrayBlock b;
+            b.add(&c->apart, ca);
+            b.add(&c->bpart, cb);
+            void *q = nullptr;
+            HIPCHECK(c, hipMalloc(&q, b.bytes()));
+            b.place(q);
+            c->apart_cap = ca;
+            c->bpart_cap = cb;
         }
     }
     const size_t need = std::max((size_t)c->plan.nwaves * c->plan.slots_per_wave,
                                  (size_t)c->plan_rest.nwaves * c->plan_rest.slots_per_wave);
     if (need <= c->part_slots) return SOL_OK;
-    if (c->part) { (void)hipFree(c->part); (void)hipFree(c->nnr2); (void)hipFree(c->nnidx); }
+    if (c->part) (void)hipFree(c->part);
     c->part = nullptr; c->nnr2 = nullptr; c->nnidx = nullptr;
-    HIPCHECK(c, hipMalloc(&c->part, need * 3 * kWave * sizeof(double)));
-    HIPCHECK(c, hipMalloc(&c->nnr2, need * kWave * sizeof(double)));
-    HIPCHECK(c, hipMalloc(&c->nnidx, need * kWave * sizeof(int32_t)));
+    c->part_slots = 0;
+    ArrayBlock b;
+    b.add(&c->part, need * 3 * kWave);
+    b.add(&c->nnr2, need * kWave);
+    b.add(&c->nnidx, need * kWave);
+    void *q = nullptr;
+    HIPCHECK(c, hipMalloc(&q, b.bytes()));
+    b.place(q);
     c->part_slots = need;
     return SOL_OK;
 }
@@ -1228,29 +1239,27 @@ int sol_create(sol_context **out, const sol_nbodies *nb, int32_t barycentric, in
     std::fill_n(&c->mesh_caps[0][0], 3 * 4, -1);
     std::fill_n(&c->quad_caps[0][0], 3 * 3, -1);
     std::fill_n(&c->quad_gas_caps[0][0][0], 3 * 3 * 2, -1);
-    if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-        (c->n >= kBesideMinBodies &&
-         (hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking) != hipSuccess ||
-          hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
-          hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess))) {
+    if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
         c->err = "hipStreamCreate failed";
         return bail(SOL_ERR_DEVICE);
     }
     const size_t np = c->np;
-    if ((r = dalloc(c, &c->mass, np)) || (r = dalloc(c, &c->gm, np)) || (r = dalloc(c, &c->radius, np)) ||
-        (r = dalloc(c, &c->density, np)) || (r = dalloc(c, &c->cd, np)) || (r = dalloc(c, &c->gs, np)) ||
-        (r = dalloc(c, &c->ge, np)) || (r = dalloc(c, &c->stop, np)) || (r = dalloc(c, &c->type, np)) ||
-        (r = dalloc(c, &c->migt, np)) || (r = dalloc(c, &c->y0, 6 * np)) || (r = dalloc(c, &c->y, 6 * np)) ||
-        (r = dalloc(c, &c->acc0, 6 * np)) || (r = dalloc(c, &c->yscale, 6 * np)) ||
-        (r = dalloc(c, &c->error, 6 * np)) || (r = dalloc(c, &c->fst, 12 * 6 * np)) ||
-        (r = dalloc(c, &c->cin, 6 * np)) || (r = dalloc(c, &c->aos, 6 * np)) ||
-        (r = dalloc(c, &c->J, np)) || (r = dalloc(c, &c->ind, 2 * (size_t)c->nblk * 6)) ||
-        (r = dalloc(c, &c->rm3, np)) || (r = dalloc(c, &c->nnd, np)) || (r = dalloc(c, &c->nni, np)) ||
-        (r = dalloc(c, &c->migc, 3 * np)) || (r = dalloc(c, &c->dragc, 3 * np)) ||
-        (r = dalloc(c, &c->errblk, c->nblk)) || (r = dalloc(c, &c->scal, 8)) || (r = dalloc(c, &c->coef, 275)) ||
-        (r = dalloc(c, &c->integ, 11 * np)) || (r = dalloc(c, &c->res_d, 1)))
-        return bail(r);
-    // pinned, in one allocation (each took 15 us)
+    {
+        ArrayBlock b;
+        b.add(&c->mass, np); b.add(&c->gm, np); b.add(&c->radius, np); b.add(&c->density, np);
+        b.add(&c->cd, np); b.add(&c->gs, np); b.add(&c->ge, np); b.add(&c->stop, np);
+        b.add(&c->type, np); b.add(&c->migt, np);
+        b.add(&c->y0, 6 * np); b.add(&c->y, 6 * np); b.add(&c->acc0, 6 * np);
+        b.add(&c->yscale, 6 * np); b.add(&c->error, 6 * np); b.add(&c->fst, 12 * 6 * np);
+        b.add(&c->cin, 6 * np); b.add(&c->aos, 6 * np);
+        b.add(&c->J, np); b.add(&c->ind, 2 * (size_t)c->nblk * 6);
+        b.add(&c->rm3, np); b.add(&c->nnd, np); b.add(&c->nni, np);
+        b.add(&c->migc, 3 * np); b.add(&c->dragc, 3 * np);
+        b.add(&c->errblk, (size_t)c->nblk); b.add(&c->scal, 8); b.add(&c->coef, 275);
+        b.add(&c->integ, 11 * np); b.add(&c->res_d, 1);
+        if ((r = b.make(c))) return bail(r);
+    }
+    // pinned, in one allocation
     {
         if (c->n <= 2 * kIoBodies) c->io_bytes = 6 * sizeof(double) * (size_t)std::min(c->n, kIoBodies);
         const size_t runs = 2 * sizeof(MeshRun), scal = 8 * sizeof(double);
@@ -1294,26 +1303,16 @@ int sol_destroy(sol_context *c)
     if (!c) return SOL_OK;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    if (c->stream2) (void)hipStreamSynchronize(c->stream2);
+    if (c->stream2) StreamPool::give_back(c->device, c->stream2);
     adjoint_release(c);
     for (void *p : c->allocs) (void)hipFree(p);
     if (c->part) (void)hipFree(c->part);
-    if (c->nnr2) (void)hipFree(c->nnr2);
-    if (c->nnidx) (void)hipFree(c->nnidx);
     if (c->apart) (void)hipFree(c->apart);
-    if (c->bpart) (void)hipFree(c->bpart);
-    {
-        void *gp[] = {c->grid.params, c->grid.bbox, c->grid.count, c->grid.start, c->grid.cellof,
-                      c->grid.rank, c->grid.spos, c->grid.r2, c->grid.idx};
-        for (void *q : gp)
-            if (q) (void)hipFree(q);
-    }
     if (c->pinned) (void)hipHostFree(c->pinned);
     if (c->integ_h) (void)hipHostFree(c->integ_h);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
     if (c->ev_join) (void)hipEventDestroy(c->ev_join);
-    if (c->stream2) (void)hipStreamDestroy(c->stream2);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return SOL_OK;

@@ -178,30 +178,39 @@ int dalloc(sol_context *c, T **p, size_t count)
     return SOL_OK;
 }
 
-// Arrays of a context in one allocation, zeroed by one fill: each of its own
-// took 15 us (30 arrays of 515 bodies: context 600 us, in one 250).
+// Several arrays in one allocation, which the first of them starts.  Each
+// allocation takes time of its own to make, to fill and to give back: a context
+// of 515 bodies made and destroyed takes 565 us with 33 of them and 400 with
+// three, of a disk of 16,385 865 us with 47 and 545 with five.
 class ArrayBlock {
 public:
     template <typename T>
     void add(T **p, size_t count)
     {
         items_.push_back({p, bytes_});
-        bytes_ += (std::max<size_t>(count, 1) * sizeof(T) + 255) / 256 * 256;
+        bytes_ += (std::max<size_t>(count, 1) * sizeof(T) + kPage - 1) / kPage * kPage;
     }
-    // Leaves the pointers alone when it fails.
+    size_t bytes() const { return bytes_; }
+    void place(void *block)
+    {
+        for (const Item &i : items_) {
+            void *at = static_cast<unsigned char *>(block) + i.at;
+            std::memcpy(i.p, &at, sizeof at);
+        }
+    }
+    // Owned by the context (freed by sol_destroy), zeroed.  Leaves the pointers
+    // alone when it fails.
     int make(sol_context *c)
     {
         unsigned char *q = nullptr;
         if (int r = dalloc(c, &q, bytes_)) return r;
-        for (const Item &i : items_) {
-            void *at = q + i.at;
-            std::memcpy(i.p, &at, sizeof at);
-        }
+        place(q);
         return SOL_OK;
     }
 
 private:
-    struct Item { void *p; size_t at; };       // the pointer's place
+    static constexpr size_t kPage = 4096;      // (at 256 bytes a mixed step of 32,769 bodies is 1.2% slower)
+    struct Item { void *p; size_t at; };       // the pointer's place, and its array's in the block
     std::vector<Item> items_;
     size_t bytes_ = 0;
 };

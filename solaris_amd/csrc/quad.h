@@ -23,8 +23,7 @@ struct QuadSync {
 };
 
 struct QuadArgs {
-    // the descriptor, and where it goes at the end.  By value: a copy to the
-    // device of its own cost 3.5 us of a Driver call
+    // the descriptor, by value, and where it goes at the end
     ResSystem system_in;
     ResSystem *system;
     QuadSync *sync;

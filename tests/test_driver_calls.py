@@ -24,3 +24,7 @@ def run(tmp_path, name):
 
 def test_driver_calls(tmp_path):
     assert "driver calls: ok" in run(tmp_path, "driver_calls_check")
+
+
+def test_context_calls(tmp_path):
+    assert "context calls: ok" in run(tmp_path, "context_calls_check")
