@@ -1456,12 +1456,13 @@ int sol_compute(sol_context *c, double t, const double *yh, double *dydt)
 {
     if (check_ctx(c) || !yh || !dydt) return SOL_ERR_ARGUMENT;
     HIPCHECK(c, hipSetDevice(c->device));
+    CallEnd end(c);
     const double *rows;
     int r = rows_in(c, yh, &rows);
     if (r) return r;
     r = evaluate_at(c, c->cin, t, 0.0, rows_out(c), EPI_ROWS, INTEG_RKF78, c->side_outputs, false, rows);
     if (r) return r;
-    return rows_done(c, dydt);
+    return end(rows_done(c, dydt));
 }
 
 int sol_get_side_outputs(sol_context *c, double *rm3, int32_t *nn, double *dist, int32_t *mig)
@@ -1469,6 +1470,7 @@ int sol_get_side_outputs(sol_context *c, double *rm3, int32_t *nn, double *dist,
     if (check_ctx(c)) return SOL_ERR_ARGUMENT;
     HIPCHECK(c, hipSetDevice(c->device));
     const size_t n = c->n;
+    CallEnd end(c);
     if (24 * n <= c->io_bytes) {
         launch_pack_side(c->stream, c->n, c->rm3, c->nnd, c->nni, c->migt, c->io_h);
         HIPCHECK(c, hipGetLastError());
@@ -1478,14 +1480,14 @@ int sol_get_side_outputs(sol_context *c, double *rm3, int32_t *nn, double *dist,
         if (dist) std::memcpy(dist, c->io_h + n, n * sizeof(double));
         if (nn) std::memcpy(nn, k, n * sizeof(int32_t));
         if (mig) std::memcpy(mig, k + n, n * sizeof(int32_t));
-        return SOL_OK;
+        return end(SOL_OK);
     }
     if (rm3) HIPCHECK(c, hipMemcpyAsync(rm3, c->rm3, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     if (nn) HIPCHECK(c, hipMemcpyAsync(nn, c->nni, n * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
     if (dist) HIPCHECK(c, hipMemcpyAsync(dist, c->nnd, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     if (mig) HIPCHECK(c, hipMemcpyAsync(mig, c->migt, n * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
     HIPCHECK(c, hipStreamSynchronize(c->stream));
-    return SOL_OK;
+    return end(SOL_OK);
 }
 
 int sol_set_mig_type(sol_context *c, const int32_t *mig)
@@ -1500,11 +1502,12 @@ int sol_set_mig_type(sol_context *c, const int32_t *mig)
 static int upload_soa(sol_context *c, const double *host, double *dst)
 {
     HIPCHECK(c, hipSetDevice(c->device));
+    CallEnd end(c);
     const double *rows;
     if (int r = rows_in(c, host, &rows)) return r;
     launch_aos_to_soa(c->stream, c->n, c->np, rows, dst);
     HIPCHECK(c, hipStreamSynchronize(c->stream));
-    return SOL_OK;
+    return end(SOL_OK);
 }
 
 int sol_set_state(sol_context *c, const double *y0)
@@ -1532,24 +1535,26 @@ int sol_get_array(sol_context *c, int32_t which, double *out)
     default: return c->fail(SOL_ERR_ARGUMENT, "unknown array %d", which);
     }
     HIPCHECK(c, hipSetDevice(c->device));
+    CallEnd end(c);
     launch_soa_to_aos(c->stream, c->n, c->np, src, rows_out(c));
-    return rows_done(c, out);
+    return end(rows_done(c, out));
 }
 
 int sol_driver(sol_context *c, int32_t integrator, double eps, sol_timeline *tl, double *body_h)
 {
     if (check_ctx(c) || !tl) return SOL_ERR_ARGUMENT;
     HIPCHECK(c, hipSetDevice(c->device));
+    CallEnd end(c);
     switch (integrator) {
-    case SOL_RUNGE_KUTTA_FEHLBERG78: return driver_rkf78(c, eps, tl, body_h, nullptr);
+    case SOL_RUNGE_KUTTA_FEHLBERG78: return end(driver_rkf78(c, eps, tl, body_h, nullptr));
     case SOL_RUNGE_KUTTA4: {
         // the RK4 step reads no error back, so its kernels may still be queued
         const int r = driver_rk4(c, tl, body_h, nullptr);
         if (r) return r;
         HIPCHECK(c, hipStreamSynchronize(c->stream));
-        return SOL_OK;
+        return end(SOL_OK);
     }
-    case SOL_DORMAND_PRINCE: return driver_dp(c, eps, tl, body_h, nullptr);
+    case SOL_DORMAND_PRINCE: return end(driver_dp(c, eps, tl, body_h, nullptr));
     default: return c->fail(SOL_ERR_UNSUPPORTED, "integrator %d is not provided", integrator);
     }
 }
@@ -1560,10 +1565,11 @@ int sol_step(sol_context *c, int32_t integrator, double time, double h)
     const int ik = integ_kind(integrator);
     if (ik < 0) return c->fail(SOL_ERR_UNSUPPORTED, "integrator %d is not provided", integrator);
     HIPCHECK(c, hipSetDevice(c->device));
+    CallEnd end(c);
     int r = run_stages(c, ik, time, h, false, nullptr);
     if (r) return r;
     HIPCHECK(c, hipStreamSynchronize(c->stream));
-    return SOL_OK;
+    return end(SOL_OK);
 }
 
 int sol_error_max(sol_context *c, int32_t integrator, double eps, double *out)
@@ -1641,6 +1647,7 @@ int sol_integrate_until(sol_context *c, int32_t integrator, double eps, sol_time
     if (tl->flush_count < 0 || tl->flush_count >= 100)
         return c->fail(SOL_ERR_ARGUMENT, "timeline flush_count %d is not in [0, 100)", tl->flush_count);
     HIPCHECK(c, hipSetDevice(c->device));
+    CallEnd end(c);
     hipEvent_t e0, e1;
     HIPCHECK(c, hipEventCreate(&e0));
     HIPCHECK(c, hipEventCreate(&e1));
@@ -1719,7 +1726,7 @@ int sol_integrate_until(sol_context *c, int32_t integrator, double eps, sol_time
         stats->path = path == kPathMesh || path == kPathQuad ? SOL_PATH_GRID : path;
         stats->slices = path == SOL_PATH_GRID ? gm.nslices : groups;
     }
-    return r;
+    return end(r);
 }
 
 int sol_integrals(sol_context *c, double *out)

@@ -154,6 +154,32 @@ struct sol_context {
     }
 };
 
+// The end of a call that queues work: one that fails in between waits for what
+// it has queued on either stream, as its kernels read and write pinned memory
+// that the next call fills, and the neighbour search may not have been joined.
+class CallEnd {
+public:
+    explicit CallEnd(sol_context *c) : c_(c) {}
+    ~CallEnd()
+    {
+        if (!failed_) return;
+        (void)hipStreamSynchronize(c_->stream);
+        if (c_->stream2) (void)hipStreamSynchronize(c_->stream2);
+    }
+    CallEnd(const CallEnd &) = delete;
+    CallEnd &operator=(const CallEnd &) = delete;
+    // r is the call's result
+    int operator()(int r)
+    {
+        failed_ = r != SOL_OK;
+        return r;
+    }
+
+private:
+    sol_context *c_;
+    bool failed_ = true;
+};
+
 #define HIPCHECK(ctx, call)                                                                    \
     do {                                                                                       \
         hipError_t e_ = (call);                                                                \

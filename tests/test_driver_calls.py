@@ -28,3 +28,7 @@ def test_driver_calls(tmp_path):
 
 def test_context_calls(tmp_path):
     assert "context calls: ok" in run(tmp_path, "context_calls_check")
+
+
+def test_error_calls(tmp_path):
+    assert "error calls: ok" in run(tmp_path, "error_calls_check")
