@@ -462,7 +462,7 @@ __global__ __launch_bounds__(kMeshThreads) void k_mesh(MeshArgs A, int max_steps
 #pragma unroll
                 for (int k = 0; k < kMeshMaxGroups / kWave; ++k)
                     if (k * kWave < pgroups) here &= k * kWave + lane >= pgroups || (int32_t)(v[k] - x) >= 0;
-                if (__all(here)) break;
+                if (__all(here) && A.ticks != 0) break;       // (no budget: never)
                 if ((it & 7) == 7 || A.ticks == 0) {
                     if (__hip_atomic_load(&sy->error, __ATOMIC_RELAXED, MESH_SCOPE) != 0) { ok = false; break; }
                     if (__builtin_amdgcn_s_memrealtime() - t0 >= A.ticks) {
