@@ -975,8 +975,8 @@ int mesh_run(sol_context *c, int path, int ik, double eps, sol_timeline *tl, int
         Q.mig_do1 = c->nb.proto_planet > 0;
         Q.mig_do2 = c->nb.giant_planet > 0;
     }
-    const double per_step = quad ? 5.0e-5 : 13.0 * (5.0e-6 + (double)c->n * (double)c->n * 1.0e-12);
-    const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(20000, (int64_t)(0.2 / per_step)));
+    // (a quad step with drag takes about 40 us)
+    const int64_t chunk = quad ? 4000 : mesh_chunk(c->n);
     A.y0_in = c->y0;
     for (bool first = true;; first = false) {
         const int64_t k = max_steps > 0 ? std::min(chunk, max_steps - S.steps) : chunk;

@@ -720,6 +720,8 @@ int sol_ensemble_run(sol_ensemble *e, int32_t integrator, double eps, int64_t ma
     // system's Driver loop (13 stage evaluations of ~3,000 + 12 n cycles)
     const double per_step = 13.0 * (3000.0 + 12.0 * e->nmax) / 2.1e9;
     int chunk = (int)std::max<int64_t>(16, std::min<int64_t>(20000, (int64_t)(0.25 / per_step)));
+    // (of the mesh form, whose launches hold their compute units, about 0.2 s)
+    if (e->mesh_state && !e->mesh_off) chunk = std::min(chunk, mesh_chunk(e->nmax));
     if (max_steps > 0) chunk = (int)std::min<int64_t>(chunk, max_steps);
     // where the last systems may take the mesh form, the launches start short
     // and grow, so that few running systems are soon noticed (run_mesh)

@@ -2,6 +2,8 @@
 // workgroups (mesh.hip).
 #pragma once
 
+#include <algorithm>
+
 #include "resident.h"
 
 namespace sol {
@@ -45,6 +47,14 @@ struct MeshArgs {
     double eps2;               // Plummer softening squared
     uint64_t ticks;            // real-time-counter ticks a wait lasts before it gives up
 };
+
+// Accepted steps of a launch for systems of up to n bodies: about 0.2 s at
+// RKF78's 13 evaluations and one attempt each.
+inline int mesh_chunk(int n)
+{
+    const double per_step = 13.0 * (5.0e-6 + (double)n * (double)n * 1.0e-12);
+    return std::max(1, (int)std::min(20000.0, 0.2 / per_step));
+}
 
 // Bodies per workgroup for n bodies, nm of them massive, with source ranges
 // [1, end_a) (massive) and [1, end_b) (the others) on at most `cus`

@@ -32,3 +32,7 @@ def test_context_calls(tmp_path):
 
 def test_error_calls(tmp_path):
     assert "error calls: ok" in run(tmp_path, "error_calls_check")
+
+
+def test_ensemble_calls(tmp_path):
+    assert "ensemble calls: ok" in run(tmp_path, "ensemble_calls_check")
