@@ -731,6 +731,8 @@ bool use_quad(sol_context *c, int ik, QuadShape *out = nullptr)
     QuadShape q{};
     q.sources = grid_sources(c) - 1;
     if (q.sources < 1 || q.sources > kQuadMaxSources) return false;
+    // a profiled context (sol_profile) keeps the launches that are timed
+    if (c->profiling && !use_grid(c, ik, nullptr) && !use_resident(c, ik)) return false;
     if (c->has_gas && !c->gas_dead) {
         SliceMap m{};
         if (!grid_slices(c, ik, &m) || m.stride > kQuadGasBodies || m.nslices < 1 ||
