@@ -69,12 +69,15 @@ struct sol_ensemble {
     double *y0 = nullptr, *y = nullptr, *acc0 = nullptr, *yscale = nullptr, *errv = nullptr, *fst = nullptr;
     double *mass = nullptr, *rm3 = nullptr, *nnd = nullptr;
     int32_t *nni = nullptr;
-    // the persistent launch: queue of slots (order_d, head_d), its shape
-    // (block threads per system, grid workgroups) and the candidates the
-    // tuner times
-    int32_t *order_d = nullptr, *head_d = nullptr;
-    std::vector<int32_t> order_h;        // the narrow queue (order_d[0 ..))
-    std::vector<int32_t> order_w;        // the wide queue (order_d[order_h.size() ..))
+    // the persistent launch: the queues of slots (queue_d: the two queues'
+    // words, the narrow queue's slots, and from count_n on the wide one's), its
+    // shape (block threads per system, grid workgroups) and the candidates
+    // the tuner times
+    int32_t *queue_d = nullptr;
+    std::vector<int32_t> queue_h;
+    std::vector<int32_t> order_h;        // the narrow queue
+    std::vector<int32_t> order_w;        // the wide queue
+    int count_n = 0, count_w = 0;        // systems of each, running or not
     int nmax = 0, cu_count = 256;
     int nmax_n = 0, nmax_w = 0;          // largest system of each queue
     int block = 0, grid = 0;
@@ -87,8 +90,7 @@ struct sol_ensemble {
     std::vector<int> cand;
     std::vector<double> cand_ms;
     hipGraphExec_t graph = nullptr, graph_w = nullptr;   // the narrow and the wide queue's launch
-    int graph_integ = -1, graph_steps = 0, graph_block = 0, graph_n = 0;
-    int graphw_integ = -1, graphw_steps = 0, graph_nw = 0;
+    int graph_integ = -1, graph_block = 0, graphw_integ = -1;      // what they were captured for
     int64_t launches = 0, graph_launches = 0;
     std::vector<int64_t> last_steps;     // per slot: steps of the previous launch
     // the mesh form for the last systems (mesh.h): their descriptors while it
@@ -115,6 +117,9 @@ struct sol_ensemble {
     } while (0)
 
 namespace {
+
+// Where the slots start in an ensemble's queue_d.
+constexpr int kQueueSlots = 2 * sizeof(QueueWords) / sizeof(int32_t);
 
 // Accepted steps of a run's first launch.
 constexpr int kFirstSteps = 16;
@@ -197,8 +202,9 @@ bool is_wide(const sol_ensemble *e, int s) { return e->wide_block > 0 && e->sys_
 // Queue orders for the next launch: the running systems of each queue that
 // have not had their steps (the narrow one only when `narrow_only`), the most work expected first
 // (n^2 times the steps the system took in the previous launch, n^2 alone
-// before the first), so that the long ones start early.
-int make_order(sol_ensemble *e, bool narrow_only = false, const std::vector<char> *had = nullptr)
+// before the first), so that the long ones start early.  steps: the accepted
+// steps of the launches that take them.
+int make_order(sol_ensemble *e, int steps, bool narrow_only = false, const std::vector<char> *had = nullptr)
 {
     e->order_h.clear();
     e->order_w.clear();
@@ -214,43 +220,46 @@ int make_order(sol_ensemble *e, bool narrow_only = false, const std::vector<char
     auto by_cost = [&](int a, int b) { return cost(a) > cost(b); };
     std::stable_sort(e->order_h.begin(), e->order_h.end(), by_cost);
     std::stable_sort(e->order_w.begin(), e->order_w.end(), by_cost);
-    const int nn = (int)e->order_h.size(), nw = (int)e->order_w.size();
-    if (nn > 0)
-        ECHECK(e, hipMemcpyAsync(e->order_d, e->order_h.data(), nn * sizeof(int32_t), hipMemcpyHostToDevice,
-                                 e->stream));
-    if (nw > 0)
-        ECHECK(e, hipMemcpyAsync(e->order_d + nn, e->order_w.data(), nw * sizeof(int32_t), hipMemcpyHostToDevice,
-                                 e->stream));
+    if (e->order_h.empty() && e->order_w.empty()) return SOL_OK;
+    const QueueWords words[2] = {{0, (int32_t)e->order_h.size(), steps, 0}, {0, (int32_t)e->order_w.size(), steps, 0}};
+    std::memcpy(e->queue_h.data(), words, sizeof words);
+    std::copy(e->order_h.begin(), e->order_h.end(), e->queue_h.begin() + kQueueSlots);
+    std::copy(e->order_w.begin(), e->order_w.end(), e->queue_h.begin() + kQueueSlots + e->count_n);
+    ECHECK(e, hipMemcpyAsync(e->queue_d, e->queue_h.data(), e->queue_h.size() * sizeof(int32_t), hipMemcpyHostToDevice,
+                             e->stream));
     return SOL_OK;
 }
 
-// Enqueues one queue's launch (the counter reset and the kernel) on st:
-// the narrow queue (order_d[0 .. nn)) or the wide one (after it).
-void enqueue_one(sol_ensemble *e, hipStream_t st, int ik, int steps, int block, bool wide, const ResArrays &A)
+// Enqueues one queue's launch (the counter reset and the kernel) on st, with
+// workgroups for all its systems, running or not: what is left of them and
+// their steps are in the queue's words.
+void enqueue_one(sol_ensemble *e, hipStream_t st, int ik, int block, bool wide, const ResArrays &A)
 {
-    const int nn = (int)e->order_h.size(), nw = (int)e->order_w.size();
+    QueueWords *words = reinterpret_cast<QueueWords *>(e->queue_d);
+    const int32_t *slots = e->queue_d + kQueueSlots;
     if (wide) {
         // RKF78: the four most-read stage derivatives in LDS where they fit
         // (one wide workgroup per CU: its registers leave room for no other)
         const int lf = ik == INTEG_RKF78 && resident_lds_bytes(e->nmax_w) + resident_queue_lds_f(e->nmax_w) + 4096 <=
                                                 e->lds_per_block ? 4 : 0;
         const int per_cu = resident_queue_occupancy(ik, e->wide_block, e->nmax_w, lf);
-        e->grid_w = std::max(1, std::min(nw, e->cu_count * per_cu));
-        launch_resident_queue(st, ik, e->sys_d, e->order_d + nn, nw, e->head_d + 1, A, steps, e->grid_w,
-                              e->wide_block, e->nmax_w, e->wide_lsh, lf);
+        e->grid_w = std::max(1, std::min(e->count_w, e->cu_count * per_cu));
+        launch_resident_queue(st, ik, e->sys_d, slots + e->count_n, words + 1, A, e->grid_w, e->wide_block, e->nmax_w,
+                              e->wide_lsh, lf);
     } else {
-        e->grid = grid_for(e, ik, block, nn);
-        launch_resident_queue(st, ik, e->sys_d, e->order_d, nn, e->head_d, A, steps, e->grid, block, e->nmax_n);
+        e->grid = grid_for(e, ik, block, e->count_n);
+        launch_resident_queue(st, ik, e->sys_d, slots, words, A, e->grid, block, e->nmax_n);
     }
 }
 
-// Captures one queue's launch into *exec (rebuilt when its key changed).
-int capture_one(sol_ensemble *e, hipGraphExec_t *exec, int ik, int steps, int block, bool wide, const ResArrays &A)
+// Captures one queue's launch into *exec (again for another integrator or
+// launch shape only).
+int capture_one(sol_ensemble *e, hipGraphExec_t *exec, int ik, int block, bool wide, const ResArrays &A)
 {
     if (*exec) { (void)hipGraphExecDestroy(*exec); *exec = nullptr; }
     hipGraph_t g;
     ECHECK(e, hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_one(e, e->stream, ik, steps, block, wide, A);
+    enqueue_one(e, e->stream, ik, block, wide, A);
     hipError_t le = hipGetLastError();
     hipError_t ce = hipStreamEndCapture(e->stream, &g);
     if (le != hipSuccess || ce != hipSuccess) return e->fail(SOL_ERR_DEVICE, "graph capture failed");
@@ -259,26 +268,25 @@ int capture_one(sol_ensemble *e, hipGraphExec_t *exec, int ik, int steps, int bl
     return SOL_OK;
 }
 
-// One persistent launch per queue over the queued systems, each for up to
-// `steps` accepted steps; through the captured graphs when `graph` is set.
+// One persistent launch per queue over the systems that make_order queued;
+// through the captured graphs when `graph` is set.
 // The wide queue runs on the ensemble's stream, the narrow one beside it
 // on the second stream (forked from the first and joined back), so the
 // two kernels share the device: each queue's launch is a graph of its own,
 // since the branches of one graph were found to run one after the other.
-int launch_queue(sol_ensemble *e, int ik, int steps, int block, bool graph)
+int launch_queue(sol_ensemble *e, int ik, int block, bool graph)
 {
     const int nn = (int)e->order_h.size(), nw = (int)e->order_w.size();
     const ResArrays A = arrays(e);
     ++e->launches;
     if (graph) {
-        if (nn > 0 && (!e->graph || e->graph_integ != ik || e->graph_steps != steps || e->graph_block != block ||
-                       e->graph_n != nn)) {
-            if (int r = capture_one(e, &e->graph, ik, steps, block, false, A)) return r;
-            e->graph_integ = ik; e->graph_steps = steps; e->graph_block = block; e->graph_n = nn;
+        if (nn > 0 && (!e->graph || e->graph_integ != ik || e->graph_block != block)) {
+            if (int r = capture_one(e, &e->graph, ik, block, false, A)) return r;
+            e->graph_integ = ik; e->graph_block = block;
         }
-        if (nw > 0 && (!e->graph_w || e->graphw_integ != ik || e->graphw_steps != steps || e->graph_nw != nw)) {
-            if (int r = capture_one(e, &e->graph_w, ik, steps, block, true, A)) return r;
-            e->graphw_integ = ik; e->graphw_steps = steps; e->graph_nw = nw;
+        if (nw > 0 && (!e->graph_w || e->graphw_integ != ik)) {
+            if (int r = capture_one(e, &e->graph_w, ik, block, true, A)) return r;
+            e->graphw_integ = ik;
         }
     }
     const bool both = nn > 0 && nw > 0;
@@ -288,12 +296,12 @@ int launch_queue(sol_ensemble *e, int ik, int steps, int block, bool graph)
     }
     if (nw > 0) {
         if (graph) ECHECK(e, hipGraphLaunch(e->graph_w, e->stream));
-        else enqueue_one(e, e->stream, ik, steps, block, true, A);
+        else enqueue_one(e, e->stream, ik, block, true, A);
     }
     if (nn > 0) {
         hipStream_t sn = both ? e->stream2 : e->stream;
         if (graph) ECHECK(e, hipGraphLaunch(e->graph, sn));
-        else enqueue_one(e, sn, ik, steps, block, false, A);
+        else enqueue_one(e, sn, ik, block, false, A);
     }
     if (both) {
         ECHECK(e, hipEventRecord(e->ev_join, e->stream2));
@@ -426,7 +434,7 @@ int tune(sol_ensemble *e, int ik, double eps, int probe_steps)
     ECHECK(e, hipMemcpyAsync(sys_save, e->sys_d, e->sys_h.size() * sizeof(ResSystem), hipMemcpyDeviceToDevice,
                              e->stream));
     // the probe times the narrow queue's shapes on its own systems
-    int r = make_order(e, true);
+    int r = make_order(e, probe_steps, true);
     e->cand_ms.assign(e->cand.size(), 0.0);
     hipEvent_t t0 = nullptr, t1 = nullptr;
     if (!r && (hipEventCreate(&t0) != hipSuccess || hipEventCreate(&t1) != hipSuccess))
@@ -434,7 +442,7 @@ int tune(sol_ensemble *e, int ik, double eps, int probe_steps)
     double best = -1.0;
     for (size_t k = 0; !r && k < e->cand.size() && !e->order_h.empty(); ++k) {
         (void)hipEventRecord(t0, e->stream);
-        r = launch_queue(e, ik, probe_steps, e->cand[k], false);
+        r = launch_queue(e, ik, e->cand[k], false);
         (void)hipEventRecord(t1, e->stream);
         if (!r && hipEventSynchronize(t1) != hipSuccess) r = e->fail(SOL_ERR_DEVICE, "tuning launch failed");
         float ms = 0.0f;
@@ -542,6 +550,9 @@ int sol_ensemble_create(sol_ensemble **out, int32_t nsys, const sol_nbodies *nbs
         e->nmax_n = e->nmax;
         e->nmax_w = 0;
     }
+    for (int k = 0; k < nsys; ++k) e->count_w += e->wide_block > 0 && nbs[k].total >= e->wide_min ? 1 : 0;
+    e->count_n = nsys - e->count_w;
+    e->queue_h.assign((size_t)kQueueSlots + nsys, 0);
     // launch shapes the tuner times for the narrow queue: the exact fit
     // (one body per thread up to 640 bodies) and the multiples of 64 below
     // it that hold the largest system at two or four bodies per thread
@@ -572,7 +583,7 @@ int sol_ensemble_create(sol_ensemble **out, int32_t nsys, const sol_nbodies *nbs
         (r = ealloc(e, &e->acc0, 6 * tot)) || (r = ealloc(e, &e->yscale, 6 * tot)) ||
         (r = ealloc(e, &e->errv, 6 * tot)) || (r = ealloc(e, &e->fst, 12 * 6 * tot)) ||
         (r = ealloc(e, &e->mass, tot)) || (r = ealloc(e, &e->rm3, tot)) || (r = ealloc(e, &e->nnd, tot)) ||
-        (r = ealloc(e, &e->nni, tot)) || (r = ealloc(e, &e->order_d, nsys)) || (r = ealloc(e, &e->head_d, 2))) {
+        (r = ealloc(e, &e->nni, tot)) || (r = ealloc(e, &e->queue_d, e->queue_h.size()))) {
         g_ens_create_error = e->err;
         sol_ensemble_destroy(e);
         return r;
@@ -628,7 +639,7 @@ int sol_ensemble_destroy(sol_ensemble *e)
     if (e->graph) (void)hipGraphExecDestroy(e->graph);
     if (e->graph_w) (void)hipGraphExecDestroy(e->graph_w);
     void *ptrs[] = {e->sys_d, e->y0,  e->y,   e->acc0, e->yscale,  e->errv,  e->fst,
-                    e->mass,  e->rm3, e->nnd, e->nni,  e->order_d, e->head_d,
+                    e->mass,  e->rm3, e->nnd, e->nni,  e->queue_d,
                     e->mesh_state, e->mesh_gm, e->mesh_pos, e->mesh_sys, e->mesh_part, e->mesh_part_of,
                     e->mesh_sync};
     for (void *p : ptrs)
@@ -740,9 +751,9 @@ int sol_ensemble_run(sol_ensemble *e, int32_t integrator, double eps, int64_t ma
         for (int s = 0; s < e->nsys; ++s) before[s] = e->sys_h[s].steps;
         if (done_steps > 0)
             if (int r = run_mesh(e, ik, k, had)) return r;
-        if (int r = make_order(e, false, &had)) return r;
+        if (int r = make_order(e, k, false, &had)) return r;
         if (!e->order_h.empty() || !e->order_w.empty()) {
-            if (int r = launch_queue(e, ik, k, e->block, true)) return r;
+            if (int r = launch_queue(e, ik, e->block, true)) return r;
             if (int r = read_systems(e)) return r;
         }
         done_steps += k;

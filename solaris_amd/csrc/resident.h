@@ -93,10 +93,15 @@ size_t resident_lds_bytes(int nmax);
 void launch_resident(hipStream_t st, int integ, ResSystem *systems, int nsys, const ResArrays &A, int max_steps,
                      int block, int nmax, size_t lds_limit);
 
+// What the persistent form reads of its queue: the counter its workgroups take
+// systems by, how many there are, and the accepted steps each is run for at
+// most.  On the device, so that a captured launch serves every queue.
+struct QueueWords { int32_t head, nsys, max_steps, pad; };
+
 // The persistent form: `grid` workgroups of `block` threads take systems
-// from the queue order[0 .. nsys) (through the device counter head, which
+// from the queue order[0 .. q->nsys) (through the counter q->head, which
 // the launch zeroes first with a one-thread kernel, so the pair can be
-// captured in a graph) and run each for up to max_steps accepted steps.
+// captured in a graph) and run each for up to q->max_steps accepted steps.
 // Bodies per thread: resident_queue_bpt(block, nmax), at most 4.  With one
 // body per thread (nmax <= block, blocks of up to 768 threads) each
 // system's bodies get up to 1 << max_lsh lanes each, which split the
@@ -104,9 +109,8 @@ void launch_resident(hipStream_t st, int integ, ResSystem *systems, int nsys, co
 int resident_queue_bpt(int block, int nmax);
 // lf = 4 (RKF78, one body per thread, blocks of up to 640 threads): F0 and
 // F3-F5 in LDS, resident_queue_lds_f(nmax) more bytes of it.
-void launch_resident_queue(hipStream_t st, int integ, ResSystem *systems, const int32_t *order, int nsys,
-                           int32_t *head, const ResArrays &A, int max_steps, int grid, int block, int nmax,
-                           int max_lsh = 0, int lf = 0);
+void launch_resident_queue(hipStream_t st, int integ, ResSystem *systems, const int32_t *order, QueueWords *q,
+                           const ResArrays &A, int grid, int block, int nmax, int max_lsh = 0, int lf = 0);
 // Workgroups of that launch one CU holds at once.
 int resident_queue_occupancy(int integ, int block, int nmax, int lf = 0);
 size_t resident_queue_lds_f(int nmax);

@@ -1234,16 +1234,16 @@ __global__ __launch_bounds__(256) void k_resident_grid(ResSystem *systems, ResAr
 // LDS rows (the lanes of a body share its row and write the same values).
 template <int INTEG, int BPT, int BOUND, int LF = 0>
 __global__ __launch_bounds__(BOUND) void k_resident_queue(ResSystem *systems, const int32_t *__restrict__ order,
-                                                          int nsys, int32_t *head, ResArrays A, int max_steps,
-                                                          int nmax, int max_lsh)
+                                                          QueueWords *q, ResArrays A, int nmax, int max_lsh)
 {
     extern __shared__ double4 lds[];
     __shared__ double red[16];
     __shared__ double sh[4];
     __shared__ double part[6 * (BOUND / kWave)];
     __shared__ int32_t slot;
+    const int nsys = __builtin_amdgcn_readfirstlane(q->nsys), max_steps = __builtin_amdgcn_readfirstlane(q->max_steps);
     for (;;) {
-        if (threadIdx.x == 0) slot = atomicAdd(head, 1);
+        if (threadIdx.x == 0) slot = atomicAdd(&q->head, 1);
         __syncthreads();
         const int32_t k = slot;
         __syncthreads();   // every thread has read slot before it is taken again
@@ -1384,15 +1384,13 @@ void launch_integ(hipStream_t st, ResSystem *systems, int nsys, const ResArrays 
 }
 
 template <int INTEG>
-void launch_queue_bpt(hipStream_t st, ResSystem *systems, const int32_t *order, int nsys, int32_t *head,
-                      const ResArrays &A, int max_steps, int grid, int block, int bpt, int nmax, size_t lds,
-                      int max_lsh, int lf)
+void launch_queue_bpt(hipStream_t st, ResSystem *systems, const int32_t *order, QueueWords *q, const ResArrays &A,
+                      int grid, int block, int bpt, int nmax, size_t lds, int max_lsh, int lf)
 {
     if constexpr (INTEG == INTEG_RKF78) {
         if (bpt == 1 && lf == 4 && block <= 640) {
             hipLaunchKernelGGL((k_resident_queue<INTEG, 1, 640, 4>), dim3(grid), dim3(block),
-                               lds + lds_f_bytes(nmax, 4), st, systems, order, nsys, head, A, max_steps, nmax,
-                               max_lsh);
+                               lds + lds_f_bytes(nmax, 4), st, systems, order, q, A, nmax, max_lsh);
             return;
         }
     }
@@ -1400,18 +1398,18 @@ void launch_queue_bpt(hipStream_t st, ResSystem *systems, const int32_t *order, 
     case 1:
         if (block > 640)
             hipLaunchKernelGGL((k_resident_queue<INTEG, 1, 768>), dim3(grid), dim3(block), lds, st, systems, order,
-                               nsys, head, A, max_steps, nmax, max_lsh);
+                               q, A, nmax, max_lsh);
         else
             hipLaunchKernelGGL((k_resident_queue<INTEG, 1, 640>), dim3(grid), dim3(block), lds, st, systems, order,
-                               nsys, head, A, max_steps, nmax, max_lsh);
+                               q, A, nmax, max_lsh);
         break;
     case 2:
         hipLaunchKernelGGL((k_resident_queue<INTEG, 2, 512>), dim3(grid), dim3(block), lds, st, systems, order,
-                           nsys, head, A, max_steps, nmax, 0);
+                           q, A, nmax, 0);
         break;
     default:
         hipLaunchKernelGGL((k_resident_queue<INTEG, 4, 512>), dim3(grid), dim3(block), lds, st, systems, order,
-                           nsys, head, A, max_steps, nmax, 0);
+                           q, A, nmax, 0);
         break;
     }
 }
@@ -1431,24 +1429,23 @@ const void *queue_kernel(int bpt, int block, int lf)
 
 int resident_queue_bpt(int block, int nmax) { return nmax <= block ? 1 : nmax <= 2 * block ? 2 : 4; }
 
-void launch_resident_queue(hipStream_t st, int integ, ResSystem *systems, const int32_t *order, int nsys,
-                           int32_t *head, const ResArrays &A, int max_steps, int grid, int block, int nmax,
-                           int max_lsh, int lf)
+void launch_resident_queue(hipStream_t st, int integ, ResSystem *systems, const int32_t *order, QueueWords *q,
+                           const ResArrays &A, int grid, int block, int nmax, int max_lsh, int lf)
 {
     const size_t lds = resident_lds_bytes(nmax);
     const int bpt = resident_queue_bpt(block, nmax);
-    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, head);
+    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, &q->head);
     switch (integ) {
     case INTEG_RKF78:
-        launch_queue_bpt<INTEG_RKF78>(st, systems, order, nsys, head, A, max_steps, grid, block, bpt, nmax, lds,
+        launch_queue_bpt<INTEG_RKF78>(st, systems, order, q, A, grid, block, bpt, nmax, lds,
                                       max_lsh, lf);
         break;
     case INTEG_RK4:
-        launch_queue_bpt<INTEG_RK4>(st, systems, order, nsys, head, A, max_steps, grid, block, bpt, nmax, lds,
+        launch_queue_bpt<INTEG_RK4>(st, systems, order, q, A, grid, block, bpt, nmax, lds,
                                     max_lsh, 0);
         break;
     default:
-        launch_queue_bpt<INTEG_DP>(st, systems, order, nsys, head, A, max_steps, grid, block, bpt, nmax, lds,
+        launch_queue_bpt<INTEG_DP>(st, systems, order, q, A, grid, block, bpt, nmax, lds,
                                    max_lsh, 0);
         break;
     }

@@ -1,7 +1,8 @@
 // Host-side check of what runs of an ensemble ask of the runtime (fake_hip.h
 // in place of the HIP library; its kernels only count steps): a launch of the
-// mesh form, which holds compute units, is cut to about 0.2 s.  Exit status 0
-// when every check holds.
+// mesh form, which holds compute units, is cut to about 0.2 s, and each queue's
+// launch is captured once and replayed however many systems are left, in the
+// next run too.  Exit status 0 when every check holds.
 #include "fake_hip.h"
 
 #include "../../include/solaris_amd.h"
@@ -45,8 +46,8 @@ int main()
             for (int k = 0; k < g_nsys; ++k) advance(A.systems[k], steps);
         }
     };
-    // a queue's launch: the steps of the shortest
-    fake::on_graph() = [] { for (int k = 0; k < g_nsys; ++k) advance(g_systems[k], 16); };
+    // the queues' launches: the systems end one after the other
+    fake::on_graph() = [] { for (int k = 0; k < g_nsys; ++k) advance(g_systems[k], 16 + k); };
     std::vector<sol_nbodies> nb(nsys);
     for (int k = 0; k < nsys; ++k) {
         nb[k] = sol_nbodies{};
@@ -76,6 +77,18 @@ int main()
     // 13 evaluations of 5 us and 1 ps a pair
     expect("steps of a mesh launch", g_longest, (long)(0.2 / (13 * (5.0e-6 + 1.0e-12 * n * n))));
     if (g_longest == 0) { std::printf("FAIL no mesh launch\n"); ++g_fails; }
+    // a run of several launches, twice
+    g_end = 300;
+    long launches = 0;
+    for (int run = 0; run < 2; ++run) {
+        fake::forget();
+        set();
+        if (sol_ensemble_run(e, SOL_RUNGE_KUTTA4, 1e-10, 0, nullptr)) { std::printf("FAIL %s\n", sol_ensemble_last_error(e)); return 1; }
+        launches += fake::calls()["hipGraphLaunch"];
+        expect(run ? "captures of the second run" : "captures of the first run", fake::calls()["hipGraphInstantiate"], run ? 0 : 2);
+    }
+    std::printf("%ld graph launches\n", launches);
+    if (launches < 8) { std::printf("FAIL few launches\n"); ++g_fails; }
     sol_ensemble_destroy(e);
     if (!g_fails) std::printf("ensemble calls: ok\n");
     return g_fails != 0;
