@@ -338,7 +338,15 @@ int sol_interactions_per_evaluation(const sol_context *ctx, double *count);
  * counterpart in the reference, where each system is a separate simulation
  * (Simulator::Integrate, Solaris/Simulator.cpp:121-178); per system the
  * semantics are those of sol_integrate.  A failing system stops with its
- * own status. */
+ * own status.
+ * Once the running systems of at least 48 sources fit the device at several
+ * workgroups each, they go on in that form, which sums in another order; the
+ * launch shape decides on the order of sums too.  A system's last digits can
+ * therefore depend on the other systems of its ensemble (the same ensemble run
+ * again has the same bits in the same launch shape), which close encounters
+ * amplify (2.5e-11 AU over two days).  With SOLARIS_AMD_NO_GRID=1, which keeps
+ * all in the queues, and SOLARIS_AMD_ENSEMBLE_BLOCK set to at least the bodies
+ * of the first queue's largest system they do not. */
 typedef struct sol_ensemble sol_ensemble;
 enum { SOL_SYSTEM_RUNNING = 0, SOL_SYSTEM_DONE = 1, SOL_SYSTEM_UNDERFLOW = 2, SOL_SYSTEM_MAXITER = 3 };
 

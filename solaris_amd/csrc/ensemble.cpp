@@ -26,7 +26,8 @@
 //
 // Once the systems still running fit the device at several workgroups each,
 // those with many sources go on in the mesh form (run_mesh), so that the last
-// few do not take their steps on one CU each.
+// few do not take their steps on one CU each.  So which form a step of theirs is
+// summed in, and with it its last digits, depends on the systems beside them.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
