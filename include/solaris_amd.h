@@ -344,7 +344,7 @@ int sol_interactions_per_evaluation(const sol_context *ctx, double *count);
  * launch shape decides on the order of sums too.  A system's last digits can
  * therefore depend on the other systems of its ensemble (the same ensemble run
  * again has the same bits in the same launch shape), which close encounters
- * amplify (2.5e-11 AU over two days).  With SOLARIS_AMD_NO_GRID=1, which keeps
+ * amplify (1e-12 to 3e-11 AU over two days).  With SOLARIS_AMD_NO_GRID=1, which keeps
  * all in the queues, and SOLARIS_AMD_ENSEMBLE_BLOCK set to at least the bodies
  * of the first queue's largest system they do not. */
 typedef struct sol_ensemble sol_ensemble;

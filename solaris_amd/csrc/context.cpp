@@ -687,9 +687,10 @@ SliceArrays system_arrays(sol_context *c)
 // and 58 in one workgroup, of 17 bodies 47 and 35.
 constexpr int kMeshMinSources = 32;
 // ... and to 23 bodies per workgroup, 5,889 bodies: RKF78 and Dormand-Prince, us
-// per attempt in the mesh form and with one launch per stage: 3,501 287 and 451,
-// 207 and 330; 5,001 464 and 465, 331 and 342; with 31 per workgroup 6,001 627
-// and 580, 452 and 426; 7,937 801 and 626, 582 and 461.
+// per attempt in the mesh form and with one launch per stage: 3,501 268 and 460,
+// 193 and 334; 5,001 455 and 470, 326 and 344; 5,889 518 and 596, 369 and 434;
+// with 31 per workgroup (another session) 6,001 627 and 580, 452 and 426; 7,937
+// 801 and 626, 582 and 461.
 constexpr int kMeshContextShare = 23;
 constexpr int kPathMesh = 100, kPathQuad = 101;     // reported as SOL_PATH_GRID
 
@@ -718,10 +719,10 @@ bool use_mesh(sol_context *c, int ik, int *share_out = nullptr, int *groups_out 
 // ones, that have at most eight sources besides the star and bodies for at
 // most a workgroup per CU (14,339 with two planets).  The Sun, two planets and
 // test particles, us per RKF78 attempt in one workgroup or in slices, and in
-// quads: 4 bodies 15 and 7.0, 128 15 and 6.6, 515 17.7 and 6.9, 5,001 18.8 and
-// 7.4, 14,338 20.4 and 8.1.  With live gas: the grid form's slices of 64 and
-// 128 places, us per RKF78 attempt: 125 bodies 64 (one workgroup) and 33, 505
-// 51 and 33, 16,389 56 and 39.
+// quads: 4 bodies 15 and 6.0, 515 17.7 and 6.7, 5,001 18.8 and 7.4, 14,338 20.4
+// and 8.0.  With live gas: the grid form's slices of 64 and 128 places, us per
+// RKF78 attempt: 125 bodies 64 (one workgroup) and 32, 505 51 and 32, 16,389 56
+// and 37.
 struct QuadShape { int sources, own, groups, places; };   // places: bodies of a workgroup with gas (0: no gas)
 
 bool use_quad(sol_context *c, int ik, QuadShape *out = nullptr)

@@ -14,9 +14,10 @@
 // What bounds it: up to about 500 bodies the latency of an exchange (a store
 // to memory, a flag, a poll and the loads of the others' positions, some
 // 3,500 of 9,500 cycles per stage) and of the chain around it; above, the
-// FP64 pair terms.  RKF78 per attempt (13 evaluations): 257 bodies 59 us
-// (one workgroup 459, one launch per stage 600), 1,501 bodies 125 us (11,800
-// and 630), 5,001 bodies 456 us (one launch per stage 980).
+// FP64 pair terms, at two waves per SIMD, where an operation takes 5.9 cycles
+// and not the 4.9 of four.  RKF78 per attempt (13 evaluations): 257 bodies 58 us
+// (one workgroup 459, one launch per stage 609), 1,501 bodies 117 us (11,900
+// and 643), 5,001 bodies 455 us (one launch per stage 470).
 //
 // Exchange.  A workgroup writes its bodies' (x, y, z) to one of two global
 // buffers with system-scope stores, waits until they are in place, and raises

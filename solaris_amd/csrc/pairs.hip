@@ -322,8 +322,9 @@ void launch_mixed(hipStream_t st, const PairPlan &plan, const float4 *J32, const
 // places) twice a round; a quarter of an item per wave, and no column sums
 // but the current ones in registers (164 VGPRs and three waves per SIMD; with
 // the row sums held and the columns carried 246 and two), measured before and
-// after, us: 3,001 bodies 59 and 21, 5,001 61 and 23, 8,193 65 and 47, 12,001
-// 115 and 76, 16,385 168 and 125, 32,769 526 and 460, 65,537 1,676 and 1,604.
+// after in turn, us: 3,001 bodies 59 and 21, 5,001 60 and 24, 8,193 63 and 46,
+// 12,001 108 and 72, 16,385 154 and 120, 32,769 472 and 419; at 65,537, whose
+// items fill the device either way, 1,580 and 1,582.
 //
 // In a diagonal item (row == column) wave j meets the column tile t by
 // d = (t - j) mod 4: for d == 0 at steps 1..32 (step 32 on lanes 0..31), for
@@ -504,9 +505,9 @@ __device__ __forceinline__ float rot_lane_f(float v)
 // the rates under this load (1.4 and 4.4 ns), which bounds it from some 16,000
 // bodies on; below, a wave's 256 pairs per lane in turn do, so the plan splits
 // an item's steps over two or four units (context.cpp).  Four waves per SIMD.
-// Measured before (whole items per wave) and after, us: 3,001 bodies 81 and 16,
-// 5,001 82 and 22, 8,193 85 and 40, 16,385 110 and 93, 32,769 339 and 277,
-// 65,537 1,070 and 868.
+// Measured before (whole items per wave) and after in turn, us: 3,001 bodies 82
+// and 16, 5,001 83 and 21, 8,193 83 and 38, 12,001 93 and 51, 16,385 101 and 85,
+// 32,769 307 and 243, 65,537 976 and 839.
 template <bool SOFT>
 __global__ __launch_bounds__(256, 4) void k_pairs_sym_mixed(SymPlan sp, const float4 *__restrict__ J32,
                                                          const double4 *__restrict__ J, double *__restrict__ apart,

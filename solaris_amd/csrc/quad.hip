@@ -24,11 +24,11 @@
 // accepted with.
 //
 // Per attempt, before (slices of resident.hip, below 129 bodies one workgroup)
-// and after, us: RKF78 of 4 bodies 15.2 and 7.0, 515 17.7 and 6.9, 5,001 18.8
-// and 7.4, 14,338 20.4 and 8.1; Dormand-Prince of 515 13.7 and 5.7; RK4 of 515
+// and after, us: RKF78 of 4 bodies 15.2 and 6.0, 515 17.7 and 6.7, 5,001 18.8
+// and 7.4, 14,338 20.4 and 8.0; Dormand-Prince of 515 13.7 and 5.3; RK4 of 515
 // 4.4 and 1.5.  An evaluation of about 120 instructions takes 0.38 us, the
-// exchange 1.9 us.  With gas, RKF78 of 125 bodies 63.7 and 32.6, 505 51.3 and
-// 33.3, 16,389 55.9 and 39.
+// exchange 1.9 us.  With gas, RKF78 of 125 bodies 63.7 and 31.7, 505 51.3 and
+// 31.9, 16,389 55.9 and 37.
 #include <float.h>
 
 #include <algorithm>
