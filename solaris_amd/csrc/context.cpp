@@ -1420,6 +1420,7 @@ int sol_set_source_ranges(sol_context *c, int32_t a, int32_t b)
     if (check_ctx(c)) return SOL_ERR_ARGUMENT;
     adjoint_invalidate(c);
     if (a > c->n || b > c->n) return c->fail(SOL_ERR_ARGUMENT, "source range beyond total");
+    HIPCHECK(c, hipSetDevice(c->device));
     c->end_massive = a;
     c->end_other = b;
     build_plan(c);

@@ -2,7 +2,8 @@
 // runtime (fake_hip.h in place of the HIP library): its arrays in a few
 // allocations, all given back; a second stream only where the neighbour search
 // runs beside a symmetric pair sum, never shared by two contexts, kept for the
-// next one.  Exit status 0 when every check holds.
+// next one; a context's memory and streams on its own device, whichever is
+// current when it is called.  Exit status 0 when every check holds.
 #include "fake_hip.h"
 
 #include "../../include/solaris_amd.h"
@@ -15,7 +16,7 @@ static void expect(const char *what, int n, long got, long most)
     ++g_fails;
 }
 
-static sol_context *make(int planets, int particles)
+static sol_context *make(int planets, int particles, int device = 0)
 {
     sol_nbodies nb{};
     nb.central_body = 1;
@@ -23,7 +24,7 @@ static sol_context *make(int planets, int particles)
     nb.test_particle = particles;
     nb.total = 1 + planets + particles;
     sol_context *c = nullptr;
-    if (sol_create(&c, &nb, 0, 0) != SOL_OK) { std::printf("FAIL sol_create: %s\n", sol_last_error(nullptr)); std::exit(1); }
+    if (sol_create(&c, &nb, 0, device) != SOL_OK) { std::printf("FAIL sol_create: %s\n", sol_last_error(nullptr)); std::exit(1); }
     return c;
 }
 
@@ -56,6 +57,19 @@ int main()
         if (fake::calls()["hipStreamCreateWithFlags"] != 7 + 6) { std::printf("FAIL contexts share a stream\n"); ++g_fails; }
         for (sol_context *x : c) sol_destroy(x);
         expect("streams kept", 9001, (long)fake::streams().size(), 4);
+    }
+    {
+        // test particles that become sources: the symmetric sum comes later
+        fake::forget();
+        sol_context *c = make(2, 9000, 1);
+        (void)hipSetDevice(0);
+        if (sol_set_source_ranges(c, 9003, 9003) != SOL_OK) { std::printf("FAIL %s\n", sol_last_error(c)); ++g_fails; }
+        (void)hipSetDevice(0);
+        if (sol_set_precision(c, SOL_PRECISION_MIXED, 0.0) != SOL_OK) { std::printf("FAIL %s\n", sol_last_error(c)); ++g_fails; }
+        expect("of a context of device 1 on device 0", 9003, fake::made_on()[0], 0);
+        if (fake::calls()["hipStreamCreateWithFlags"] != 2) { std::printf("FAIL no second stream\n"); ++g_fails; }
+        (void)hipSetDevice(0);
+        sol_destroy(c);
     }
     if (!g_fails) std::printf("context calls: ok\n");
     return g_fails != 0;

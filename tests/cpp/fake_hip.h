@@ -31,6 +31,8 @@ inline std::map<std::string, long> &calls() { static std::map<std::string, long>
 inline std::map<std::string, long> &kernels() { static std::map<std::string, long> m; return m; }   // launches by name
 inline std::map<const void *, std::string> &names() { static std::map<const void *, std::string> m; return m; }
 inline std::vector<ihipStream_t *> &streams() { static std::vector<ihipStream_t *> v; return v; }
+inline int &device() { static int d = 0; return d; }               // the current device, of two
+inline std::map<int, long> &made_on() { static std::map<int, long> m; return m; }   // allocations and streams by device
 inline std::map<void *, size_t> &device_memory() { static std::map<void *, size_t> m; return m; }
 inline std::function<void(const std::string &, void **)> &on_kernel()
 {
@@ -62,7 +64,7 @@ inline long pending()
     for (ihipStream_t *s : streams()) n += s->queued - s->done;
     return n;
 }
-inline void forget() { calls().clear(); kernels().clear(); }
+inline void forget() { calls().clear(); kernels().clear(); made_on().clear(); }
 struct Launch { dim3 grid, block; size_t lds; hipStream_t stream; };
 inline std::vector<Launch> &pushed() { static std::vector<Launch> v; return v; }
 }  // namespace fake
@@ -107,6 +109,7 @@ hipError_t hipMalloc(void **p, size_t n)
     FAKE("hipMalloc");
     *p = std::calloc(1, n);
     fake::device_memory()[*p] = n;
+    ++fake::made_on()[fake::device()];
     return hipSuccess;
 }
 hipError_t hipFree(void *p) { ++fake::calls()["hipFree"]; fake::device_memory().erase(p); std::free(p); return hipSuccess; }
@@ -132,6 +135,7 @@ hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned)
 {
     FAKE("hipStreamCreateWithFlags");
     *s = new ihipStream_t;
+    ++fake::made_on()[fake::device()];
     fake::streams().push_back(*s);
     return hipSuccess;
 }
@@ -170,9 +174,9 @@ hipError_t hipEventSynchronize(hipEvent_t e)
     return hipSuccess;
 }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 1.0f; return hipSuccess; }
-hipError_t hipSetDevice(int) { return hipSuccess; }
-hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
-hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
+hipError_t hipSetDevice(int d) { fake::device() = d; return hipSuccess; }
+hipError_t hipGetDevice(int *d) { *d = fake::device(); return hipSuccess; }
+hipError_t hipGetDeviceCount(int *n) { *n = 2; return hipSuccess; }
 hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *p, int)
 {
     std::memset(p, 0, sizeof *p);
